@@ -74,6 +74,22 @@ int nsvf_svo_intersect(const float* ray_start, const float* ray_dir,
                        int n_max, int32_t* idx, float* min_depth,
                        float* max_depth, void* stream);
 
+/* nsvf_svo_intersect with a device workspace of nsvf_svo_workspace_bytes()
+ * (4-byte aligned; its contents are not read, and it is free again once the
+ * call's kernels have run).  With one tree for all rays a first kernel checks
+ * that each node's octant holds the leaves below it, as in every tree of
+ * nsvf_build_octree, and the traversal then prunes with the octants instead
+ * of the reference's boxes of twice their size: the same outputs, in about
+ * half the time.  A tree that does not pass, or a tree per ray batch, is
+ * traversed as by nsvf_svo_intersect.                                      */
+int64_t nsvf_svo_workspace_bytes(void);
+int nsvf_svo_intersect_ws(const float* ray_start, const float* ray_dir,
+                          const float* points, const int32_t* children, int B,
+                          int M, int T, int tree_shared, float voxelsize,
+                          int n_max, int32_t* idx, float* min_depth,
+                          float* max_depth, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
 /* Host-side octree build over integer voxel coordinates (half-voxel units).
  * Replaces `_ext.build_octree(center, points, depth)`
  * (fairnr/clib/src/octree.cpp:125-136).  Host pointers.  Two calls: the

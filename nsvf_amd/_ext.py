@@ -112,9 +112,12 @@ def svo_intersect(ray_start, ray_dir, points, children, voxelsize, n_max):
     lo = torch.empty((B, M, n_max), dtype=torch.float32, device=dev)
     hi = torch.empty((B, M, n_max), dtype=torch.float32, device=dev)
     shared = int(points.size(0) == 1)
-    check(lib().nsvf_svo_intersect(_ptr(ray_start), _ptr(ray_dir), _ptr(points), _ptr(children),
-                                   B, M, points.size(1), shared, float(_scalar(voxelsize)), n_max,
-                                   _ptr(idx), _ptr(lo), _ptr(hi), _stream(dev)), "svo_intersect")
+    ws_bytes = int(lib().nsvf_svo_workspace_bytes())
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    check(lib().nsvf_svo_intersect_ws(_ptr(ray_start), _ptr(ray_dir), _ptr(points), _ptr(children),
+                                      B, M, points.size(1), shared, float(_scalar(voxelsize)),
+                                      n_max, _ptr(idx), _ptr(lo), _ptr(hi), _ptr(ws), ws_bytes,
+                                      _stream(dev)), "svo_intersect")
     return idx, lo, hi
 
 

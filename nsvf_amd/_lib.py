@@ -36,6 +36,8 @@ SIGNATURES = {
     "nsvf_version": ([], _I),
     "nsvf_aabb_intersect": ([_P, _P, _P, _I, _I, _I, _I, _F, _I, _P, _P, _P, _P], _I),
     "nsvf_svo_intersect": ([_P, _P, _P, _P, _I, _I, _I, _I, _F, _I, _P, _P, _P, _P], _I),
+    "nsvf_svo_workspace_bytes": ([], _L),
+    "nsvf_svo_intersect_ws": ([_P, _P, _P, _P, _I, _I, _I, _I, _F, _I, _P, _P, _P, _P, _L, _P], _I),
     "nsvf_build_octree": ([_P, _P, _I, _I, ctypes.POINTER(_P), ctypes.POINTER(_I)], _I),
     "nsvf_octree_take": ([_P, _P, _P], _I),
     "nsvf_inverse_cdf_sampling": ([_P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _F, _I, _P, _P, _P, _P, _P], _I),

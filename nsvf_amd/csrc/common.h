@@ -70,4 +70,37 @@ __device__ __forceinline__ bool ray_aabb(const float o[3], const float inv[3],
   return true;
 }
 
+// Slab test against a box given by its corners; with mn = fp32(c - h) and
+// mx = fp32(c + h) this is the reference's test (intersect_gpu.cu:93-94
+// evaluates (c - h) - o and (c + h) - o) bit for bit.  The reference returns
+// early (per axis: hi < f_low, lo > f_high, then f_low > f_high); here every
+// axis runs and only the final f_low > f_high decides, which is the same
+// test: f_low only grows and f_high only shrinks, so any early exit leaves
+// f_low > f_high at the end, and without one the running values are the
+// reference's.  The swap is a compare-and-select, as the reference's
+// ternaries, so an axis whose bounds come out NaN (direction 0 and origin on
+// the slab plane) is not swapped (a min / max pair would drop its NaN); the
+// running bounds then ignore a NaN as the reference's failed comparisons do,
+// since fmaxf / fminf return the other operand.  No branches: the traversals
+// run one test per child and lane without divergence, and the three axes'
+// loads are in flight together.
+__device__ __forceinline__ bool ray_box(const float o[3], const float inv[3], const float mn[3],
+                                        const float mx[3], float* out_lo, float* out_hi) {
+  float f_low = 0.0f;
+  float f_high = 100000.0f;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const float l0 = (mn[a] - o[a]) * inv[a];
+    const float h0 = (mx[a] - o[a]) * inv[a];
+    const bool sw = h0 < l0;
+    const float lo = sw ? h0 : l0;
+    const float hi = sw ? l0 : h0;
+    f_low = fmaxf(f_low, lo);
+    f_high = fminf(f_high, hi);
+  }
+  *out_lo = f_low;
+  *out_hi = f_high;
+  return !(f_low > f_high);
+}
+
 }  // namespace nsvf

@@ -36,37 +36,11 @@ constexpr int kMaxLevels = 24;
 // ---------------------------------------------------------------------------
 // hits
 
-// Slab test against a box given by its corners; with mn = fp32(c - h) and
-// mx = fp32(c + h) this is the reference's test (intersect_gpu.cu:93-94
-// evaluates (c - h) - o and (c + h) - o) bit for bit.  The reference returns
-// early (per axis: hi < f_low, lo > f_high, then f_low > f_high); here every
-// axis runs and only the final f_low > f_high decides, which is the same
-// test: f_low only grows and f_high only shrinks, so any early exit leaves
-// f_low > f_high at the end, and without one the running values are the
-// reference's.  The swap and the updates are compare-and-selects, as the
-// reference's ternaries, so an axis whose bounds come out NaN (direction 0
-// and origin on the slab plane) fails every comparison and changes nothing
-// (a min / max pair would not: it drops the NaN operand).  No branches: the
-// traversal runs one test per child and lane without divergence.
+// ray_box against a packed record's box (its fourth components are other data).
 __device__ __forceinline__ bool ray_box(const float o[3], const float inv[3], const float4& mn,
                                         const float4& mx, float* out_lo, float* out_hi) {
-  float f_low = 0.0f;
-  float f_high = 100000.0f;
-  const float a0[3] = {mn.x, mn.y, mn.z};
-  const float a1[3] = {mx.x, mx.y, mx.z};
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const float l0 = (a0[a] - o[a]) * inv[a];
-    const float h0 = (a1[a] - o[a]) * inv[a];
-    const bool sw = h0 < l0;
-    const float lo = sw ? h0 : l0;
-    const float hi = sw ? l0 : h0;
-    f_low = (lo > f_low) ? lo : f_low;
-    f_high = (hi < f_high) ? hi : f_high;
-  }
-  *out_lo = f_low;
-  *out_hi = f_high;
-  return !(f_low > f_high);
+  const float a0[3] = {mn.x, mn.y, mn.z}, a1[3] = {mx.x, mx.y, mx.z};
+  return nsvf::ray_box(o, inv, a0, a1, out_lo, out_hi);
 }
 
 // A ray's hit row as the traversal fills it, with what the kernel needs
