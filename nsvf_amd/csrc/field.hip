@@ -19,7 +19,9 @@
 //         features; lane group g = lane/16 holds features
 //         {4g..4g+3, 16+4g..16+4g+3} of its K-tile.
 //   FP32: v_mfma_f32_16x16x4_f32.  K-tile of 4 features; lane group g holds
-//         feature 16t + 4g + i of K-tile (t, i).
+//         feature 16t + 4g + i of K-tile (t, i).  Where the weights fit the
+//         LDS as FP16 pairs, the FP16 matrix units at FP32 accuracy instead
+//         (mlp_f16x3.h), with the FP32 MFMAs for tiles that are not finite.
 // Both layouts make a lane gather the same 8 embedding features per 32.
 //
 // Weight fragments: [layer][m-tile][k-tile][64 lanes][8 bf16 | 1 f32],
@@ -28,6 +30,7 @@
 #include <cmath>
 #include <mutex>
 
+#include "mlp_f16x3.h"
 #include "render.h"
 
 namespace nsvf {
@@ -245,6 +248,76 @@ struct LatticeSource {
     else
       corner_weights(sc, int32_t(v), x, w, key);
     return true;
+  }
+};
+
+// The sources as the FP16-split kernel reads them, a wave's 32-sample tiles
+// one after another: next(base, M) starts on the tile at `base` (its loads are
+// in flight until weights() needs them), then weights(j, w, key) gives its
+// samples 16 j + lane % 16, as Source::weights<true> does.
+template <class Src>
+struct TileReader;
+
+// The next tile's records are loaded while the current tile is evaluated.
+template <>
+struct TileReader<StreamSource> {
+  const StreamSource& src;
+  SampleRec rec[2];
+  __device__ __forceinline__ explicit TileReader(const StreamSource& s) : src(s) {}
+  __device__ __forceinline__ void next(int64_t base, int64_t M) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int64_t s = base + 16 * j + (threadIdx.x & 15);
+      rec[j] = SampleRec{-1, 0.0f, 0.0f, 0};
+      if (s < M) rec[j] = src.samples[src.list ? src.list[s] : s];
+    }
+  }
+  __device__ __forceinline__ bool weights(int j, float w[8], int32_t key[8]) const {
+    if (rec[j].idx < 0) return false;
+    float x[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      x[a] = src.rays.start[int64_t(rec[j].ray) * 3 + a] +
+             src.rays.dir[int64_t(rec[j].ray) * 3 + a] * rec[j].depth;
+    corner_weights_fast(src.sc, rec[j].idx, x, w, key);
+    return true;
+  }
+};
+
+// A tile lies in one voxel (bits^3 is a multiple of 64).  The offsets of the
+// lattice's planes stand in the wave's lanes (bits <= 64), and l / bits is a
+// multiplication: bits^3 (bits - 1) < 2^32.
+template <>
+struct TileReader<LatticeSource> {
+  const LatticeSource& src;
+  float plane;
+  uint32_t magic;
+  int64_t v;
+  uint32_t l0;
+  int64_t left;  // samples from the tile's base to the end
+  __device__ __forceinline__ explicit TileReader(const LatticeSource& s) : src(s) {
+    const int i = threadIdx.x & 63;
+    plane = float(2 * i + 1 - src.bits) / float(src.bits - 1) * src.half_voxel;
+    magic = uint32_t((uint64_t(1) << 32) / uint32_t(src.bits)) + 1;
+  }
+  __device__ __forceinline__ void next(int64_t base, int64_t M) {
+    const int64_t per = int64_t(src.bits) * src.bits * src.bits;
+    const int64_t q = base / per;
+    v = src.voxel0 + q;
+    l0 = uint32_t(base - q * per);
+    left = M - base;
+  }
+  __device__ __forceinline__ bool weights(int j, float w[8], int32_t key[8]) const {
+    const int t = 16 * j + (threadIdx.x & 15);
+    const uint32_t l = l0 + t, bits = src.bits;
+    const uint32_t ij = __umulhi(l, magic), i = __umulhi(ij, magic);
+    const uint32_t ijk[3] = {i, ij - i * bits, l - ij * bits};
+    float x[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+      x[a] = src.sc.centers[v * 3 + a] + __shfl(plane, int(ijk[a]), 64);
+    corner_weights_fast(src.sc, int32_t(v), x, w, key);
+    return t < left;
   }
 };
 
@@ -1338,124 +1411,206 @@ __global__ __launch_bounds__(64 * kFusedWaves, 1) void field_fused_kernel(
   }
 }
 
-// FP32 variant: same structure on v_mfma_f32_16x16x4_f32, weights read from
-// global memory (fragments of 64 floats).
-template <int D, int H, int L, class Src, class Sink>
-__global__ __launch_bounds__(kFieldBlock) void field_f32_kernel(
-    Src src, const int32_t* m_dev, int64_t m_max, const float* __restrict__ wfrag,
-    const float* __restrict__ bias, Sink sink) {
-  constexpr int NT = 2;
+// The FP32 field.  A wave's tile is 32 samples (two n-tiles); lane (g, c)
+// gathers its features of samples c and 16 + c, x[j][4 t + i] = feature
+// 16 t + 4 g + i.
+constexpr int kF32NT = 2;
+
+template <int D, class Weights>
+__device__ __forceinline__ void gather_f32_tile(const FieldScene& sc, int g,
+                                                float (&x)[kF32NT][4 * ((D + 15) / 16)],
+                                                Weights weights) {
+  constexpr int KT0 = 4 * ((D + 15) / 16);
+#pragma unroll
+  for (int j = 0; j < kF32NT; ++j) {
+    float w[8];
+    int32_t key[8];
+    const bool valid = weights(j, w, key);
+#pragma unroll
+    for (int kt32 = 0; kt32 < (KT0 + 7) / 8; ++kt32) {
+      float f[8];
+      if (valid) {
+        gather8_fma<D>(sc, w, key, kt32, g, f);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f[i] = 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (8 * kt32 + i < KT0) x[j][8 * kt32 + i] = f[i];
+    }
+  }
+}
+
+// The MLP of one wave tile on v_mfma_f32_16x16x4_f32, weights read from
+// global memory (fragments of 64 floats): out[j] = the head's 4 sums (biases
+// added) of sample c on the lanes of group 0.
+template <int D, int H, int L>
+__device__ __forceinline__ void mlp_f32_tile(const float (&x)[kF32NT][4 * ((D + 15) / 16)],
+                                             const float* __restrict__ wfrag,
+                                             const float* __restrict__ bias, int lane, int g,
+                                             f32x4 (&out)[kF32NT]) {
+  constexpr int NT = kF32NT;
   constexpr int KT0 = 4 * ((D + 15) / 16);  // k-tiles (t, i) of the input
   constexpr int KTH = H / 4;
   constexpr int MTH = H / 16;
-  const int lane = threadIdx.x & 63, g = lane >> 4, col = lane & 15;
-  const int64_t M = m_dev ? min(int64_t(*m_dev), m_max) : m_max;
-  const int64_t tiles = (M + 16 * NT - 1) / (16 * NT);
-  for (int64_t t = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6); t < tiles;
-       t += int64_t(gridDim.x) * 4) {
-    const int64_t base = t * 16 * NT;
-    sink.begin_tile(base, M, 16 * NT);
-    float x0[KT0][NT];
+  float xh[KTH][NT];
+  const float* A = wfrag;
+#pragma unroll
+  for (int mt = 0; mt < MTH; ++mt) {
+    f32x4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kt = 0; kt < KT0; ++kt) {
+      const float a = A[(mt * KT0 + kt) * 64 + lane];
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x[j][kt], acc[j], 0, 0, 0);
+    }
+    const float4 bb = *reinterpret_cast<const float4*>(bias + 16 * mt + 4 * g);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-      const int64_t s = base + 16 * j + col;
-      float w[8];
-      int32_t key[8];
-      const bool valid = s < M && src.template weights<false>(s, w, key);
-#pragma unroll
-      for (int kt32 = 0; kt32 < (KT0 + 7) / 8; ++kt32) {
-        float f[8];
-        if (valid) {
-          gather8<D>(src.sc, w, key, kt32, g, f);
-        } else {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) f[i] = 0.0f;
-        }
-        // features 32*kt32 + 4g + i -> k-tile (t = 2*kt32, i); 32*kt32 + 16 +
-        // 4g + i -> k-tile (t = 2*kt32 + 1, i)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if ((2 * kt32) * 4 + i < KT0) x0[(2 * kt32) * 4 + i][j] = f[i];
-          if ((2 * kt32 + 1) * 4 + i < KT0) x0[(2 * kt32 + 1) * 4 + i][j] = f[4 + i];
-        }
-      }
+      xh[4 * mt + 0][j] = fmaxf(acc[j][0] + bb.x, 0.0f);
+      xh[4 * mt + 1][j] = fmaxf(acc[j][1] + bb.y, 0.0f);
+      xh[4 * mt + 2][j] = fmaxf(acc[j][2] + bb.z, 0.0f);
+      xh[4 * mt + 3][j] = fmaxf(acc[j][3] + bb.w, 0.0f);
     }
-    float xh[KTH][NT];
-    {
-      const float* A = wfrag;
-#pragma unroll
-      for (int mt = 0; mt < MTH; ++mt) {
-        f32x4 acc[NT];
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kt = 0; kt < KT0; ++kt) {
-          const float a = A[(mt * KT0 + kt) * 64 + lane];
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, x0[kt][j], acc[j], 0, 0, 0);
-        }
-        const float4 bb = *reinterpret_cast<const float4*>(bias + 16 * mt + 4 * g);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          xh[4 * mt + 0][j] = fmaxf(acc[j][0] + bb.x, 0.0f);
-          xh[4 * mt + 1][j] = fmaxf(acc[j][1] + bb.y, 0.0f);
-          xh[4 * mt + 2][j] = fmaxf(acc[j][2] + bb.z, 0.0f);
-          xh[4 * mt + 3][j] = fmaxf(acc[j][3] + bb.w, 0.0f);
-        }
-      }
-    }
-    const float* A = wfrag + MTH * KT0 * 64;
+  }
+  A = wfrag + MTH * KT0 * 64;
 #pragma unroll 1
-    for (int l = 1; l < L; ++l) {
-      float nx[KTH][NT];
+  for (int l = 1; l < L; ++l) {
+    float nx[KTH][NT];
 #pragma unroll
-      for (int mt = 0; mt < MTH; ++mt) {
-        f32x4 acc[NT];
-#pragma unroll
-        for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kt = 0; kt < KTH; ++kt) {
-          const float a = A[(mt * KTH + kt) * 64 + lane];
-#pragma unroll
-          for (int j = 0; j < NT; ++j)
-            acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, xh[kt][j], acc[j], 0, 0, 0);
-        }
-        const float4 bb = *reinterpret_cast<const float4*>(bias + H * l + 16 * mt + 4 * g);
-#pragma unroll
-        for (int j = 0; j < NT; ++j) {
-          nx[4 * mt + 0][j] = fmaxf(acc[j][0] + bb.x, 0.0f);
-          nx[4 * mt + 1][j] = fmaxf(acc[j][1] + bb.y, 0.0f);
-          nx[4 * mt + 2][j] = fmaxf(acc[j][2] + bb.z, 0.0f);
-          nx[4 * mt + 3][j] = fmaxf(acc[j][3] + bb.w, 0.0f);
-        }
-      }
-#pragma unroll
-      for (int kt = 0; kt < KTH; ++kt)
-#pragma unroll
-        for (int j = 0; j < NT; ++j) xh[kt][j] = nx[kt][j];
-      A += MTH * KTH * 64;
-    }
-    {
+    for (int mt = 0; mt < MTH; ++mt) {
       f32x4 acc[NT];
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kt = 0; kt < KTH; ++kt) {
-        const float a = A[kt * 64 + lane];
+        const float a = A[(mt * KTH + kt) * 64 + lane];
 #pragma unroll
         for (int j = 0; j < NT; ++j)
           acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, xh[kt][j], acc[j], 0, 0, 0);
       }
-      const float* B = bias + H * L;
+      const float4 bb = *reinterpret_cast<const float4*>(bias + H * l + 16 * mt + 4 * g);
 #pragma unroll
       for (int j = 0; j < NT; ++j) {
-        const int64_t s = base + 16 * j + col;
-        sink.put(j, s, g == 0 && s < M, acc[j][0] + B[0], acc[j][1] + B[1], acc[j][2] + B[2],
-                 acc[j][3] + B[3]);
+        nx[4 * mt + 0][j] = fmaxf(acc[j][0] + bb.x, 0.0f);
+        nx[4 * mt + 1][j] = fmaxf(acc[j][1] + bb.y, 0.0f);
+        nx[4 * mt + 2][j] = fmaxf(acc[j][2] + bb.z, 0.0f);
+        nx[4 * mt + 3][j] = fmaxf(acc[j][3] + bb.w, 0.0f);
       }
-      sink.end_tile(base);
     }
+#pragma unroll
+    for (int kt = 0; kt < KTH; ++kt)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) xh[kt][j] = nx[kt][j];
+    A += MTH * KTH * 64;
+  }
+  f32x4 acc[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int kt = 0; kt < KTH; ++kt) {
+    const float a = A[kt * 64 + lane];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+      acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, xh[kt][j], acc[j], 0, 0, 0);
+  }
+  const float* B = bias + H * L;
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) out[j][r] = acc[j][r] + B[r];
+}
+
+template <class Sink>
+__device__ __forceinline__ void put_f32_tile(Sink& sink, const f32x4 (&out)[kF32NT], int64_t base,
+                                             int64_t M, int g, int col) {
+#pragma unroll
+  for (int j = 0; j < kF32NT; ++j) {
+    const int64_t s = base + 16 * j + col;
+    sink.put(j, s, g == 0 && s < M, out[j][0], out[j][1], out[j][2], out[j][3]);
+  }
+  sink.end_tile(base);
+}
+
+// Shapes whose FP16 weight parts do not fit the LDS: the whole field on the
+// FP32 MFMAs.
+template <int D, int H, int L, class Src, class Sink>
+__global__ __launch_bounds__(kFieldBlock) void field_f32_kernel(
+    Src src, const int32_t* m_dev, int64_t m_max, const float* __restrict__ wfrag,
+    const float* __restrict__ bias, Sink sink) {
+  const int lane = threadIdx.x & 63, g = lane >> 4, col = lane & 15;
+  const int64_t M = m_dev ? min(int64_t(*m_dev), m_max) : m_max;
+  const int64_t tiles = (M + 16 * kF32NT - 1) / (16 * kF32NT);
+  for (int64_t t = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6); t < tiles;
+       t += int64_t(gridDim.x) * 4) {
+    const int64_t base = t * 16 * kF32NT;
+    sink.begin_tile(base, M, 16 * kF32NT);
+    float x[kF32NT][4 * ((D + 15) / 16)];
+    gather_f32_tile<D>(src.sc, g, x, [&](int j, float w[8], int32_t key[8]) {
+      const int64_t s = base + 16 * j + col;
+      return s < M && src.template weights<true>(s, w, key);
+    });
+    f32x4 out[kF32NT];
+    mlp_f32_tile<D, H, L>(x, wfrag, bias, lane, g, out);
+    put_f32_tile(sink, out, base, M, g, col);
+  }
+}
+
+// The FP32 field with its MLP on the FP16 matrix units (F16Mlp: FP32
+// accuracy), the gather as above.  Bound: the matrix pipe and the vector unit
+// together -- per tile and SIMD 7.3 k cycles of MFMAs against about 4 k of
+// epilogue (sums, ReLU, column maxima, hi / lo parts) and 2 k of gather, which
+// only the SIMD's other wave overlaps.
+// Against field_f32_kernel, whose matrix work alone takes 5.3 times as long:
+// 26.9 M lattice points 50.2 -> 5.9 ms, the 7.5 M samples of a 400 x 400 view
+// 14.7 -> 1.93 ms.
+template <int D, int H, int L, class Src, class Sink>
+__global__ __launch_bounds__(64 * kF16Waves, 1) void field_f16x3_kernel(
+    Src src, const int32_t* m_dev, int64_t m_max, const float* __restrict__ wfrag,
+    const float* __restrict__ bias, Sink sink) {
+  static_assert(kF16NT == kF32NT, "one tile shape for both paths");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  const int lane = threadIdx.x & 63, g = lane >> 4, col = lane & 15;
+  const int64_t M = m_dev ? min(int64_t(*m_dev), m_max) : m_max;
+  const int64_t tiles = (M + kF16Samples - 1) / kF16Samples;
+  if (int64_t(blockIdx.x) * kF16Waves >= tiles) return;  // no tile: no weight staging
+  const auto mlp = F16Mlp<D, H, L>::stage(wfrag, bias, smem_raw);
+  // consecutive tiles per wave: neighbouring samples' corner rows stay in L1
+  const int64_t waves = int64_t(gridDim.x) * kF16Waves, each = (tiles + waves - 1) / waves;
+  const int64_t first = (int64_t(blockIdx.x) * kF16Waves +
+                         __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * each;
+  const int64_t last = min(first + each, tiles);
+  TileReader<Src> reader(src);
+  if (first < last) reader.next(first * kF16Samples, M);
+  for (int64_t t = first; t < last; ++t) {
+    const int64_t base = t * kF16Samples;
+    sink.begin_tile(base, M, kF16Samples);
+    float x[kF32NT][D / 4];
+    const auto gather = [&] {
+      gather_f32_tile<D>(src.sc, g, x, [&](int j, float w[8], int32_t key[8]) {
+        return reader.weights(j, w, key);
+      });
+    };
+    gather();
+    f32x4 out[kF32NT];
+    const bool done = mlp.tile(x, lane, g, out, [&](int l) {
+      if (l == 1 && t + 1 < last) reader.next(base + kF16Samples, M);
+    });
+    if (!done) {
+      // the weights' address as a value of this branch: its loads' addresses
+      // would otherwise be formed before the loop and spilled
+      const float* wf = wfrag;
+      asm volatile("" : "+s"(wf));
+      reader.next(base, M);
+      gather();
+      mlp_f32_tile<D, H, L>(x, wf, bias, lane, g, out);
+      if (t + 1 < last) reader.next(base + kF16Samples, M);
+    }
+    put_f32_tile(sink, out, base, M, g, col);
   }
 }
 
@@ -1576,6 +1731,19 @@ int64_t bf16x3_workspace_bytes(int64_t m_max) {
 // as blocks retire instead of waiting for the whole launch; a block's
 // weight staging is amortised over its waves' 32 tiles.
 constexpr int64_t kX3TilesPerWave = 32;
+// The same for the FP16-split FP32 field, whose blocks convert their weights
+// (about 8 us): twice the tiles.
+constexpr int64_t kF16TilesPerWave = 64;
+
+// Whether the FP32 field of a shape runs on the FP16 matrix units: its hi and
+// lo weights must fit the LDS (and its input be whole k-tiles).
+template <int D, int H, int L>
+constexpr bool f16x3_fits() {
+  if constexpr (D % 32 == 0 && H % 32 == 0)
+    return F16Mlp<D, H, L>::fits();
+  else
+    return false;
+}
 
 template <int D, int H, int L>
 int launch_embed_bf16x3(FieldScene sc, FieldRays rays, const SampleRec* samples,
@@ -1695,11 +1863,23 @@ template <int D, int H, int L, class Src, class Sink>
 int launch_f32(const Src& src, const int32_t* m_dev, int64_t m_max, const void* wfrag,
                const float* bias, const Sink& sink, hipStream_t stream) {
   const int64_t tiles = ceil_div(m_max, 32);
-  const int64_t blocks = std::min<int64_t>(ceil_div(tiles, 4), 2048);
-  hipLaunchKernelGGL((field_f32_kernel<D, H, L, Src, Sink>), dim3(unsigned(blocks)),
-                     dim3(kFieldBlock), 0, stream, src, m_dev, m_max,
-                     static_cast<const float*>(wfrag), bias, sink);
-  return check_launch("field_f32");
+  if constexpr (f16x3_fits<D, H, L>()) {
+    const auto kernel = field_f16x3_kernel<D, H, L, Src, Sink>;
+    constexpr size_t lds = F16Mlp<D, H, L>::LDS_BYTES;
+    static const int64_t resident = resident_blocks(kernel, 64 * kF16Waves, lds);
+    const int64_t blocks =
+        std::max<int64_t>(std::min<int64_t>(resident, ceil_div(tiles, kF16Waves)),
+                          ceil_div(tiles, kF16Waves * kF16TilesPerWave));
+    hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(64 * kF16Waves), lds, stream, src,
+                       m_dev, m_max, static_cast<const float*>(wfrag), bias, sink);
+    return check_launch("field_f16x3");
+  } else {
+    const int64_t blocks = std::min<int64_t>(ceil_div(tiles, 4), 2048);
+    hipLaunchKernelGGL((field_f32_kernel<D, H, L, Src, Sink>), dim3(unsigned(blocks)),
+                       dim3(kFieldBlock), 0, stream, src, m_dev, m_max,
+                       static_cast<const float*>(wfrag), bias, sink);
+    return check_launch("field_f32");
+  }
 }
 
 template <int D, int H, int L>
