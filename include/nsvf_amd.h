@@ -447,7 +447,8 @@ int nsvf_render_reuse_fill(const int32_t* hit_list, const int32_t* n_hit_dev,
 /* Field evaluation of a sample stream: trilinear gather fused with the MLP
  * (L hidden ReLU layers of width H on a D-wide embedding, 4-wide head).
  *   precision 0: BF16 MFMA with FP32 accumulation, wfrag = packed bf16;
- *   precision 1: FP32 MFMA, wfrag = packed f32;
+ *   precision 1: FP32 (on FP16 hi / lo parts at FP32 accuracy where the
+ *     shape's weights fit the LDS, else FP32 MFMA), wfrag = packed f32;
  *   precision 2: split BF16 ("bf16x3"): every product W X as
  *     Wl Xh + Wh Xl + Wh Xh with W = Wh + Wl, X = Xh + Xl (bf16 parts),
  *     FP32 accumulation; wfrag = packed bf16 hi / lo fragment pairs; needs
@@ -630,7 +631,10 @@ int nsvf_march_end(const int32_t* hit_list, int64_t n_hit, const int32_t* off,
 /* The field MLP for training (fairnr/modules/field.py:217-279: L Linear +
  * ReLU layers of width H over D inputs, a 4-wide head; output (sigma,
  * sigmoid(r, g, b)), which the reference differentiates with torch
- * autograd), forward and backward on FP32 MFMA.  Built for D=32, H=128,
+ * autograd), forward and backward at FP32 accuracy: FP16 hi / lo parts of
+ * scaled FP32 operands, or the FP32 MFMAs for the tiles (forward) and calls
+ * (backward) with a value that is not finite or, in the backward, a weight or
+ * a sample's largest feature outside 2^-40 .. 2^60.  Built for D=32, H=128,
  * L=3 (nsvf_mlp_train_supported); other shapes return NSVF_EINVAL and the
  * size queries -1.
  * Parameters in torch layout: weights[l] [out][in] and biases[l] [out] for
@@ -655,11 +659,12 @@ int nsvf_mlp_train_backward(int D, int H, int L, const float* packed,
                             float* demb, float* partial, int64_t partial_floats,
                             float* dparams, void* stream);
 
-/* The same backward with the activations' recomputation, the input
- * gradients W^T dz and the parameter gradients in split BF16 (three BF16
- * MFMAs per product on hi / lo operand parts, hi = bf16(f), lo = bf16(f -
- * hi), FP32 accumulation: about FP32's accuracy); the head's recomputed
- * logits and input gradient stay FP32; still deterministic.  No
+/* The same backward with the activations' recomputation (logits included),
+ * the input gradients W^T dz and the parameter gradients in split BF16
+ * (three BF16 MFMAs per product on hi / lo operand parts, hi = bf16(f), lo
+ * = bf16(f - hi), FP32 accumulation: about FP32's accuracy); the head's
+ * input gradient and the bias gradients' sums stay FP32; still
+ * deterministic.  No
  * counterpart in the reference (its backward is torch autograd over FP32
  * Linear layers).  x3w: x3_frags(D, H, L) fragments of 1024 bf16 bit
  * patterns (512 hi, then 512 lo), 16-byte aligned, in the order W_0 [H/16

@@ -61,20 +61,21 @@ __device__ __forceinline__ float f16_unscale(int e) { return __int_as_float((e -
 
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 
-// hi and lo parts of s x and s y (s a power of two) as packed pairs: the
+// hi and lo parts of s x and t y (powers of two s, t) as packed pairs: the
 // products and differences are exact, so each part is rounded once.  One
 // v_fma_mix instruction per part (fused in FP32, then rounded to a half of
 // the register); written out, since the compiler forms the second hi twice.
-__device__ __forceinline__ void f16_split2(float x, float y, float s, f16x2& hi, f16x2& lo) {
+__device__ __forceinline__ void f16_split2(float x, float y, float s, float t, f16x2& hi,
+                                           f16x2& lo) {
   unsigned int h, l;
   asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(h) : "v"(x), "v"(s));
-  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(h) : "v"(y), "v"(s));
+  asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(h) : "v"(y), "v"(t));
   asm("v_fma_mixlo_f16 %0, %1, %2, -%3 op_sel:[0,0,0] op_sel_hi:[0,0,1]"
       : "=v"(l)
       : "v"(x), "v"(s), "v"(h));
   asm("v_fma_mixhi_f16 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
       : "+v"(l)
-      : "v"(y), "v"(s), "v"(h));
+      : "v"(y), "v"(t), "v"(h));
   hi = __builtin_bit_cast(f16x2, h);
   lo = __builtin_bit_cast(f16x2, l);
 }
@@ -132,7 +133,8 @@ struct F16Mlp {
 #pragma unroll
       for (int i = 0; i < 8; i += 2) {
         f16x2 h, l;
-        f16_split2(wfrag[(8 * f + i) * 64 + lane], wfrag[(8 * f + i + 1) * 64 + lane], s, h, l);
+        f16_split2(wfrag[(8 * f + i) * 64 + lane], wfrag[(8 * f + i + 1) * 64 + lane], s, s,
+                   h, l);
         hi[i] = h[0];
         hi[i + 1] = h[1];
         lo[i] = l[0];
@@ -143,6 +145,28 @@ struct F16Mlp {
     }
     __syncthreads();
     return F16Mlp{w, b, big};
+  }
+
+  // The same from FP16 fragments packed before (their scales follow from the
+  // layers' largest |weight|, top[0..L]): those of layers 0..L-1 at frags, the
+  // head's at head (512 floats per fragment, hi then lo).
+  static __device__ F16Mlp stage_packed(const float* __restrict__ frags,
+                                        const float* __restrict__ head,
+                                        const float* __restrict__ top,
+                                        const float* __restrict__ biases, unsigned char* lds) {
+    float4* w = reinterpret_cast<float4*>(lds);
+    float* b = reinterpret_cast<float*>(lds + WEIGHT_BYTES);
+    float* big = b + BIASES;
+    constexpr int BODY = (FRAGS - KTH) * 128, ALL = FRAGS * 128;  // float4s
+    static_assert(ALL % 512 == 0 && BODY % 512 == 0, "whole rounds of 512 threads");
+#pragma unroll 4
+    for (int i = threadIdx.x; i < ALL; i += 64 * kF16Waves)
+      w[i] = i < BODY ? reinterpret_cast<const float4*>(frags)[i]
+                      : reinterpret_cast<const float4*>(head)[i - BODY];
+    for (int i = threadIdx.x; i < BIASES; i += 64 * kF16Waves) b[i] = biases[i];
+    if (threadIdx.x <= L) big[threadIdx.x] = top[threadIdx.x];
+    __syncthreads();
+    return F16Mlp{reinterpret_cast<const f16x8*>(w), b, big};
   }
 
   // What a sample's column carries between layers: the factor that turns a
@@ -170,7 +194,7 @@ struct F16Mlp {
   static __device__ __forceinline__ void put2(float x, float y, float s, int i, f16x8& oh,
                                               f16x8& ol) {
     f16x2 h, l;
-    f16_split2(x, y, s, h, l);
+    f16_split2(x, y, s, s, h, l);
     oh[i] = h[0];
     oh[i + 1] = h[1];
     ol[i] = l[0];

@@ -12,7 +12,7 @@
 // activations stay in registers through all layers.  The backward products
 // dX^T = W^T dY^T use fragments of W^T packed in the same order.
 //
-// Backward kernel.  A block of 8 waves takes 128 samples at a time (16 per
+// FP32 backward kernel.  A block of 8 waves takes 128 samples at a time (16 per
 // wave).  Each wave recomputes its tile's forward pass (every layer's output
 // kept in registers), then walks the layers back: the head's dlogits (the
 // sigmoid's derivative fused), then per layer dz = dh * (h > 0), the input
@@ -28,24 +28,13 @@
 // order for a given sample count: the gradients are deterministic, with no
 // atomics.
 //
-// Split-BF16 backward (mlp_train_backward_kernel<..., true>).  The same
-// kernel with the forward recomputation of the hidden layers, the input
-// gradients dX^T = W^T dz^T and the weight and bias gradients on
-// v_mfma_f32_16x16x32_bf16 in split BF16: an
-// FP32 operand f is hi + lo with hi = bf16(f), lo = bf16(f - hi), and a
-// product is Wl Xh + Wh Xl + Wh Xh (FP32 accumulation; the dropped Wl Xl is
-// 2^-16 of it), so these products keep about FP32's accuracy at three BF16
-// MFMAs per 16x16x32 tile against eight FP32 16x16x4 MFMAs.  The weight
-// fragments (forward and transposed, hi and lo) come from global memory,
-// 288 KB that stay in L2; a k-tile's operand lane (g, c) holds features
-// 32 kt + 4 g + i and 32 kt + 16 + 4 g + i (i < 4) of sample c -- the
-// accumulators of m-tiles 2 kt and 2 kt + 1, so a layer's FP32 output
-// splits into the next layer's operands in registers.  The weight
-// gradients sum over samples, the MFMA's k: dz and the layer input are
-// staged in LDS as hi and lo planes of [feature][sample] bf16, so an
-// operand (8 samples of one feature) is one 16-byte read, and each wave
-// keeps its rows of every dW in registers as in the FP32 kernel.  The
-// head's recomputed logits and its input gradient (4 wide) stay in FP32.
+// That is the FP32 kernel, which now runs for inputs that are not finite (or
+// far outside FP16's reach) only; the forward and backward otherwise run on
+// the 16-bit matrix units at FP32 accuracy (mlp_f16x3.h and
+// mlp_train_backward_kernel below), and the split-BF16 form (FieldMLPx3) is
+// the same backward kernel on BF16 parts: an FP32 operand f is hi + lo with
+// hi = bf16(f), lo = bf16(f - hi), a product Wl Xh + Wh Xl + Wh Xh in FP32
+// accumulators.
 #include <algorithm>
 
 #include "common.h"
@@ -71,10 +60,6 @@ typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
 
-__device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
 // (a, b) as packed bf16 pairs hi = bf16(a, b) and lo = bf16(a - hi, b - hi)
 // (round to nearest even; the differences are exact in FP32).
 __device__ __forceinline__ void split2(float a, float b, unsigned int& hi, unsigned int& lo) {
@@ -83,38 +68,6 @@ __device__ __forceinline__ void split2(float a, float b, unsigned int& hi, unsig
   const bf16x2 l = __builtin_convertvector(f32x2{a - hf[0], b - hf[1]}, bf16x2);
   hi = __builtin_bit_cast(unsigned int, h);
   lo = __builtin_bit_cast(unsigned int, l);
-}
-
-// The split operands of k-tile kt from a lane's FP32 values v[4 mt + r]
-// (feature 16 mt + 4 g + r): positions 0-3 from m-tile 2 kt, 4-7 from
-// m-tile 2 kt + 1.
-template <int N>
-__device__ __forceinline__ void split_ktile(const float (&v)[N], int kt, bf16x8& hi,
-                                            bf16x8& lo) {
-  unsigned int h[4], l[4];
-#pragma unroll
-  for (int p = 0; p < 4; ++p) split2(v[8 * kt + 2 * p], v[8 * kt + 2 * p + 1], h[p], l[p]);
-  hi = __builtin_bit_cast(bf16x8, u32x4{h[0], h[1], h[2], h[3]});
-  lo = __builtin_bit_cast(bf16x8, u32x4{l[0], l[1], l[2], l[3]});
-}
-
-// acc + the split product over KT k-tiles with fragments F (per fragment
-// 64 hi then 64 lo bf16x8 lane vectors), fragment kt at F + 128 kt; per
-// k-tile in the order Wl Xh, Wh Xl, Wh Xh -- the renderer's split-BF16 MLP
-// kernel's order, with the bias as the initial accumulator there too, so a
-// recomputed layer equals that kernel's forward bit for bit.
-template <int KT>
-__device__ __forceinline__ f32x4 mfma3_chain(const bf16x8* __restrict__ F,
-                                             const bf16x8 (&xh)[KT], const bf16x8 (&xl)[KT],
-                                             int lane, f32x4 acc) {
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt) {
-    const bf16x8 wh = F[128 * kt + lane], wl = F[128 * kt + 64 + lane];
-    acc = mfma32(wl, xh[kt], acc);
-    acc = mfma32(wh, xl[kt], acc);
-    acc = mfma32(wh, xh[kt], acc);
-  }
-  return acc;
 }
 
 // Closes one m-tile's loads and MFMAs: left to itself the scheduler hoists
@@ -163,7 +116,9 @@ struct TrainDims {
   static constexpr int T_FRAGS = T_HEAD + MT;
   static constexpr int64_t T_BASE = int64_t(F_FRAGS) * 64;
   static constexpr int64_t BIAS_BASE = T_BASE + int64_t(T_FRAGS) * 64;
-  static constexpr int64_t PACKED = BIAS_BASE + int64_t(L) * H + 4;
+  // per layer: largest |w|, largest row sum |w|, largest column sum |w|,
+  // largest |b| (L + 1 of each)
+  static constexpr int64_t STATS_BASE = BIAS_BASE + int64_t(L) * H + 4;
   // parameter gradients in torch order: W_0 [H][D], b_0 [H], ..., W_L [4][H], b_L [4]
   static constexpr int64_t P_W0 = 0, P_B0 = int64_t(H) * D;
   static constexpr int64_t P_LAYER1 = P_B0 + H;
@@ -177,6 +132,11 @@ struct TrainDims {
   static constexpr int X_T0 = X_HIDDEN + (L - 1) * MT * KXH;
   static constexpr int X_THIDDEN = X_T0 + MT0 * KXH;
   static constexpr int X_FRAGS = X_THIDDEN + (L - 1) * MT * KXH;
+  // the FP16 fragments (the same, then the head's forward ones) end the
+  // packed weights, 512 floats each
+  static constexpr int64_t F16_BASE = STATS_BASE + 4 * (L + 1);
+  static constexpr int F16_FRAGS = X_FRAGS + KXH;
+  static constexpr int64_t PACKED = F16_BASE + int64_t(F16_FRAGS) * 512;
 };
 
 // out[mt] = relu(W x + b) over the MT m-tiles: fragments A [MT][KT], input x
@@ -225,186 +185,9 @@ __device__ __forceinline__ void forward_tile(const float* __restrict__ emb, int6
   z = mfma_chain<T::KTH>(packed + T::F_HEAD * 64, h[L - 1], lane);
 }
 
-// Split-BF16 staging of the weight-gradient operands in LDS: per operand a
-// hi and a lo plane of [feature rows][kXRow] bf16 with the block's 128
-// samples along a row, so an MFMA operand (8 samples of one feature) is
-// one 16-byte read; 136 = 128 + 8 staggers the rows over the banks.
-constexpr int kXRow = 136;
-constexpr int kXPlane = kTrainChunk * kXRow;  // bf16 per plane
-
-// The split of a lane's values v[4 mt + r] (feature 16 mt + 4 g + r of
-// block sample s) for m-tiles mt < NMT, into rows of the planes ph / pl.
-template <int NMT, int N>
-__device__ __forceinline__ void stage_split(unsigned short* ph, unsigned short* pl,
-                                            const float (&v)[N], int g, int s) {
-  static_assert(4 * NMT <= N, "values");
-  // one lane address per plane; the rows are constant offsets from it
-  unsigned short* qh = ph + 4 * g * kXRow + s;
-  unsigned short* ql = pl + 4 * g * kXRow + s;
-#pragma unroll
-  for (int mt = 0; mt < NMT; ++mt)
-#pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      unsigned int hw, lw;
-      split2(v[4 * mt + 2 * p], v[4 * mt + 2 * p + 1], hw, lw);
-      const int row = 16 * mt + 2 * p;
-      qh[row * kXRow] = static_cast<unsigned short>(hw);
-      qh[(row + 1) * kXRow] = static_cast<unsigned short>(hw >> 16);
-      ql[row * kXRow] = static_cast<unsigned short>(lw);
-      ql[(row + 1) * kXRow] = static_cast<unsigned short>(lw >> 16);
-    }
-}
-
-__device__ __forceinline__ bf16x8 lds8(const unsigned short* p) {
-  return *reinterpret_cast<const bf16x8*>(p);
-}
-
-// Weight and bias gradients over the block's samples in split BF16:
-// acc[mi] += sum over samples of A row ra x B row rb0 + 16 mi, and (kBias)
-// accb += the sum of A row ra (its product with a row of ones, whose lo
-// part is 0), with A rows from planes (pah, pal) -- zero where !a_on -- and
-// B rows from (pbh, pbl); the lane reads samples 32 ks + 8 g.. of each
-// 32-sample step.  One step at a time with a fence per m-tile, so that the
-// operand reads are not hoisted into registers the kernel does not have.
-template <int NMI, bool kBias>
-__device__ __forceinline__ void dw_x3(const unsigned short* pah, const unsigned short* pal,
-                                      int ra, const unsigned short* pbh,
-                                      const unsigned short* pbl, int rb0, int g, bool a_on,
-                                      f32x4 (&acc)[NMI], f32x4& accb) {
-  const bf16x8 zero = {};
-  const bf16x8 ones = __builtin_bit_cast(
-      bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
-#pragma unroll 1
-  for (int ks = 0; ks < kTrainChunk / 32; ++ks) {
-    const int off = 32 * ks + 8 * g;
-    const bf16x8 ah = a_on ? lds8(pah + ra * kXRow + off) : zero;
-    const bf16x8 al = a_on ? lds8(pal + ra * kXRow + off) : zero;
-#pragma unroll
-    for (int mi = 0; mi < NMI; ++mi) {
-      const int rb = rb0 + 16 * mi;
-      const bf16x8 bh = lds8(pbh + rb * kXRow + off), bl = lds8(pbl + rb * kXRow + off);
-      acc[mi] = mfma32(al, bh, acc[mi]);
-      acc[mi] = mfma32(ah, bl, acc[mi]);
-      acc[mi] = mfma32(ah, bh, acc[mi]);
-      tile_fence();
-    }
-    if (kBias) {
-      accb = mfma32(al, ones, accb);
-      accb = mfma32(ah, ones, accb);
-    }
-  }
-}
-
 // ReLU as an integer max on the float's bits (the split-BF16 MLP kernel's).
 __device__ __forceinline__ float relu_bits(float x) {
   return __int_as_float(max(__float_as_int(x), 0));
-}
-
-// A split-BF16 layer over MT m-tiles: y[4 mt + r] = (relu of, kRelu) the
-// chain of mfma3_chain over fragments A [MT][KT] (fragment (mt, kt) at
-// A + 128 (mt KT + kt)) on operands xh / xl, from the bias b (kBias) or 0.
-// kAhead: the next m-tile's fragments are loaded before the current one's
-// MFMAs -- they come from L2, and waiting for them at the start of every
-// m-tile cost 15% of the backward (4.8 -> 4.05 ms on 3.09 M samples with
-// the recomputation and the hidden layers' input gradients loading ahead).
-template <int KT, int MT, bool kBias, bool kRelu, bool kAhead>
-__device__ __forceinline__ void layer_x3(const bf16x8* __restrict__ A, const bf16x8 (&xh)[KT],
-                                         const bf16x8 (&xl)[KT], const float* __restrict__ b,
-                                         float (&y)[4 * MT], int lane, int g) {
-  bf16x8 ch[KT], cl[KT];
-  if (kAhead) {
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      ch[kt] = A[128 * kt + lane];
-      cl[kt] = A[128 * kt + 64 + lane];
-    }
-  }
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (kBias) acc = *reinterpret_cast<const f32x4*>(b + 16 * mt + 4 * g);
-    if (kAhead) {
-      bf16x8 nh[KT], nl[KT];
-      if (mt + 1 < MT) {
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-          nh[kt] = A[128 * ((mt + 1) * KT + kt) + lane];
-          nl[kt] = A[128 * ((mt + 1) * KT + kt) + 64 + lane];
-        }
-      }
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) {
-        acc = mfma32(cl[kt], xh[kt], acc);
-        acc = mfma32(ch[kt], xl[kt], acc);
-        acc = mfma32(ch[kt], xh[kt], acc);
-      }
-      if (mt + 1 < MT) {
-#pragma unroll
-        for (int kt = 0; kt < KT; ++kt) {
-          ch[kt] = nh[kt];
-          cl[kt] = nl[kt];
-        }
-      }
-    } else {
-      acc = mfma3_chain<KT>(A + 128 * mt * KT, xh, xl, lane, acc);
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) y[4 * mt + r] = kRelu ? relu_bits(acc[r]) : acc[r];
-    tile_fence();
-  }
-}
-
-// dense_relu in split BF16 (relu(W x + b), the bias as the initial
-// accumulator), fragments loaded an m-tile ahead.
-template <int KT, int MT>
-__device__ __forceinline__ void dense_relu_x3(const bf16x8* __restrict__ A,
-                                              const bf16x8 (&xh)[KT], const bf16x8 (&xl)[KT],
-                                              const float* __restrict__ b, float (&y)[4 * MT],
-                                              int lane, int g) {
-  layer_x3<KT, MT, true, true, true>(A, xh, xl, b, y, lane, g);
-}
-
-// Layer 0 in split BF16 from the input x0 (k-tile order of forward_tile).
-template <int D, int H, int L>
-__device__ __forceinline__ void layer0_x3(const bf16x8* __restrict__ X, const float (&x0)[D / 4],
-                                          const float* __restrict__ bias, float (&h0)[H / 4],
-                                          int lane, int g) {
-  using T = TrainDims<D, H, L>;
-  bf16x8 xh[T::KX0], xl[T::KX0];
-#pragma unroll
-  for (int kt = 0; kt < T::KX0; ++kt) split_ktile(x0, kt, xh[kt], xl[kt]);
-  dense_relu_x3<T::KX0, T::MT>(X, xh, xl, bias, h0, lane, g);
-}
-
-// forward_tile with the hidden layers in split BF16 (fragments X); the head
-// stays FP32.
-template <int D, int H, int L>
-__device__ __forceinline__ void forward_tile_x3(const float* __restrict__ emb, int64_t M,
-                                                const float* __restrict__ packed,
-                                                const bf16x8* __restrict__ X, int64_t s,
-                                                float (&x0)[D / 4], float (&h)[L][H / 4],
-                                                f32x4& z, int lane, int g) {
-  using T = TrainDims<D, H, L>;
-  const float* bias = packed + T::BIAS_BASE;
-#pragma unroll
-  for (int t = 0; t < D / 16; ++t) {
-    float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (s < M) v = *reinterpret_cast<const float4*>(emb + s * D + 16 * t + 4 * g);
-    x0[4 * t + 0] = v.x;
-    x0[4 * t + 1] = v.y;
-    x0[4 * t + 2] = v.z;
-    x0[4 * t + 3] = v.w;
-  }
-  layer0_x3<D, H, L>(X, x0, bias, h[0], lane, g);
-#pragma unroll
-  for (int l = 1; l < L; ++l) {
-    bf16x8 xh[T::KXH], xl[T::KXH];
-#pragma unroll
-    for (int kt = 0; kt < T::KXH; ++kt) split_ktile(h[l - 1], kt, xh[kt], xl[kt]);
-    dense_relu_x3<T::KXH, T::MT>(X + 128 * (T::X_HIDDEN + (l - 1) * T::MT * T::KXH), xh, xl,
-                                 bias + l * H, h[l], lane, g);
-  }
-  z = mfma_chain<T::KTH>(packed + T::F_HEAD * 64, h[L - 1], lane);
 }
 
 // out[s] = (sigma, sigmoid(r), sigmoid(g), sigmoid(b)) of emb[s] for s < M.
@@ -414,7 +197,7 @@ __device__ __forceinline__ void forward_tile_x3(const float* __restrict__ emb, i
 // consecutive tiles, the next one's features loaded while it evaluates one.
 // Bound: the matrix pipe and the epilogue's vector instructions (mlp_f16x3.h).
 // On the FP32 MFMAs, with the fragments from L2, 1,000,003 samples took
-// 948 us, now 210; 4,093 samples 42 and 21 us, of which staging is 15.
+// 948 us, now 215; 4,093 samples 42 and 17 us.
 template <int D, int H, int L>
 __global__ __launch_bounds__(64 * kF16Waves, 1) void mlp_train_forward_kernel(
     const float* __restrict__ emb, int64_t M, const float* __restrict__ packed,
@@ -422,7 +205,10 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void mlp_train_forward_kernel(
   using T = TrainDims<D, H, L>;
   constexpr int NT = kF16NT;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-  const auto mlp = F16Mlp<D, H, L>::stage(packed, packed + T::BIAS_BASE, smem_raw);
+  const auto mlp = F16Mlp<D, H, L>::stage_packed(packed + T::F16_BASE,
+                                                 packed + T::F16_BASE + int64_t(T::X_FRAGS) * 512,
+                                                 packed + T::STATS_BASE, packed + T::BIAS_BASE,
+                                                 smem_raw);
   const int lane = threadIdx.x & 63, g = lane >> 4, col = lane & 15;
   const int64_t tiles = (M + kF16Samples - 1) / kF16Samples;
   const int64_t waves = int64_t(gridDim.x) * kF16Waves, each = (tiles + waves - 1) / waves;
@@ -485,13 +271,13 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void mlp_train_forward_kernel(
 // Backward: demb [M][D] and this block's partial parameter gradients
 // (partial + blockIdx.x * PARAMS, torch order), from dout [M][4] = the
 // gradient of (sigma, r, g, b) after the sigmoid.  Needs H == 16 * waves.
-// X3: the forward recomputation and the input gradients of layers 0..L-1
-// in split BF16 with the fragments x3w (TrainDims::X_FRAGS of them).
-template <int D, int H, int L, bool X3>
-__global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_kernel(
+// On the FP32 MFMAs: runs where one of the nflags flags is set, the whole
+// call again (grids differ: the sum over partials looks at the same flags).
+template <int D, int H, int L>
+__global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
     const float* __restrict__ emb, int64_t M, const float* __restrict__ packed,
-    const bf16x8* __restrict__ x3w, const float* __restrict__ dout, float* __restrict__ demb,
-    float* __restrict__ partial) {
+    const float* __restrict__ dout, float* __restrict__ demb, float* __restrict__ partial,
+    const int32_t* __restrict__ flags, int nflags) {
   using T = TrainDims<D, H, L>;
   static_assert(T::MT == kTrainWaves, "one hidden m-tile per wave");
   static_assert(D % 16 == 0 && D <= H, "input width");
@@ -517,12 +303,9 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_kernel(
 
   float* my_dz = lds_dz + (w * 16 + col) * kLdsRow;
   float* my_x = lds_x + (w * 16 + col) * kLdsRow;
-  // split-BF16 planes (X3): dz hi, dz lo, x hi, x lo
-  unsigned short* pzh = reinterpret_cast<unsigned short*>(smem_raw);
-  unsigned short* pzl = pzh + kXPlane;
-  unsigned short* pxh = pzl + kXPlane;
-  unsigned short* pxl = pxh + kXPlane;
-  const int sb = w * 16 + col;  // this lane's sample in the block
+  int flagged = 0;
+  for (int i = threadIdx.x; i < nflags; i += kTrainBlock) flagged |= flags[i];
+  if (!__syncthreads_or(flagged)) return;
   const int64_t chunks = (M + kTrainChunk - 1) / kTrainChunk;
   for (int64_t ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
     const int64_t s = ch * kTrainChunk + w * 16 + col;
@@ -531,10 +314,7 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_kernel(
     float x0[T::KT0];
     float h[L][T::KTH];
     f32x4 z;
-    if constexpr (X3)
-      forward_tile_x3<D, H, L>(emb, M, pk, opaque(x3w), s, x0, h, z, lane, g);
-    else
-      forward_tile<D, H, L>(emb, M, pk, s, x0, h, z, lane, g);
+    forward_tile<D, H, L>(emb, M, pk, s, x0, h, z, lane, g);
     // dlogits on the lanes of group 0: d sigma as given, d rgb through the
     // sigmoid's derivative y (1 - y)
     f32x4 dl = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -549,36 +329,20 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_kernel(
       dl[3] = d.w * (y3 * (1.0f - y3));
     }
     // ---- head: dW_head = dl^T h[L-1], dh = W_head^T dl
-    if constexpr (X3) {
-      if (g == 0) {
-        const float dlv[4] = {dl[0], dl[1], dl[2], dl[3]};
-        stage_split<1>(pzh, pzl, dlv, 0, sb);
-      }
-      stage_split<T::MT>(pxh, pxl, h[L - 1], g, sb);
-      __syncthreads();
-      f32x4 ghv[1] = {gh};
-      if (w == 0)
-        dw_x3<1, true>(pzh, pzl, col, pxh, pxl, 16 * w + col, g, col < 4, ghv, ghb);
-      else
-        dw_x3<1, false>(pzh, pzl, col, pxh, pxl, 16 * w + col, g, col < 4, ghv, ghb);
-      gh = ghv[0];
-      __syncthreads();
-    } else {
-      if (g == 0) *reinterpret_cast<f32x4*>(my_dz) = dl;
+    if (g == 0) *reinterpret_cast<f32x4*>(my_dz) = dl;
 #pragma unroll
-      for (int mt = 0; mt < T::MT; ++mt)
-        *reinterpret_cast<f32x4*>(my_x + 16 * mt + 4 * g) = f32x4{
-            h[L - 1][4 * mt], h[L - 1][4 * mt + 1], h[L - 1][4 * mt + 2], h[L - 1][4 * mt + 3]};
-      __syncthreads();
+    for (int mt = 0; mt < T::MT; ++mt)
+      *reinterpret_cast<f32x4*>(my_x + 16 * mt + 4 * g) = f32x4{
+          h[L - 1][4 * mt], h[L - 1][4 * mt + 1], h[L - 1][4 * mt + 2], h[L - 1][4 * mt + 3]};
+    __syncthreads();
 #pragma unroll 1
-      for (int kk = 0; kk < kTrainChunk / 4; ++kk) {
-        const int row = (4 * kk + g) * kLdsRow;
-        const float a = col < 4 ? lds_dz[row + col] : 0.0f;
-        gh = mfma4(a, lds_x[row + 16 * w + col], gh);
-        if (w == 0) ghb = mfma4(a, 1.0f, ghb);
-      }
-      __syncthreads();
+    for (int kk = 0; kk < kTrainChunk / 4; ++kk) {
+      const int row = (4 * kk + g) * kLdsRow;
+      const float a = col < 4 ? lds_dz[row + col] : 0.0f;
+      gh = mfma4(a, lds_x[row + 16 * w + col], gh);
+      if (w == 0) ghb = mfma4(a, 1.0f, ghb);
     }
+    __syncthreads();
     float dh[T::KTH];
     {
       // operand B of W_head^T: lane group g takes logit g of sample c
@@ -601,54 +365,29 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_kernel(
       float dz[T::KTH];
 #pragma unroll
       for (int k = 0; k < T::KTH; ++k) dz[k] = h[l][k] > 0.0f ? dh[k] : 0.0f;
-      if constexpr (X3) {
-        stage_split<T::MT>(pzh, pzl, dz, g, sb);
-      } else {
 #pragma unroll
-        for (int mt = 0; mt < T::MT; ++mt)
-          *reinterpret_cast<f32x4*>(my_dz + 16 * mt + 4 * g) =
-              f32x4{dz[4 * mt], dz[4 * mt + 1], dz[4 * mt + 2], dz[4 * mt + 3]};
-      }
+      for (int mt = 0; mt < T::MT; ++mt)
+        *reinterpret_cast<f32x4*>(my_dz + 16 * mt + 4 * g) =
+            f32x4{dz[4 * mt], dz[4 * mt + 1], dz[4 * mt + 2], dz[4 * mt + 3]};
       if (l > 0) {
         // the first layer's output again, from x0: keeping it from the
         // forward pass would hold 32 more registers through every later phase
-        if (l == 1) {
-          if constexpr (X3)
-            layer0_x3<D, H, L>(opaque(x3w), x0, bias, h[0], lane, g);
-          else
-            dense_relu<T::KT0, T::MT>(opaque(packed), x0, bias, h[0], lane, g);
-        }
-        if constexpr (X3) {
-          stage_split<T::MT>(pxh, pxl, h[l - 1], g, sb);
-        } else {
+        if (l == 1) dense_relu<T::KT0, T::MT>(opaque(packed), x0, bias, h[0], lane, g);
 #pragma unroll
-          for (int mt = 0; mt < T::MT; ++mt)
-            *reinterpret_cast<f32x4*>(my_x + 16 * mt + 4 * g) =
-                f32x4{h[l - 1][4 * mt], h[l - 1][4 * mt + 1], h[l - 1][4 * mt + 2],
-                      h[l - 1][4 * mt + 3]};
-        }
+        for (int mt = 0; mt < T::MT; ++mt)
+          *reinterpret_cast<f32x4*>(my_x + 16 * mt + 4 * g) =
+              f32x4{h[l - 1][4 * mt], h[l - 1][4 * mt + 1], h[l - 1][4 * mt + 2],
+                    h[l - 1][4 * mt + 3]};
       } else {
-        if constexpr (X3) {
-          stage_split<T::MT0>(pxh, pxl, x0, g, sb);
-        } else {
 #pragma unroll
-          for (int t = 0; t < T::MT0; ++t)
-            *reinterpret_cast<f32x4*>(my_x + 16 * t + 4 * g) =
-                f32x4{x0[4 * t], x0[4 * t + 1], x0[4 * t + 2], x0[4 * t + 3]};
-        }
+        for (int t = 0; t < T::MT0; ++t)
+          *reinterpret_cast<f32x4*>(my_x + 16 * t + 4 * g) =
+              f32x4{x0[4 * t], x0[4 * t + 1], x0[4 * t + 2], x0[4 * t + 3]};
       }
       __syncthreads();
-      // weight gradient rows 16w..16w+15 of layer l: split BF16 over the
-      // block's 128 samples, or FP32 4 samples per step
-      if constexpr (X3) {
-        if (l > 0)
-          dw_x3<T::MT, true>(pzh, pzl, 16 * w + col, pxh, pxl, col, g, true,
-                             gw[l > 0 ? l - 1 : 0], gb[l]);
-        else
-          dw_x3<T::MT0, true>(pzh, pzl, 16 * w + col, pxh, pxl, col, g, true, gw0, gb[l]);
-      }
+      // weight gradient rows 16w..16w+15 of layer l, 4 samples per step
 #pragma unroll 1
-      for (int kk = 0; kk < (X3 ? 0 : kTrainChunk / 4); ++kk) {
+      for (int kk = 0; kk < kTrainChunk / 4; ++kk) {
         const int row = (4 * kk + g) * kLdsRow;
         const float a = lds_dz[row + 16 * w + col];
         if (l > 0) {
@@ -664,25 +403,7 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_kernel(
         gb[l] = mfma4(a, 1.0f, gb[l]);
       }
       __syncthreads();
-      if constexpr (X3) {
-        bf16x8 dzh[T::KXH], dzl[T::KXH];
-#pragma unroll
-        for (int kt = 0; kt < T::KXH; ++kt) split_ktile(dz, kt, dzh[kt], dzl[kt]);
-        const bf16x8* Xt = opaque(x3w);
-        if (l > 0) {
-          layer_x3<T::KXH, T::MT, false, false, true>(
-              Xt + 128 * (T::X_THIDDEN + (l - 1) * T::MT * T::KXH), dzh, dzl, nullptr, dh, lane,
-              g);
-        } else {
-#pragma unroll
-          for (int mt = 0; mt < T::MT0; ++mt) {
-            const f32x4 acc = mfma3_chain<T::KXH>(Xt + 128 * (T::X_T0 + mt * T::KXH), dzh,
-                                                  dzl, lane, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-            if (s < M) *reinterpret_cast<f32x4*>(demb + s * D + 16 * mt + 4 * g) = acc;
-            tile_fence();
-          }
-        }
-      } else if (l > 0) {
+      if (l > 0) {
         const float* A = At + (T::T_HIDDEN + (l - 1) * T::MT * T::KTH) * 64;
 #pragma unroll
         for (int mt = 0; mt < T::MT; ++mt) {
@@ -723,84 +444,966 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_kernel(
   }
 }
 
-// dparams[p] = sum over blocks b = 0, 1, ... of partial[b][p].
-__global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ partial,
-                                                           int nb, int64_t P,
-                                                           float* __restrict__ dparams) {
-  const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (p >= P) return;
-  float acc = 0.0f;
-  for (int b = 0; b < nb; ++b) acc = acc + partial[int64_t(b) * P + p];
-  dparams[p] = acc;
+// ---------------------------------------------------------------------------
+// The backward kernel on the 16-bit matrix units: FP16 hi / lo parts (FP32
+// accuracy, as in mlp_f16x3.h) or, for FieldMLPx3, split BF16.
+//
+// A block of 8 waves takes 64 samples at a time.  The layers' outputs live in
+// LDS as hi and lo planes of [feature][sample]; wave w computes output
+// features 16w..16w+15 of every layer for all 64 samples, so a layer's
+// weights are read once per block and 64 samples (each wave its own 8 KB from
+// L2, loaded while the previous layer ends) where a wave per 16 samples read
+// all 288 KB for each of them.  A layer's products run as Y = X W^T, so a
+// lane's accumulator holds four consecutive samples of one feature and goes
+// out as one 8-byte store per part; the next layer's operand (8 features of a
+// sample) comes back through the transposing LDS read (ds_read_b64_tr_b16),
+// and the weight gradients' operands (8 samples of a feature) are plain
+// 16-byte reads of the same planes.  Rows are padded to 72 halves (36 banks);
+// unpadded rows with their units permuted by row gave the same conflicts and
+// needed an address register per tile.
+//
+//   phases (a barrier after each): the chunk's features; layers 0, 1, 2; the
+//   head with the logits' gradients; dz2 (dW_head); dW_2 and dz1; dW_1 and
+//   dz0; dW_0 and the input gradient.
+//
+// dz2 takes the plane set of no layer, dz1 takes h2's and dz0 takes dz2's,
+// which are dead by then.  The ReLU masks stay in registers (a bit per value).
+// The weight gradients accumulate in registers over the whole kernel, a wave
+// holding 32 x 64 of each hidden layer's, 16 x 32 of the first's and 4 x 16 of
+// the head's; the bias gradients are FP32 sums of dz.  Block partials are
+// added in block order, so the gradients do not depend on timing.
+//
+// Scales (FP16 only; all powers of two, exact).  Weights as in mlp_f16x3.h.  A
+// sample's activations are scaled by a bound of its layer's outputs, from the
+// layers' largest row sums |W| and biases: one layer past the sample's
+// largest feature for h0, two for h1, and for h2 two past its largest h0 (an
+// FP16 pair covers 2^40, so a loose bound costs no accuracy until it is 2^17
+// too large).  The logits' gradients of a sample are divided by the power of
+// two below their largest, everything behind them is linear in it, and the
+// bounds of dz are then the same for every sample; the input gradient is
+// multiplied back.  In the weight gradients, sums over samples, each sample's
+// factor multiplies dz when it is read, relative to the chunk's largest.
+// The FP16 matrix unit's sums come out low on average (measured: every bias
+// gradient's error negative, whatever its own sign).  That is below FP32's
+// rounding in one product, but a parameter's gradient adds a million: so every second sample's normalised gradient, and
+// every second chunk's weight gradient, is computed with the other sign.  (With
+// one sign the bias gradients were 3e-6 off on a million samples, FP32 MFMAs
+// 1e-6.)
+// An operand that is not finite or outside 2^-40 .. 2^60 raises the block's
+// flag, and the FP32 kernel below then computes the whole call.
+//
+// Bound: LDS reads (about 15 k cycles per 64 samples at 128 B per cycle)
+// beside 12.5 k of MFMAs, and the phases' barriers.
+// Per million samples, against the form before (each wave its own 16 samples,
+// all weights from L2 for each): FP32 2,970 -> 1,170 us, split BF16 about
+// 1,900 -> 1,250 us (686 -> 460 us in the training step of 8,192 rays); 4,093
+// samples 109 -> 31 us.  The FP32 gradients are 4.9e-7 off 64 bits at most, 1.3e-6
+// before.
+constexpr int kBwdWaves = 8;
+constexpr int kBwdBlock = 64 * kBwdWaves;
+constexpr int kBwdChunk = 64;                // samples per block step
+constexpr int kBwdRow = 72;                  // halves per plane row
+constexpr int kBwdPlane = 128 * kBwdRow;     // halves per hidden plane
+constexpr int kBwdPlane0 = 32 * kBwdRow;     // halves per input plane
+
+typedef __attribute__((ext_vector_type(2))) unsigned int u32x2;
+typedef __attribute__((ext_vector_type(4))) short s16x4;
+
+struct BwdLds {
+  unsigned short x0[2 * kBwdPlane0];         // input: hi plane, lo plane
+  unsigned short t[4][2 * kBwdPlane];        // h0, h1, h2, dz2
+  float dl[kBwdChunk][4];                    // logits' gradients (normalised)
+  unsigned short head[2][4][4][4][8];        // head weights hi / lo: [kt][g][logit][i]
+  float back[4][kBwdChunk];                  // accumulator -> sum, layers 0..2 and head
+  float scale[3][kBwdChunk];                 // sum -> parts, h0, h1, h2
+  _Float16 factor[3][kBwdChunk];             // weight gradients' sample factors: x0, h0, h1
+  float unit[kBwdChunk];                     // 2^k of the normalised gradients (0: none)
+  float factor2[kBwdChunk];                  // the head's weight gradient's sample factors
+  int top0[kBwdChunk];                       // largest h0 (float bits)
+  int wild;
+};
+static_assert(sizeof(BwdLds) <= 160 * 1024, "LDS");
+
+template <bool F16>
+__device__ __forceinline__ f32x4 mm16(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (F16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
+                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
-// Packs one layer W [Hout][Hin] (row-major, torch's Linear weight):
-// mode 0: forward fragments [ceil(Hout/16)][Hin/4][64], lane (g, c) of
-//   fragment (mt, 4t + i) = W[16 mt + c][16 t + 4 g + i] (0 past Hout);
-// mode 1: transposed fragments [Hin/16][Hout/4][64], lane (g, c) of
-//   fragment (mt, 4t + i) = W[16 t + 4 g + i][16 mt + c];
-// mode 2 (the 4-wide head): [Hin/16][64], lane (g, c) of fragment mt =
-//   W[g][16 mt + c].
-__global__ __launch_bounds__(256) void pack_layer_kernel(const float* __restrict__ W, int Hout,
-                                                         int Hin, int mode,
-                                                         float* __restrict__ dst, int64_t n) {
-  const int64_t f = int64_t(blockIdx.x) * 256 + threadIdx.x;
-  if (f >= n) return;
-  const int lane = int(f & 63), g = lane >> 4, c = lane & 15;
-  const int64_t frag = f >> 6;
-  float v = 0.0f;
-  if (mode == 0) {
-    const int KT = Hin / 4;
-    const int mt = int(frag / KT), kt = int(frag % KT), t = kt >> 2, i = kt & 3;
-    const int row = 16 * mt + c;
-    if (row < Hout) v = W[int64_t(row) * Hin + 16 * t + 4 * g + i];
-  } else if (mode == 1) {
-    const int KT = Hout / 4;
-    const int mt = int(frag / KT), kt = int(frag % KT), t = kt >> 2, i = kt & 3;
-    v = W[int64_t(16 * t + 4 * g + i) * Hin + 16 * mt + c];
+// a * b as split parts, hi b_lo, lo b_hi, hi b_hi (for BF16 the forward
+// kernel's order: Wl Xh, Wh Xl, Wh Xh with W in b).
+template <bool F16>
+__device__ __forceinline__ f32x4 mm16x3(u32x4 ah, u32x4 al, u32x4 bh, u32x4 bl, f32x4 c) {
+  c = mm16<F16>(ah, bl, c);
+  c = mm16<F16>(al, bh, c);
+  return mm16<F16>(ah, bh, c);
+}
+
+// Parts of s0 a and s1 b as packed pairs (BF16: s0 = s1 = 1).
+template <bool F16>
+__device__ __forceinline__ void parts2(float a, float b, float s0, float s1, unsigned int& hi,
+                                       unsigned int& lo) {
+  if constexpr (F16) {
+    f16x2 h, l;
+    f16_split2(a, b, s0, s1, h, l);
+    hi = __builtin_bit_cast(unsigned int, h);
+    lo = __builtin_bit_cast(unsigned int, l);
   } else {
-    v = W[int64_t(g) * Hin + 16 * frag + c];
+    split2(a, b, hi, lo);
   }
-  dst[f] = v;
+}
+
+__device__ __forceinline__ u32x4 lds128(const unsigned short* p) {
+  return *reinterpret_cast<const u32x4*>(p);
+}
+
+// Halves from a plane's start to (row r, sample i).
+__device__ __forceinline__ int bwd_at(int r, int i) { return r * kBwdRow + i; }
+
+// An operand of 8 features of a lane's sample, transposed out of a plane of
+// [feature][sample] rows: p = the lane's address (row 4 g + i / 4, sample
+// 4 (i % 4), i = lane % 16) of the k-tile's first half; the second is 16 rows
+// on.  Lane (g, c) gets features 4 g + 0..3 and 16 + 4 g + 0..3 of sample c.
+__device__ __forceinline__ u32x4 lds_tr(const unsigned short* p) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
+  const s16x4 b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 16 * kBwdRow));
+  const u32x2 x = __builtin_bit_cast(u32x2, a), y = __builtin_bit_cast(u32x2, b);
+  return u32x4{x[0], x[1], y[0], y[1]};
+}
+
+typedef const __attribute__((address_space(1))) u32x4* global_u32x4;
+
+// The wave's weight fragments of a layer: KT pairs at F (fragment: 64 lanes of
+// hi, then of lo).
+template <int KT>
+struct BwdFrags {
+  u32x4 h[KT], l[KT];
+  __device__ __forceinline__ void load(global_u32x4 F, int lane) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      h[kt] = F[128 * kt + lane];
+      l[kt] = F[128 * kt + 64 + lane];
+    }
+  }
+};
+
+// acc[m] += the layer's products for samples 16 m.. over KT k-tiles: operand
+// planes at p + at[m] (the lane's transposing address; lo plane `lo` halves on).  The
+// four sample tiles' chains alternate; a scheduling barrier closes each k-tile
+// (the SIMD's other wave covers its reads: a second set of operands in
+// registers was spilled).  FP16: the small products have sums of their own, so
+// that only KT accumulations round at the result's size.
+template <bool F16, int KT>
+__device__ __forceinline__ void bwd_layer(const unsigned short* p, const int (&at)[4], int lo,
+                                          const BwdFrags<KT>& w, f32x4 (&acc)[4]) {
+  f32x4 small[4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m) small[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    u32x4 ah[4], al[4];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) ah[m] = lds_tr(p + at[m] + kt * 32 * kBwdRow);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) al[m] = lds_tr(p + at[m] + kt * 32 * kBwdRow + lo);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      (F16 ? small[m] : acc[m]) = mm16<F16>(ah[m], w.l[kt], F16 ? small[m] : acc[m]);
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      (F16 ? small[m] : acc[m]) = mm16<F16>(al[m], w.h[kt], F16 ? small[m] : acc[m]);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) acc[m] = mm16<F16>(ah[m], w.h[kt], acc[m]);
+    tile_fence();
+  }
+  if constexpr (F16) {
+#pragma unroll
+    for (int m = 0; m < 4; ++m) acc[m] = acc[m] + small[m];
+  }
+}
+
+// sum[a][b] += 2^e x the sum over the chunk's samples of rows A (dz, NA tiles
+// of 16) and B (the layer's input, NB tiles): rows from pa / pb on, the lane's
+// at[ks] halves on (row c, sample 32 ks + 8 g), lo planes `lo_a` / `lo_b` halves
+// on; factor: the samples' factors; by: their sign in this chunk.  A chunk's products start from 0 and are added by the vector unit:
+// the matrix unit rounds its accumulations toward zero, which over a block's
+// hundreds of steps into one accumulator cost 4e-6 of the gradient (1e-6 so).
+template <bool F16, int NA, int NB>
+__device__ __forceinline__ void bwd_dw(const unsigned short* pa, int lo_a,
+                                       const unsigned short* pb, int lo_b, const int (&at)[2],
+                                       const _Float16* factor, int g, int e, float by,
+                                       f32x4 (&sum)[NA][NB]) {
+  constexpr int KS = kBwdChunk / 32;
+  u32x4 ah[KS][NA], al[KS][NA];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int a = 0; a < NA; ++a) {
+      ah[ks][a] = lds128(pa + at[ks] + a * 16 * kBwdRow);
+      al[ks][a] = lds128(pa + at[ks] + a * 16 * kBwdRow + lo_a);
+      if constexpr (F16) {
+        const f16x8 f = *reinterpret_cast<const f16x8*>(factor + 32 * ks + 8 * g);
+        ah[ks][a] = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, ah[ks][a]) * f);
+        al[ks][a] = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, al[ks][a]) * f);
+      }
+    }
+#pragma unroll
+  for (int b = 0; b < NB; ++b) {
+    f32x4 acc[NA];
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[a] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const u32x4 bh = lds128(pb + at[ks] + b * 16 * kBwdRow);
+      const u32x4 bl = lds128(pb + at[ks] + b * 16 * kBwdRow + lo_b);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[a] = mm16<F16>(ah[ks][a], bl, acc[a]);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[a] = mm16<F16>(al[ks][a], bh, acc[a]);
+#pragma unroll
+      for (int a = 0; a < NA; ++a) acc[a] = mm16<F16>(ah[ks][a], bh, acc[a]);
+    }
+    tile_fence();
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sum[a][b][r] = F16 ? __fmaf_rn(__builtin_amdgcn_ldexpf(acc[a][r], e), by, sum[a][b][r])
+                           : sum[a][b][r] + acc[a][r];
+    // the sums as values of this place: the compiler would otherwise move the
+    // additions to the end of the step and keep both operands until then
+#pragma unroll
+    for (int a = 0; a < NA; ++a) asm volatile("" : "+v"(sum[a][b]));
+  }
+}
+
+// Largest of the 16 lanes of a group, to its lane 15 (DPP row shifts; v >= 0).
+__device__ __forceinline__ int row_max15(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
+  return max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
+}
+
+// Exponent window of the FP16 form's operands, 2^-40 to 2^60 (or 0): every
+// factor formed from two of them is a normal number.
+constexpr int kTameLow = 87, kTameHigh = 187;
+__device__ __forceinline__ bool tame(float v) {
+  const int e = int(__float_as_uint(v) >> 23);
+  return v == 0.0f || (e >= kTameLow && e <= kTameHigh);
+}
+__device__ __forceinline__ int tame_exponent(float v) {
+  return min(max(int(__float_as_uint(v) >> 23), kTameLow), kTameHigh);
+}
+// The exponent e of f16_unscale(e) * f16_unscale(ew).
+__device__ __forceinline__ int feature_exponent(float back, int ew) {
+  return (__float_as_int(back) >> 23) + 127 - (ew - 14) + 14;
+}
+
+template <int D, int H, int L, bool F16>
+__global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
+    const float* __restrict__ emb, int64_t M, const float* __restrict__ packed,
+    const u32x4* __restrict__ frags, const float* __restrict__ dout, float* __restrict__ demb,
+    float* __restrict__ partial, int32_t* __restrict__ flags) {
+  using T = TrainDims<D, H, L>;
+  static_assert(D == 32 && H == 128 && L == 3, "the phases below");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
+  BwdLds& S = *reinterpret_cast<BwdLds*>(smem_raw);
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const float* bias = packed + T::BIAS_BASE;
+
+  // the layers' weight exponents and bounds (FP16)
+  [[maybe_unused]] int ew[4] = {0, 0, 0, 0};
+  [[maybe_unused]] float rowsum[4], maxb[4];
+  [[maybe_unused]] int ez[3] = {0, 0, 0};   // exponents of dz2, dz1, dz0
+  bool wild = false;
+  if constexpr (F16) {
+    const float* st = packed + T::STATS_BASE;
+    float bound = 2.0f;   // of the normalised logits' gradients
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+      wild = wild || !tame(st[l]) || !tame(st[4 + l]) || !tame(st[8 + l]) ||
+             !(st[12 + l] <= 0x1p60f);
+      ew[l] = tame_exponent(st[l]);
+      rowsum[l] = st[4 + l];
+      maxb[l] = st[12 + l];
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {   // dz2 through the head, dz1 through W_2, dz0 through W_1
+      bound = bound * st[8 + 3 - k];
+      wild = wild || !tame(bound);
+      ez[k] = tame_exponent(bound);
+    }
+  }
+  // the head's weights: parts in LDS (operand of the logits), FP32 columns of
+  // this lane's feature (its input gradient)
+  for (int i = threadIdx.x; i < 4 * 4 * 4 * 4; i += kBwdBlock) {
+    // pair p of logit o, k-tile kt, group gg: features 32 kt + {4 gg + ..}
+    const int p = i & 3, o = (i >> 2) & 3, gg = (i >> 4) & 3, kt = i >> 6;
+    const int j = 2 * p, f = 32 * kt + (j < 4 ? 4 * gg + j : 16 + 4 * gg + j - 4);
+    // packed head fragment mt, lane (o, c) = W[o][16 mt + c]
+    const float* WT = packed + T::T_BASE + T::T_HEAD * 64;
+    const float a = WT[(f >> 4) * 64 + o * 16 + (f & 15)];
+    const float b = WT[((f + 1) >> 4) * 64 + o * 16 + ((f + 1) & 15)];
+    const float s = F16 ? f16_scale(ew[3]) : 1.0f;
+    unsigned int hi, lo;
+    parts2<F16>(a, b, s, s, hi, lo);
+    *reinterpret_cast<unsigned int*>(&S.head[0][kt][gg][o][j]) = hi;
+    *reinterpret_cast<unsigned int*>(&S.head[1][kt][gg][o][j]) = lo;
+  }
+  // this lane's biases (feature c of the wave's, logit c of the head) and head
+  // weights
+  float bl[3], bh;
+#pragma unroll
+  for (int l = 0; l < 3; ++l) bl[l] = bias[l * H + 16 * w + c];
+  bh = bias[L * H + (c & 3)];
+  float wh[4];
+#pragma unroll
+  for (int o = 0; o < 4; ++o)
+    wh[o] = packed[T::T_BASE + (T::T_HEAD + w) * 64 + o * 16 + c];
+  if (threadIdx.x == 0) S.wild = 0;
+  for (int i = threadIdx.x; i < kBwdChunk; i += kBwdBlock) S.top0[i] = 0;
+
+  const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 gw2[2][4], gw1[2][4], gw0[1][2], gh = zero4;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) gw2[a][b] = gw1[a][b] = zero4;
+  gw0[0][0] = gw0[0][1] = zero4;
+  float gb[3] = {0.0f, 0.0f, 0.0f}, ghb = 0.0f;
+
+  const int64_t chunks = (M + kBwdChunk - 1) / kBwdChunk;
+  // the chunk's features: thread (sample, features 4 j..) = threadIdx / 8, % 8
+  const int xs = threadIdx.x >> 3, xj = threadIdx.x & 7;
+  float4 xin = {0.0f, 0.0f, 0.0f, 0.0f};
+  const auto load_x = [&](int64_t ch) {
+    const int64_t s = ch * kBwdChunk + xs;
+    xin = (ch < chunks && s < M) ? *reinterpret_cast<const float4*>(emb + s * D + 4 * xj)
+                                 : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  };
+  load_x(blockIdx.x);
+  __syncthreads();
+
+  for (int64_t ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
+    const int64_t s0 = ch * kBwdChunk;
+    const float sign = (ch / gridDim.x) & 1 ? -1.0f : 1.0f;   // of the chunk's weight gradients
+    // the lane index as a value of this step: the addresses formed from it
+    // would otherwise be kept from step to step, and spilled
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int g = lane >> 4, c = lane & 15;
+    // lane addresses in a plane: transposing (layers, per sample tile), own
+    // store (feature row 16 w + c, samples 4 g of each tile), rows of the weight
+    // gradients (row c, samples 8 g of each half)
+    int at_tr[4], at_out[4], at_row[2];
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      at_tr[m] = bwd_at(4 * g + (c >> 2), 16 * m + 4 * (c & 3));
+      at_out[m] = 16 * w * kBwdRow + bwd_at(c, 16 * m + 4 * g);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) at_row[ks] = bwd_at(c, 32 * ks + 8 * g);
+    // global memory for certain: behind opaque() the address would be generic,
+    // and a generic load also waits for the LDS
+    const global_u32x4 F = (global_u32x4)opaque(frags);
+    // ---- the features' parts and the sample's scales
+    {
+      float sx = 1.0f;
+      if constexpr (F16) {
+        int m = 0;
+        m = max(m, __float_as_int(xin.x) & 0x7FFFFFFF);
+        m = max(m, __float_as_int(xin.y) & 0x7FFFFFFF);
+        m = max(m, __float_as_int(xin.z) & 0x7FFFFFFF);
+        m = max(m, __float_as_int(xin.w) & 0x7FFFFFFF);
+        m = max(m, __builtin_amdgcn_mov_dpp(m, 0xB1, 0xF, 0xF, true));
+        m = max(m, __builtin_amdgcn_mov_dpp(m, 0x4E, 0xF, 0xF, true));
+        m = max(m, __builtin_amdgcn_mov_dpp(m, 0x141, 0xF, 0xF, true));
+        const float xm = __int_as_float(m);
+        wild = wild || !tame(xm);
+        const int ex = tame_exponent(xm);
+        sx = f16_scale(ex);
+        const float t0 = __fmaf_rn(rowsum[0], xm, maxb[0]) * 1.001f;
+        const float t1 = __fmaf_rn(rowsum[1], t0, maxb[1]) * 1.001f;
+        wild = wild || !(t0 <= 0x1p60f) || !(t1 <= 0x1p60f);
+        const int e0 = tame_exponent(t0), e1 = tame_exponent(t1);
+        if (xj == 0) {
+          S.back[0][xs] = f16_unscale(ex) * f16_unscale(ew[0]);
+          S.scale[0][xs] = f16_scale(e0);
+          S.back[1][xs] = f16_unscale(e0) * f16_unscale(ew[1]);
+          S.scale[1][xs] = f16_scale(e1);
+          S.back[2][xs] = f16_unscale(e1) * f16_unscale(ew[2]);
+        }
+      }
+      unsigned int h0, l0, h1, l1;
+      parts2<F16>(xin.x, xin.y, sx, sx, h0, l0);
+      parts2<F16>(xin.z, xin.w, sx, sx, h1, l1);
+      const unsigned int hv[2] = {h0, h1}, lv[2] = {l0, l1};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        unsigned short* q = &S.x0[bwd_at(4 * xj + k, xs)];
+        q[0] = static_cast<unsigned short>(hv[k >> 1] >> 16 * (k & 1));
+        q[kBwdPlane0] = static_cast<unsigned short>(lv[k >> 1] >> 16 * (k & 1));
+      }
+    }
+    BwdFrags<1> f0;
+    f0.load(F + 128 * w, lane);
+    load_x(ch + gridDim.x);
+    // the outputs' gradients that waves 0-3 need at the head
+    float dy[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (w < 4) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t s = s0 + 16 * w + 4 * g + r;
+        if (s < M) dy[r] = dout[s * 4 + (c & 3)];
+      }
+    }
+    BwdFrags<4> f;
+    __syncthreads();
+
+    // relu(z) of an accumulator into plane set l, the mask bits, and (F16) the
+    // samples' largest value for layer 0
+    unsigned int mask[3];
+    const auto forward_out = [&](f32x4 (&acc)[4], int l) {
+      unsigned int bits = 0;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        f32x4 sc = {1.0f, 1.0f, 1.0f, 1.0f};
+        float h[4];
+        if constexpr (F16) {
+          const f32x4 bk = *reinterpret_cast<const f32x4*>(&S.back[l][16 * m + 4 * g]);
+          sc = *reinterpret_cast<const f32x4*>(&S.scale[l][16 * m + 4 * g]);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) h[r] = fmaxf(__fmaf_rn(acc[m][r], bk[r], bl[l]), 0.0f);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) h[r] = relu_bits(acc[m][r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) bits |= (h[r] > 0.0f ? 1u : 0u) << (4 * m + r);
+        u32x2 hi, lo;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          unsigned int hw, lw;
+          parts2<F16>(h[2 * p], h[2 * p + 1], sc[2 * p], sc[2 * p + 1], hw, lw);
+          hi[p] = hw;
+          lo[p] = lw;
+        }
+        *reinterpret_cast<u32x2*>(&S.t[l][at_out[m]]) = hi;
+        *reinterpret_cast<u32x2*>(&S.t[l][kBwdPlane + at_out[m]]) = lo;
+        if constexpr (F16) {
+          if (l == 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int top = row_max15(__float_as_int(h[r]));
+              if (c == 15) atomicMax(&S.top0[16 * m + 4 * g + r], top);
+            }
+          }
+        }
+        tile_fence();
+      }
+      mask[l] = bits;
+    };
+    const auto start = [&](f32x4 (&acc)[4], int l) {
+      // BF16: the bias is the initial accumulator, as in the forward kernel
+      const float b = F16 ? 0.0f : bl[l];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) acc[m] = f32x4{b, b, b, b};
+    };
+
+    // ---- layers 0, 1, 2
+    f32x4 acc[4];
+    start(acc, 0);
+    bwd_layer<F16, 1>(S.x0, at_tr, kBwdPlane0, f0, acc);
+    f.load(F + 128 * (T::X_HIDDEN + w * T::KXH), lane);
+    forward_out(acc, 0);
+    __syncthreads();
+    if constexpr (F16) {
+      // h2's scale, two layers past the sample's largest h0
+      if (threadIdx.x < kBwdChunk) {
+        const float t1 = __fmaf_rn(rowsum[1], __int_as_float(S.top0[threadIdx.x]), maxb[1]);
+        const float t2 = __fmaf_rn(rowsum[2], t1 * 1.001f, maxb[2]) * 1.001f;
+        wild = wild || !(t2 <= 0x1p60f);
+        const int e2 = tame_exponent(t2);
+        S.scale[2][threadIdx.x] = f16_scale(e2);
+        S.back[3][threadIdx.x] = f16_unscale(e2) * f16_unscale(ew[3]);
+      }
+    }
+    start(acc, 1);
+    bwd_layer<F16, 4>(S.t[0], at_tr, kBwdPlane, f, acc);
+    f.load(F + 128 * (T::X_HIDDEN + (T::MT + w) * T::KXH), lane);
+    forward_out(acc, 1);
+    __syncthreads();
+    start(acc, 2);
+    bwd_layer<F16, 4>(S.t[1], at_tr, kBwdPlane, f, acc);
+    // W_2^T for dz1
+    f.load(F + 128 * (T::X_THIDDEN + (T::MT + w) * T::KXH), lane);
+    forward_out(acc, 2);
+    __syncthreads();
+
+    // ---- the head: wave m takes samples 16 m..; lanes c < 4 hold logit c of
+    // samples 4 g + r
+    if (w < 4) {
+      f32x4 z = zero4;
+      if constexpr (!F16) {
+        z = f32x4{bh, bh, bh, bh};
+      }
+      const int at_w = bwd_at(4 * g + (c >> 2), 16 * w + 4 * (c & 3));
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        const unsigned short* p = &S.t[2][at_w + kt * 32 * kBwdRow];
+        const u32x4 ah = lds_tr(p), al = lds_tr(p + kBwdPlane);
+        const u32x4 bh = lds128(S.head[0][kt][g][c & 3]), bl = lds128(S.head[1][kt][g][c & 3]);
+        z = mm16x3<F16>(ah, al, bh, bl, z);
+      }
+      if constexpr (F16) {
+        const f32x4 bk = *reinterpret_cast<const f32x4*>(&S.back[3][16 * w + 4 * g]);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) z[r] = __fmaf_rn(z[r], bk[r], bh);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = 16 * w + 4 * g + r;
+        const float d = dy[r];
+        const float y = logistic(z[r]);
+        float v = (c & 3) == 0 ? d : d * (y * (1.0f - y));
+        if (c < 4) ghb += v;
+        if constexpr (F16) {
+          int m = __float_as_int(v) & 0x7FFFFFFF;
+          m = max(m, __builtin_amdgcn_mov_dpp(m, 0xB1, 0xF, 0xF, true));
+          m = max(m, __builtin_amdgcn_mov_dpp(m, 0x4E, 0xF, 0xF, true));
+          const int e = max(m >> 23, 1);
+          wild = wild || e > kTameHigh;
+          // 2^(127 - e) and back, negative for odd samples
+          const int odd = int(uint32_t(r & 1) << 31);
+          v = v * __int_as_float(((254 - min(e, 253)) << 23) | odd);
+          if (c == 0) S.unit[i] = m == 0 ? 0.0f : __int_as_float((min(e, 253) << 23) | odd);
+        }
+        if (c < 4) S.dl[i][c] = v;
+      }
+    }
+    __syncthreads();
+
+    // the samples' factors (lane = sample): exponents q of the normalised
+    // gradient times a layer's input, the chunk's largest, and the factors
+    // relative to it -- every wave the head's, one wave each of the others
+    int top[4] = {0, 0, 0, 0};
+    if constexpr (F16) {
+      const float u = S.unit[lane];
+      const int e = (__float_as_int(u) & 0x7FFFFFFF) >> 23;
+      const float us = copysignf(sign, u * sign);   // the sample's sign times the chunk's
+      int q[4];
+      q[0] = e + feature_exponent(S.back[0][lane], ew[0]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) q[k + 1] = e + 268 - (__float_as_int(S.scale[k][lane]) >> 23);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int m = u == 0.0f ? 0 : q[k];   // exponents are positive
+        top[k] = __builtin_amdgcn_readlane(row_max15(m), 15);
+#pragma unroll
+        for (int r = 1; r < 4; ++r)
+          top[k] = max(top[k], __builtin_amdgcn_readlane(row_max15(m), 16 * r + 15));
+        const int d = q[k] - top[k];
+        if (k < 3) {
+          if (w == k)
+            S.factor[k][lane] =
+                u == 0.0f ? _Float16(0.0f)
+                          : _Float16(us * __int_as_float((127 + max(d, -40)) << 23));
+        } else {   // 2^(13 + d), 0 far below
+          S.factor2[lane] = u == 0.0f ? 0.0f : us * __int_as_float(max(140 + d, 0) << 23);
+        }
+      }
+      wave_sync();   // factor2: every wave writes the same values and reads them
+    }
+    // ---- dz of a layer's accumulator (values v, sample 16 m + 4 g + r) into
+    // plane set `to`; the bias gradient in true units
+    const auto dz_out = [&](float (&v)[4][4], unsigned int bits, int to, int l, float sz) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        f32x4 u = {1.0f, 1.0f, 1.0f, 1.0f};
+        if constexpr (F16) u = *reinterpret_cast<const f32x4*>(&S.unit[16 * m + 4 * g]);
+        u32x2 hi, lo;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[m][r] = (bits >> (4 * m + r)) & 1u ? v[m][r] : 0.0f;
+          gb[l] = F16 ? __fmaf_rn(v[m][r], u[r], gb[l]) : gb[l] + v[m][r];
+        }
+        asm volatile("" : "+v"(gb[l]));
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          unsigned int hw, lw;
+          parts2<F16>(v[m][2 * p], v[m][2 * p + 1], sz, sz, hw, lw);
+          hi[p] = hw;
+          lo[p] = lw;
+        }
+        *reinterpret_cast<u32x2*>(&S.t[to][at_out[m]]) = hi;
+        *reinterpret_cast<u32x2*>(&S.t[to][kBwdPlane + at_out[m]]) = lo;
+        tile_fence();
+      }
+    };
+    // ---- dz2 = mask (W_head^T dl) in FP32, and dW_head
+    {
+      float v[4][4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float4 d = *reinterpret_cast<const float4*>(S.dl[16 * m + 4 * g + r]);
+          v[m][r] = __fmaf_rn(wh[3], d.w, __fmaf_rn(wh[2], d.z, __fmaf_rn(wh[1], d.y, wh[0] * d.x)));
+          if (r == 3) tile_fence();
+        }
+      dz_out(v, mask[2], 3, 2, F16 ? f16_scale(ez[0]) : 1.0f);
+    }
+    f32x4 ghc = zero4;
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      // dl of logit c (lanes c < 4) for samples 32 ks + 8 g + i, with their factors
+      unsigned int hw[4], lw[4];
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        float v[2], s[2] = {1.0f, 1.0f};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int i = 32 * ks + 8 * g + 2 * p + k;
+          v[k] = c < 4 ? S.dl[i][c & 3] : 0.0f;
+          if constexpr (F16) s[k] = S.factor2[i];
+        }
+        parts2<F16>(v[0], v[1], s[0], s[1], hw[p], lw[p]);
+      }
+      const unsigned short* pb = &S.t[2][16 * w * kBwdRow + at_row[ks]];
+      ghc = mm16x3<F16>(u32x4{hw[0], hw[1], hw[2], hw[3]}, u32x4{lw[0], lw[1], lw[2], lw[3]},
+                        lds128(pb), lds128(pb + kBwdPlane), ghc);
+      tile_fence();
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      gh[r] = F16 ? __fmaf_rn(__builtin_amdgcn_ldexpf(ghc[r], top[3] + 128 - 409), sign, gh[r])
+                  : gh[r] + ghc[r];
+    asm volatile("" : "+v"(gh));
+    __syncthreads();
+    if (threadIdx.x < kBwdChunk) S.top0[threadIdx.x] = 0;
+
+    const int row2 = 32 * (w & 3) * kBwdRow, col2 = 64 * (w >> 2) * kBwdRow;
+    // ---- dW_2 (dz2 x h1); dz1 = mask (W_2^T dz2) into h2's planes
+#pragma unroll
+    for (int m = 0; m < 4; ++m) acc[m] = zero4;
+    bwd_layer<F16, 4>(S.t[3], at_tr, kBwdPlane, f, acc);
+    f.load(F + 128 * (T::X_THIDDEN + w * T::KXH), lane);
+    bwd_dw<F16, 2, 4>(&S.t[3][row2], kBwdPlane, &S.t[1][col2], kBwdPlane, at_row, S.factor[2], g,
+                      top[2] + ez[0] - 409, sign, gw2);
+    {
+      const float bk = F16 ? f16_unscale(ez[0]) * f16_unscale(ew[2]) : 1.0f;
+      float v[4][4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[m][r] = F16 ? acc[m][r] * bk : acc[m][r];
+      dz_out(v, mask[1], 2, 1, F16 ? f16_scale(ez[1]) : 1.0f);
+    }
+    __syncthreads();
+    // ---- dW_1 (dz1 x h0); dz0 = mask (W_1^T dz1) into dz2's planes
+#pragma unroll
+    for (int m = 0; m < 4; ++m) acc[m] = zero4;
+    bwd_layer<F16, 4>(S.t[2], at_tr, kBwdPlane, f, acc);
+    // W_0^T: the input gradient's tile w & 1 (features) of samples 16 (w / 2)..
+    f.load(F + 128 * (T::X_T0 + (w & 1) * T::KXH), lane);
+    bwd_dw<F16, 2, 4>(&S.t[2][row2], kBwdPlane, &S.t[0][col2], kBwdPlane, at_row, S.factor[1], g,
+                      top[1] + ez[1] - 409, sign, gw1);
+    {
+      const float bk = F16 ? f16_unscale(ez[1]) * f16_unscale(ew[1]) : 1.0f;
+      float v[4][4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[m][r] = F16 ? acc[m][r] * bk : acc[m][r];
+      dz_out(v, mask[0], 3, 0, F16 ? f16_scale(ez[2]) : 1.0f);
+    }
+    __syncthreads();
+    // ---- dW_0 (dz0 x features) and the input gradient W_0^T dz0, whose
+    // products run as W X so that a lane holds 4 features of a sample
+    {
+      const int m = w >> 1;
+      const int at_m = bwd_at(4 * g + (c >> 2), 16 * m + 4 * (c & 3));
+      f32x4 d = zero4;
+#pragma unroll
+      for (int kt = 0; kt < 4; ++kt) {
+        const unsigned short* p = &S.t[3][at_m + kt * 32 * kBwdRow];
+        d = mm16x3<F16>(f.h[kt], f.l[kt], lds_tr(p), lds_tr(p + kBwdPlane), d);
+      }
+      const int i = 16 * m + c;
+      if constexpr (F16) d = (d * (f16_unscale(ez[2]) * f16_unscale(ew[0]))) * S.unit[i];
+      if (s0 + i < M)
+        *reinterpret_cast<f32x4*>(demb + (s0 + i) * D + 16 * (w & 1) + 4 * g) = d;
+    }
+    bwd_dw<F16, 1, 2>(&S.t[3][16 * w * kBwdRow], kBwdPlane, S.x0, kBwdPlane0, at_row, S.factor[0], g,
+                      top[0] + ez[2] - 409, sign, gw0);
+    __syncthreads();
+  }
+
+  // ---- the block's partial sums, in torch order
+  if (wild) S.wild = 1;
+  float* P = partial + int64_t(blockIdx.x) * T::PARAMS;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int64_t o = int64_t(32 * (w & 3) + 16 * a + 4 * g + r) * H + 64 * (w >> 2) + 16 * b + c;
+        P[T::P_LAYER1 + o] = gw1[a][b][r];
+        P[T::P_LAYER1 + int64_t(H) * H + H + o] = gw2[a][b][r];
+      }
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+      P[T::P_W0 + int64_t(16 * w + 4 * g + r) * D + 16 * b + c] = gw0[0][b][r];
+    if (g == 0) P[T::P_HEAD + int64_t(r) * H + 16 * w + c] = gh[r];
+  }
+#pragma unroll
+  for (int l = 0; l < 3; ++l) {
+    float v = gb[l];
+    v = v + __shfl_xor(v, 16, 64);
+    v = v + __shfl_xor(v, 32, 64);
+    const int64_t at = l == 0 ? T::P_B0 : T::P_LAYER1 + (l - 1) * (int64_t(H) * H + H) + int64_t(H) * H;
+    if (g == 0) P[at + 16 * w + c] = v;
+  }
+  // the head's bias: waves 0-3 hold their samples' sums (lanes c < 4)
+  ghb = ghb + __shfl_xor(ghb, 16, 64);
+  ghb = ghb + __shfl_xor(ghb, 32, 64);
+  if (w < 4 && lane < 4) S.dl[w][lane] = ghb;
+  __syncthreads();
+  if (threadIdx.x < 4)
+    P[T::P_HEAD + 4 * H + threadIdx.x] =
+        ((S.dl[0][threadIdx.x] + S.dl[1][threadIdx.x]) + S.dl[2][threadIdx.x]) + S.dl[3][threadIdx.x];
+  if (F16 && threadIdx.x == 0) flags[blockIdx.x] = S.wild;
+}
+
+// dparams[p] = the sum over blocks of partial[b][p], in a fixed order: lane
+// group j of a block's 16 adds blocks j, j + 16, ..., four loads in flight, and
+// the 16 sums are added in order.  nb16 partials, or nb32 where a flag is set.
+// A thread per parameter waited for nb loads one by one: 61 us for 256
+// partials, now 16.
+constexpr int kSumCols = 16;   // parameters per block
+__global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restrict__ partial,
+                                                           int nb16, int nb32, int64_t P,
+                                                           const int32_t* __restrict__ flags,
+                                                           float* __restrict__ dparams) {
+  __shared__ float sums[16][kSumCols];
+  int flagged = 0;
+  if (flags)
+    for (int i = threadIdx.x; i < nb16; i += 256) flagged |= flags[i];
+  const int nb = __syncthreads_or(flagged) ? nb32 : nb16;
+  const int j = threadIdx.x / kSumCols, q = threadIdx.x % kSumCols;
+  const int64_t p = int64_t(blockIdx.x) * kSumCols + q;
+  float acc = 0.0f;
+  if (p < P) {
+    int b = j;
+    for (; b + 48 < nb; b += 64) {
+      const float v0 = partial[int64_t(b) * P + p], v1 = partial[int64_t(b + 16) * P + p];
+      const float v2 = partial[int64_t(b + 32) * P + p], v3 = partial[int64_t(b + 48) * P + p];
+      acc = (((acc + v0) + v1) + v2) + v3;
+    }
+    for (; b < nb; b += 16) acc = acc + partial[int64_t(b) * P + p];
+  }
+  sums[j][q] = acc;
+  __syncthreads();
+  if (j == 0 && p < P) {
+#pragma unroll
+    for (int k = 1; k < 16; ++k) acc = acc + sums[k][q];
+    dparams[p] = acc;
+  }
+}
+
+// The layers' weights and biases, device pointers.
+struct TrainLayers {
+  const float* w[8];
+  const float* b[8];
+};
+
+// Block l: layer l's largest |w|, row sum |w|, column sum |w| and |b| (not
+// finite where a value is not).
+template <int D, int H, int L>
+__global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
+                                                         float* __restrict__ stats) {
+  __shared__ int best[4];
+  __shared__ float cols[H];
+  const int l = blockIdx.x, rows = l < L ? H : 4, in = l == 0 ? D : H;
+  const float* W = net.w[l];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  if (threadIdx.x < 4) best[threadIdx.x] = 0;
+  if (threadIdx.x < H) cols[threadIdx.x] = 0.0f;
+  __syncthreads();
+  // |x| as integer bits order as the values do, NaN and infinity on top
+  const auto up = [&](int k, float v) {
+    int m = __float_as_int(v) & 0x7FFFFFFF;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) m = max(m, __shfl_xor(m, d, 64));
+    if (lane == 0) atomicMax(&best[k], m);
+  };
+  // a wave's rows, all loads in flight
+  constexpr int R = H / 16;
+  float v[R][H / 64];
+#pragma unroll
+  for (int i = 0; i < R; ++i)
+#pragma unroll
+    for (int q = 0; q < H / 64; ++q) {
+      const int r = wave + 16 * i, k = lane + 64 * q;
+      v[i][q] = r < rows && k < in ? fabsf(W[r * in + k]) : 0.0f;
+    }
+  float top = 0.0f, widest = 0.0f;
+  float mine[H / 64] = {};
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int q = 0; q < H / 64; ++q) {
+      top = __int_as_float(max(__float_as_int(top), __float_as_int(v[i][q])));
+      mine[q] += v[i][q];
+      sum += v[i][q];
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    widest = __int_as_float(max(__float_as_int(widest), __float_as_int(sum) & 0x7FFFFFFF));
+  }
+  up(1, widest);
+  up(0, top);
+#pragma unroll
+  for (int q = 0; q < H / 64; ++q) atomicAdd(&cols[lane + 64 * q], mine[q]);
+  float b = 0.0f;
+  for (int i = threadIdx.x; i < rows; i += 1024)
+    b = __int_as_float(max(__float_as_int(b), __float_as_int(net.b[l][i]) & 0x7FFFFFFF));
+  up(3, b);
+  __syncthreads();
+  up(2, threadIdx.x < H ? cols[threadIdx.x] : 0.0f);
+  __syncthreads();
+  // row and column sums a little above their rounding
+  if (threadIdx.x < 4) {
+    const float v = __int_as_float(best[threadIdx.x]);
+    stats[threadIdx.x * (L + 1) + l] = threadIdx.x == 1 || threadIdx.x == 2 ? v * 1.001f : v;
+  }
+}
+
+// Element e (of 64 lanes x 8) of the 16-bit kernels' fragment f, in the order
+// of TrainDims::X_* and then the head's forward fragments: lane (g, c) of
+// fragment (mt, kt) holds W[16 mt + c][32 kt + 4 g + i, + 16 for i >= 4] of its
+// layer, or of the layer's transpose.
+template <int D, int H, int L>
+__device__ __forceinline__ float fragment_value(const TrainLayers& net, int f, int lane, int i,
+                                                int* layer) {
+  using T = TrainDims<D, H, L>;
+  bool transposed = false;
+  int l, n, KT;
+  if (f < T::X_HIDDEN) {
+    l = 0, n = f, KT = T::KX0;
+  } else if (f < T::X_T0) {
+    n = f - T::X_HIDDEN, l = 1 + n / (T::MT * T::KXH), n %= T::MT * T::KXH, KT = T::KXH;
+  } else if (f < T::X_THIDDEN) {
+    transposed = true, l = 0, n = f - T::X_T0, KT = T::KXH;
+  } else if (f < T::X_FRAGS) {
+    transposed = true;
+    n = f - T::X_THIDDEN, l = 1 + n / (T::MT * T::KXH), n %= T::MT * T::KXH, KT = T::KXH;
+  } else {
+    l = L, n = f - T::X_FRAGS, KT = T::KXH;
+  }
+  *layer = l;
+  const int g = lane >> 4, c = lane & 15;
+  const int row = 16 * (n / KT) + c, col = 32 * (n % KT) + 4 * g + (i & 3) + (i >= 4 ? 16 : 0);
+  const int in = l == 0 ? D : H;
+  if (transposed) return net.w[l][col * in + row];
+  return l == L && row >= 4 ? 0.0f : net.w[l][row * in + col];
+}
+
+// Packs the weights: the FP32 fragments of TrainDims (forward, then
+// transposed), the biases, and the FP16 fragments scaled by the layers' power
+// of two (stats: mlp_stats_kernel's, in `packed`).  Thread per float.
+//   forward [ceil(Hout/16)][Hin/4][64], lane (g, c) of fragment (mt, 4t + i)
+//     = W[16 mt + c][16 t + 4 g + i] (0 past Hout);
+//   transposed [Hin/16][Hout/4][64], lane (g, c) of fragment (mt, 4t + i)
+//     = W[16 t + 4 g + i][16 mt + c];
+//   transposed head [Hin/16][64], lane (g, c) of fragment mt = W[g][16 mt + c].
+// One launch (after the stats') where each layer and form and each bias took
+// one of its own: 25 -> 17 us per call, 2 launches instead of 12.
+template <int D, int H, int L>
+__global__ __launch_bounds__(256) void mlp_pack_kernel(TrainLayers net,
+                                                       float* __restrict__ packed) {
+  using T = TrainDims<D, H, L>;
+  const int64_t p = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (p >= T::PACKED || (p >= T::STATS_BASE && p < T::F16_BASE)) return;
+  if (p >= T::F16_BASE) {
+    // pairs of parts: thread = (fragment, part, lane, pair)
+    const int64_t q = p - T::F16_BASE;
+    const int f = int(q / 512), part = int(q / 256) & 1, lane = int(q / 4) & 63, i = 2 * int(q & 3);
+    int l;
+    const float a = fragment_value<D, H, L>(net, f, lane, i, &l);
+    const float b = fragment_value<D, H, L>(net, f, lane, i + 1, &l);
+    const float s = f16_scale(min(f16_exponent(packed[T::STATS_BASE + l]), 254));
+    f16x2 hi, lo;
+    f16_split2(a, b, s, s, hi, lo);
+    packed[p] = __builtin_bit_cast(float, part ? lo : hi);
+    return;
+  }
+  if (p >= T::BIAS_BASE) {
+    const int q = int(p - T::BIAS_BASE), l = min(q / H, L);
+    packed[p] = net.b[l][q - l * H];
+    return;
+  }
+  const bool transposed = p >= T::T_BASE;
+  const int64_t q = transposed ? p - T::T_BASE : p;
+  const int lane = int(q & 63), g = lane >> 4, c = lane & 15;
+  int n = int(q >> 6), l, KT;
+  if (!transposed) {
+    if (n < T::F_HIDDEN) {
+      l = 0, KT = T::KT0;
+    } else {
+      n -= T::F_HIDDEN, l = min(1 + n / (T::MT * T::KTH), L), n -= (l - 1) * T::MT * T::KTH;
+      KT = T::KTH;
+    }
+    const int row = 16 * (n / KT) + c, kt = n % KT, in = l == 0 ? D : H;
+    packed[p] = l == L && row >= 4 ? 0.0f : net.w[l][row * in + 16 * (kt >> 2) + 4 * g + (kt & 3)];
+    return;
+  }
+  if (n >= T::T_HEAD) {
+    packed[p] = net.w[L][g * H + 16 * (n - T::T_HEAD) + c];
+    return;
+  }
+  if (n < T::T_HIDDEN) {
+    l = 0;
+  } else {
+    n -= T::T_HIDDEN, l = 1 + n / (T::MT * T::KTH), n %= T::MT * T::KTH;
+  }
+  const int mt = n / T::KTH, kt = n % T::KTH, in = l == 0 ? D : H;
+  packed[p] = net.w[l][(16 * (kt >> 2) + 4 * g + (kt & 3)) * in + 16 * mt + c];
 }
 
 template <int D, int H, int L>
 int pack_impl(const float* const* weights, const float* const* biases, float* packed,
               hipStream_t st) {
   using T = TrainDims<D, H, L>;
-  auto launch = [&](const float* W, int Hout, int Hin, int mode, float* dst, int64_t n) {
-    hipLaunchKernelGGL(pack_layer_kernel, dim3(unsigned(ceil_div(n, 256))), dim3(256), 0, st, W,
-                       Hout, Hin, mode, dst, n);
-  };
-  launch(weights[0], H, D, 0, packed, int64_t(T::MT) * T::KT0 * 64);
-  for (int l = 1; l < L; ++l)
-    launch(weights[l], H, H, 0, packed + (int64_t(T::F_HIDDEN) + (l - 1) * T::MT * T::KTH) * 64,
-           int64_t(T::MT) * T::KTH * 64);
-  launch(weights[L], 4, H, 0, packed + int64_t(T::F_HEAD) * 64, int64_t(T::KTH) * 64);
-  float* Tp = packed + T::T_BASE;
-  launch(weights[0], H, D, 1, Tp, int64_t(T::MT0) * T::KTH * 64);
-  for (int l = 1; l < L; ++l)
-    launch(weights[l], H, H, 1, Tp + (int64_t(T::T_HIDDEN) + (l - 1) * T::MT * T::KTH) * 64,
-           int64_t(T::MT) * T::KTH * 64);
-  launch(weights[L], 4, H, 2, Tp + int64_t(T::T_HEAD) * 64, int64_t(T::MT) * 64);
-  if (check_launch("mlp_train_pack") != NSVF_OK) return NSVF_ELAUNCH;
-  float* bias = packed + T::BIAS_BASE;
+  static_assert(L + 1 <= 8, "TrainLayers");
+  TrainLayers net{};
   for (int l = 0; l <= L; ++l) {
-    const hipError_t e = hipMemcpyAsync(bias + int64_t(l) * H, biases[l],
-                                        sizeof(float) * (l < L ? H : 4),
-                                        hipMemcpyDeviceToDevice, st);
-    if (e != hipSuccess)
-      return set_error(NSVF_ELAUNCH, "mlp_train_pack: bias copy: %s", hipGetErrorString(e));
+    net.w[l] = weights[l];
+    net.b[l] = biases[l];
   }
-  return NSVF_OK;
+  hipLaunchKernelGGL((mlp_stats_kernel<D, H, L>), dim3(L + 1), dim3(1024), 0, st, net,
+                     packed + T::STATS_BASE);
+  if (check_launch("mlp_train_stats") != NSVF_OK) return NSVF_ELAUNCH;
+  hipLaunchKernelGGL((mlp_pack_kernel<D, H, L>), dim3(unsigned(ceil_div(T::PACKED, 256))),
+                     dim3(256), 0, st, net, packed);
+  return check_launch("mlp_train_pack");
 }
 
-int backward_blocks(int64_t M) {
-  return int(std::max<int64_t>(1, std::min<int64_t>(ceil_div(M, kTrainChunk), kMaxTrainBlocks)));
+// Blocks (and partials) of the 16-bit backward kernel and of the FP32 one.
+int backward_blocks(int64_t M, int64_t chunk) {
+  return int(std::max<int64_t>(1, std::min<int64_t>(ceil_div(M, chunk), kMaxTrainBlocks)));
 }
 
 constexpr size_t kBackwardLds = size_t(2) * kTrainChunk * kLdsRow * sizeof(float);
-constexpr size_t kBackwardLdsX3 = size_t(4) * kXPlane * sizeof(unsigned short);
 
 bool train_shape_ok(int D, int H, int L) { return D == 32 && H == 128 && L == 3; }
 
@@ -825,7 +1428,9 @@ int64_t nsvf_mlp_train_param_floats(int D, int H, int L) {
 
 int64_t nsvf_mlp_train_partial_floats(int D, int H, int L, int64_t M) {
   if (!train_shape_ok(D, H, L) || M < 0) return -1;
-  return int64_t(backward_blocks(M)) * TrainDims<32, 128, 3>::PARAMS;
+  // the blocks' partial sums, then their flags
+  const int64_t nb = backward_blocks(M, kBwdChunk);
+  return nb * TrainDims<32, 128, 3>::PARAMS + (M > 0 ? nb : 0);
 }
 
 int nsvf_mlp_train_pack(int D, int H, int L, const float* const* weights,
@@ -874,24 +1479,31 @@ static int train_backward(const char* name, int D, int H, int L, const float* pa
   if (!packed || !partial || !dparams || (M > 0 && (!emb || !dout || !demb)))
     return set_error(NSVF_EINVAL, "%s: null pointer", name);
   using T = TrainDims<32, 128, 3>;
-  const int nb = backward_blocks(M);
-  if (partial_floats < int64_t(nb) * T::PARAMS)
+  const int64_t need = nsvf_mlp_train_partial_floats(D, H, L, M);
+  if (partial_floats < need)
     return set_error(NSVF_EINVAL, "%s: partial buffer of %lld floats, %lld needed", name,
-                     static_cast<long long>(partial_floats),
-                     static_cast<long long>(int64_t(nb) * T::PARAMS));
+                     static_cast<long long>(partial_floats), static_cast<long long>(need));
   hipStream_t st = as_stream(stream);
-  const bf16x8* x3 = reinterpret_cast<const bf16x8*>(x3w);
-  if (x3w)
-    hipLaunchKernelGGL((mlp_train_backward_kernel<32, 128, 3, true>), dim3(nb),
-                       dim3(kTrainBlock), kBackwardLdsX3, st, emb, M, packed, x3, dout, demb,
-                       partial);
-  else
-    hipLaunchKernelGGL((mlp_train_backward_kernel<32, 128, 3, false>), dim3(nb),
-                       dim3(kTrainBlock), kBackwardLds, st, emb, M, packed, x3, dout, demb,
-                       partial);
-  if (check_launch(name) != NSVF_OK) return NSVF_ELAUNCH;
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(unsigned(ceil_div(T::PARAMS, 256))), dim3(256), 0,
-                     st, partial, nb, T::PARAMS, dparams);
+  const int nb = backward_blocks(M, kBwdChunk), nb32 = backward_blocks(M, kTrainChunk);
+  int32_t* flags = x3w || M == 0 ? nullptr
+                                 : reinterpret_cast<int32_t*>(partial + int64_t(nb) * T::PARAMS);
+  if (x3w || M == 0) {
+    hipLaunchKernelGGL((mlp_train_backward_kernel<32, 128, 3, false>), dim3(nb), dim3(kBwdBlock),
+                       sizeof(BwdLds), st, emb, M, packed, reinterpret_cast<const u32x4*>(x3w),
+                       dout, demb, partial, flags);
+    if (check_launch(name) != NSVF_OK) return NSVF_ELAUNCH;
+  } else {
+    hipLaunchKernelGGL((mlp_train_backward_kernel<32, 128, 3, true>), dim3(nb), dim3(kBwdBlock),
+                       sizeof(BwdLds), st, emb, M, packed,
+                       reinterpret_cast<const u32x4*>(packed + T::F16_BASE), dout, demb, partial,
+                       flags);
+    if (check_launch(name) != NSVF_OK) return NSVF_ELAUNCH;
+    hipLaunchKernelGGL((mlp_train_backward_f32_kernel<32, 128, 3>), dim3(nb32), dim3(kTrainBlock),
+                       kBackwardLds, st, emb, M, packed, dout, demb, partial, flags, nb);
+    if (check_launch(name) != NSVF_OK) return NSVF_ELAUNCH;
+  }
+  hipLaunchKernelGGL(sum_partials_kernel, dim3(unsigned(ceil_div(T::PARAMS, kSumCols))), dim3(256),
+                     0, st, partial, nb, nb32, T::PARAMS, flags, dparams);
   return check_launch("mlp_train_sum_partials");
 }
 

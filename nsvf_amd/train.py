@@ -15,8 +15,8 @@ through three parts:
 Here the geometry stages are the fused renderer's kernels (one coarse sample
 stream per batch of rays), and the gather, the MLP and the compositing are
 autograd Functions over hand-written HIP forward and backward kernels, all
-deterministic and atomic-free (the MLP on FP32 MFMA; torch.nn.Linear with
-torch autograd, as in the reference, on request).
+deterministic (the MLP at FP32 accuracy; torch.nn.Linear with torch autograd,
+as in the reference, on request).
 """
 from __future__ import annotations
 
@@ -211,7 +211,8 @@ def pack_mlp_train(weights, biases):
 class FieldMLP(torch.autograd.Function):
     """The field MLP (field.py:217-279): L Linear + ReLU layers, then a
     4-wide head, output (sigma, sigmoid(r, g, b)).  Forward and backward are
-    the hand-written FP32-MFMA kernels: the backward recomputes the
+    hand-written kernels at FP32 accuracy (on FP16 hi / lo parts; on the FP32
+    MFMAs where a value is not finite): the backward recomputes the
     activations from the input rather than storing them, and sums the
     weight gradients over samples in a fixed order (deterministic).
     Arguments: emb [M,D], then W_0, b_0, ..., W_L, b_L in torch layout."""
@@ -352,8 +353,8 @@ class FieldMLPx3(FieldMLP):
     features written as its operand tiles, the weights packed on the device
     each call -- and the backward kernel with the activations'
     recomputation, the input gradients and the parameter gradients in split
-    BF16 too (its head's recomputed logits and input gradient in FP32),
-    deterministic like FieldMLP's."""
+    BF16 too (the head's input gradient in FP32), deterministic like
+    FieldMLP's."""
 
     @staticmethod
     def forward(ctx, emb, *params):
@@ -411,12 +412,10 @@ class TrainableField(nn.Module):
     """The trainable state of a voxel scene: corner embeddings [K,D] and the
     field MLP (L hidden ReLU layers, a 4-wide head: sigma, sigmoid RGB).
 
-    mlp="hip": the MLP runs forward and backward on the hand-written
-    FP32-MFMA kernels (FieldMLP; built for D=32, H=128, L=3 -- other shapes
-    raise); mlp="hip_x3": forward and backward in split BF16 (FieldMLPx3:
-    outputs within about 1e-5 of FP32, gradients about as close; the
-    backward's head -- recomputed logits and their input gradient -- stays
-    FP32);
+    mlp="hip": the MLP runs forward and backward on the hand-written FP32
+    kernels (FieldMLP; built for D=32, H=128, L=3 -- other shapes raise);
+    mlp="hip_x3": forward and backward in split BF16 (FieldMLPx3: outputs
+    within about 1e-5 of FP32, gradients about as close);
     mlp="torch": torch.nn.functional.linear with torch autograd, as in the
     reference."""
 

@@ -114,3 +114,102 @@ def test_weights_not_finite(device):
     bs[2] = bs[2].copy()
     bs[2][7] = 0
     _check(out, emb, ws, bs)
+
+
+def _backward(emb, ws, bs, dout, device):
+    leaves = [torch.from_numpy(a).to(device).requires_grad_()
+              for a in [emb] + [x for wb in zip(ws, bs) for x in wb]]
+    out = FieldMLP.apply(*leaves)
+    return [g.cpu().double() for g in
+            torch.autograd.grad(out, leaves, torch.from_numpy(dout).to(device))]
+
+
+def _backward64(emb, ws, bs, dout, dead=()):
+    """float64 autograd, and dout with the samples near a ReLU kink zeroed;
+    dead: samples whose first layer's outputs are taken as 0."""
+    e = torch.from_numpy(emb).double().requires_grad_()
+    ps = [torch.from_numpy(x).double().requires_grad_() for wb in zip(ws, bs) for x in wb]
+    h, near = e, torch.zeros(len(emb), dtype=torch.bool)
+    for i in range(len(ws)):
+        z = h @ ps[2 * i].T + ps[2 * i + 1]
+        if i + 1 < len(ws):
+            scale = (h.detach().abs() @ ps[2 * i].detach().abs().T + ps[2 * i + 1].detach().abs())
+            near |= (z.detach().abs() < 1e-5 * scale).any(1)
+            h = torch.relu(z)
+            if i == 0 and len(dead):
+                keep = torch.ones(len(emb), 1, dtype=torch.float64)
+                keep[list(dead)] = 0
+                h = h * keep
+    near[list(dead)] = False
+    out = torch.cat([z[:, :1], torch.sigmoid(z[:, 1:])], 1)
+    dout = dout.copy()
+    dout[near.numpy()] = 0
+    return torch.autograd.grad(out, [e, *ps], torch.from_numpy(dout).double()), dout
+
+
+def _close(got, want, what):
+    # FP32's bar of the training tests: 2e-5 of a tensor's largest entry
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a - b).abs().max() <= 2e-5 * max(float(b.abs().max()), 1e-37), (what, i)
+
+
+@pytest.mark.parametrize("M", [1, 63, 64, 65, 130, 64 * 256 + 3])
+def test_backward_sample_counts(device, M):
+    ws, bs = _mlp(7)
+    rng = np.random.default_rng(M)
+    emb = (rng.standard_normal((M, 32)) * 0.1).astype(np.float32)
+    dout = rng.standard_normal((M, 4)).astype(np.float32)
+    want, dout = _backward64(emb, ws, bs, dout)
+    _close(_backward(emb, ws, bs, dout, device), want, M)
+
+
+@pytest.mark.parametrize("emb_scale,dout_scale,scales", [
+    (1.0, 1e-25, (1, 1, 1, 1)), (1.0, 1e15, (1, 1, 1, 1)), (1e4, 1.0, (1, 1e-3, 1, 1e-2)),
+    (1e-4, 1.0, (1e3, 1e2, 1e-4, 1)), (1e-30, 1.0, (1, 1, 1, 1)), (1.0, 1.0, (1e25, 1, 1, 1e-25))])
+def test_backward_scales(device, emb_scale, dout_scale, scales):
+    """Gradients over 20 decades in one call, samples without any, operands
+    far from 1 -- the last two beyond the FP16 form's window, so FP32 MFMAs."""
+    ws, bs = _mlp(8, scales)
+    rng = np.random.default_rng(11)
+    emb = (rng.standard_normal((300, 32)) * 0.1 * emb_scale).astype(np.float32)
+    dout = (rng.standard_normal((300, 4)) * dout_scale
+            * 10.0 ** rng.uniform(-12, 0, (300, 1))).astype(np.float32)
+    dout[::7] = 0
+    want, dout = _backward64(emb, ws, bs, dout)
+    got = _backward(emb, ws, bs, dout, device)
+    _close(got, want, (emb_scale, dout_scale))
+    # a sample's own gradient, however small beside the others'
+    size = want[0].abs().amax(1)
+    err = (got[0] - want[0]).abs().amax(1)
+    assert (err <= 1e-4 * size + 1e-37).all()
+
+
+def test_backward_not_finite(device):
+    """A NaN feature: its sample's first layer is all 0 (fmax), so the NaN
+    reaches that feature's column of dW_0 only; the call runs on the FP32
+    MFMAs."""
+    ws, bs = _mlp(9)
+    rng = np.random.default_rng(12)
+    emb = (rng.standard_normal((200, 32)) * 0.1).astype(np.float32)
+    dout = rng.standard_normal((200, 4)).astype(np.float32)
+    want, dout = _backward64(emb, ws, bs, dout, dead=(70,))
+    bad = emb.copy()
+    bad[70, 5] = np.nan
+    got = _backward(bad, ws, bs, dout, device)
+    assert got[1][:, 5].isnan().all()
+    got[1][:, 5] = want[1][:, 5]
+    _close(got, want, "NaN feature")
+
+
+def test_backward_gradient_not_finite(device):
+    """An infinite output gradient stays with its sample's input gradient."""
+    ws, bs = _mlp(10)
+    rng = np.random.default_rng(13)
+    emb = (rng.standard_normal((150, 32)) * 0.1).astype(np.float32)
+    dout = rng.standard_normal((150, 4)).astype(np.float32)
+    want, dout = _backward64(emb, ws, bs, dout)
+    dout[33, 0] = np.inf
+    got = _backward(emb, ws, bs, dout, device)
+    keep = np.arange(150) != 33
+    _close([got[0][keep]], [want[0][keep]], "infinite gradient")
+    assert not got[0][33].isfinite().all() and not got[1].isfinite().all()
