@@ -478,6 +478,20 @@ int nsvf_field_eval(int precision, int D, int H, int L, const float* centers,
                     const float* bias, float* out, void* workspace,
                     int64_t workspace_bytes, void* stream);
 
+/* nsvf_field_eval at precision 1 on the FP32 matrix units for every shape, in
+ * the order of FP32 sums that this library has always had.  Both kernels are
+ * within FP32 rounding of the exact field, but where samples are placed by
+ * probabilities computed from the field (hierarchical views), a last bit can
+ * move a ray's last step across the end of its bins and change the sample
+ * list, so those views keep the one order.                                  */
+int nsvf_field_eval_f32(int D, int H, int L, const float* centers,
+                        const int32_t* feats, const float* values,
+                        float voxel_size, const float* ray_start,
+                        const float* ray_dir, const void* samples,
+                        const int32_t* list, const int32_t* m_dev,
+                        int64_t m_max, const void* wfrag, const float* bias,
+                        float* out, void* stream);
+
 /* nsvf_field_eval without a caller workspace and without allocating: the
  * BF16 (0) and split-BF16 (2) paths stage their operand tiles in a static
  * device array of nsvf_field_static_scratch_bytes() bytes (64 MiB) that

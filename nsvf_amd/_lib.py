@@ -92,6 +92,7 @@ SIGNATURES = {
     "nsvf_field_workspace_bytes": ([_I, _I, _I, _I, _L], _L),
     "nsvf_field_eval": ([_I, _I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _P, _P, _L, _P, _P, _P, _P,
                          _L, _P], _I),
+    "nsvf_field_eval_f32": ([_I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _P, _P, _L, _P, _P, _P, _P], _I),
     "nsvf_field_embed_bf16": ([_I, _I, _I, _P, _P, _P, _F, _P, _P, _P, _P, _P, _L, _P, _L, _P],
                               _I),
     "nsvf_field_mlp_bf16": ([_I, _I, _I, _P, _L, _P, _L, _P, _P, _P, _P, _P], _I),

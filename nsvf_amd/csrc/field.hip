@@ -1536,8 +1536,8 @@ __device__ __forceinline__ void put_f32_tile(Sink& sink, const f32x4 (&out)[kF32
   sink.end_tile(base);
 }
 
-// Shapes whose FP16 weight parts do not fit the LDS: the whole field on the
-// FP32 MFMAs.
+// The whole field on the FP32 MFMAs: shapes whose FP16 weight parts do not fit
+// the LDS, and nsvf_field_eval_f32.
 template <int D, int H, int L, class Src, class Sink>
 __global__ __launch_bounds__(kFieldBlock) void field_f32_kernel(
     Src src, const int32_t* m_dev, int64_t m_max, const float* __restrict__ wfrag,
@@ -1860,10 +1860,20 @@ int launch_bf16(const Src& src, const int32_t* m_dev, int64_t m_max, const void*
 }
 
 template <int D, int H, int L, class Src, class Sink>
+int launch_f32_mfma(const Src& src, const int32_t* m_dev, int64_t m_max, const void* wfrag,
+                    const float* bias, const Sink& sink, hipStream_t stream) {
+  const int64_t blocks = std::min<int64_t>(ceil_div(ceil_div(m_max, 32), 4), 2048);
+  hipLaunchKernelGGL((field_f32_kernel<D, H, L, Src, Sink>), dim3(unsigned(blocks)),
+                     dim3(kFieldBlock), 0, stream, src, m_dev, m_max,
+                     static_cast<const float*>(wfrag), bias, sink);
+  return check_launch("field_f32");
+}
+
+template <int D, int H, int L, class Src, class Sink>
 int launch_f32(const Src& src, const int32_t* m_dev, int64_t m_max, const void* wfrag,
                const float* bias, const Sink& sink, hipStream_t stream) {
-  const int64_t tiles = ceil_div(m_max, 32);
   if constexpr (f16x3_fits<D, H, L>()) {
+    const int64_t tiles = ceil_div(m_max, 32);
     const auto kernel = field_f16x3_kernel<D, H, L, Src, Sink>;
     constexpr size_t lds = F16Mlp<D, H, L>::LDS_BYTES;
     static const int64_t resident = resident_blocks(kernel, 64 * kF16Waves, lds);
@@ -1874,11 +1884,7 @@ int launch_f32(const Src& src, const int32_t* m_dev, int64_t m_max, const void* 
                        m_dev, m_max, static_cast<const float*>(wfrag), bias, sink);
     return check_launch("field_f16x3");
   } else {
-    const int64_t blocks = std::min<int64_t>(ceil_div(tiles, 4), 2048);
-    hipLaunchKernelGGL((field_f32_kernel<D, H, L, Src, Sink>), dim3(unsigned(blocks)),
-                       dim3(kFieldBlock), 0, stream, src, m_dev, m_max,
-                       static_cast<const float*>(wfrag), bias, sink);
-    return check_launch("field_f32");
+    return launch_f32_mfma<D, H, L>(src, m_dev, m_max, wfrag, bias, sink, stream);
   }
 }
 
@@ -2057,6 +2063,30 @@ int nsvf_field_eval(int precision, int D, int H, int L, const float* centers,
   NSVF_FIELD_CASE(32, 256, 4)
 #undef NSVF_FIELD_CASE
   return set_error(NSVF_EINVAL, "field_eval: unsupported shape D=%d H=%d L=%d", D, H, L);
+}
+
+int nsvf_field_eval_f32(int D, int H, int L, const float* centers, const int32_t* feats,
+                        const float* values, float voxel_size, const float* ray_start,
+                        const float* ray_dir, const void* samples, const int32_t* list,
+                        const int32_t* m_dev, int64_t m_max, const void* wfrag,
+                        const float* bias, float* out, void* stream) {
+  clear_error();
+  if (m_max <= 0) return NSVF_OK;
+  if (!centers || !feats || !values || !ray_start || !ray_dir || !samples || !m_dev || !wfrag ||
+      !bias || !out)
+    return set_error(NSVF_EINVAL, "field_eval_f32: null pointer");
+  const FieldScene sc{centers, feats, values, voxel_size, 1.0f / voxel_size, is_pow2(voxel_size)};
+  const StreamSource src{sc, FieldRays{ray_start, ray_dir},
+                         static_cast<const SampleRec*>(samples), list};
+  const StoreSink sink{reinterpret_cast<float4*>(out), list};
+#define NSVF_FIELD_CASE(d, h, l)    \
+  if (D == d && H == h && L == l) \
+    return launch_f32_mfma<d, h, l>(src, m_dev, m_max, wfrag, bias, sink, as_stream(stream));
+  NSVF_FIELD_CASE(32, 128, 3)
+  NSVF_FIELD_CASE(48, 256, 4)
+  NSVF_FIELD_CASE(32, 256, 4)
+#undef NSVF_FIELD_CASE
+  return set_error(NSVF_EINVAL, "field_eval_f32: unsupported shape D=%d H=%d L=%d", D, H, L);
 }
 
 int64_t nsvf_field_static_scratch_bytes(void) { return kStaticScratchBytes; }
