@@ -153,6 +153,19 @@ int nsvf_inverse_cdf_sampling_rows(const int32_t* pts_idx, const float* min_dept
                                    float fixed_step_size, int compat,
                                    int32_t* out_idx, float* out_depth,
                                    float* out_dists, int64_t* flags, void* stream);
+/* The same, raising *max_valid (device i32, cleared by the caller) to the
+ * largest number of samples with a voxel id in one row: the length the
+ * reference's wrapper trims the rows to (fairnr/clib/__init__.py:276-281). */
+int nsvf_inverse_cdf_sampling_rows_max(const int32_t* pts_idx,
+                                       const float* min_depth,
+                                       const float* max_depth,
+                                       const float* noise, const float* probs,
+                                       const float* steps, int N, int P, int S,
+                                       int group, int chunk,
+                                       float fixed_step_size, int compat,
+                                       int32_t* out_idx, float* out_depth,
+                                       float* out_dists, int32_t* max_valid,
+                                       void* stream);
 
 /* ------------------------------------------------------------------------
  * Pruning scores (fairnr/modules/encoder.py:605-654, nsvf.py:143-146): for

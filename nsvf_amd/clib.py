@@ -129,6 +129,14 @@ def inverse_cdf_sampling_rows(pts_idx, min_depth, max_depth, probs, steps, fixed
                               noise=None, max_steps=None, compat=True):
     """One launch over [N,P] rows with the reference's grouping semantics.
     Returns untrimmed [N, max_steps] outputs and max_steps."""
+    return _icdf_rows(pts_idx, min_depth, max_depth, probs, steps, fixed_step_size, noise,
+                      max_steps, compat)[:4]
+
+
+def _icdf_rows(pts_idx, min_depth, max_depth, probs, steps, fixed_step_size, noise, max_steps,
+               compat):
+    """inverse_cdf_sampling_rows, and a device int32 [1]: the largest number of
+    samples with a voxel id in a row."""
     N, P = pts_idx.shape
     dev = pts_idx.device
     if max_steps is None:
@@ -143,12 +151,12 @@ def inverse_cdf_sampling_rows(pts_idx, min_depth, max_depth, probs, steps, fixed
     oi = torch.empty((N, max_steps), dtype=torch.int32, device=dev)
     od = torch.empty((N, max_steps), dtype=torch.float32, device=dev)
     ot = torch.empty((N, max_steps), dtype=torch.float32, device=dev)
-    check(lib().nsvf_inverse_cdf_sampling_rows(_ptr(pi), _ptr(mn), _ptr(mx), _ptr(noise), _ptr(pr),
-                                               _ptr(st), N, P, max_steps, ICDF_GROUPS, ICDF_CHUNK,
-                                               float(_scalar(fixed_step_size)), int(bool(compat)),
-                                               _ptr(oi), _ptr(od), _ptr(ot), None, _stream(dev)),
-          "inverse_cdf_sampling")
-    return oi, od, ot, max_steps
+    most = torch.zeros(1, dtype=torch.int32, device=dev)
+    check(lib().nsvf_inverse_cdf_sampling_rows_max(
+        _ptr(pi), _ptr(mn), _ptr(mx), _ptr(noise), _ptr(pr), _ptr(st), N, P, max_steps,
+        ICDF_GROUPS, ICDF_CHUNK, float(_scalar(fixed_step_size)), int(bool(compat)), _ptr(oi),
+        _ptr(od), _ptr(ot), _ptr(most), _stream(dev)), "inverse_cdf_sampling")
+    return oi, od, ot, max_steps, most
 
 
 class InverseCDFRaySampling(Function):
@@ -163,10 +171,11 @@ class InverseCDFRaySampling(Function):
         if not deterministic:
             noise = min_depth.new_zeros(N, max_steps, dtype=torch.float32).uniform_().clamp(
                 min=0.001, max=0.999)
-        si, sd, sx, _ = inverse_cdf_sampling_rows(pts_idx, min_depth, max_depth, probs, steps,
-                                                  fixed_step_size, noise, max_steps)
+        si, sd, sx, _, most = _icdf_rows(pts_idx, min_depth, max_depth, probs, steps,
+                                         fixed_step_size, noise, max_steps, True)
         sd, sx = sd.type_as(min_depth), sx.type_as(min_depth)
-        si, sd, sx = _trim(si, sd, sx)
+        max_len = int(most.item())
+        si, sd, sx = si[:, :max_len], sd[:, :max_len], sx[:, :max_len]
         ctx.mark_non_differentiable(si)
         ctx.mark_non_differentiable(sd)
         ctx.mark_non_differentiable(sx)
