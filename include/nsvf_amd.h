@@ -321,6 +321,11 @@ int nsvf_render_hits_ordered(const float* ray_start, const float* ray_dir,
                              int T, int depth, int n_max, float step_size,
                              void* hits, int32_t* count, float* tot,
                              int32_t* hit_flag, int32_t* bound, void* stream);
+/* 1 if the traversal walks each ray of a call of R rays on its own (smaller
+ * calls), where an order of the rays gives nothing; 0 if 64 rays share a walk
+ * and coherent neighbours make it shorter.                                  */
+int nsvf_render_hits_alone(int64_t R);
+
 /* Sort keys for such a grouping, one pass over the rays: keys[r] (int64) =
  * direction octant << 42 | origin cell << 30 | Morton code of the direction
  * (10 bits per axis over [-1, 1]), the origin cell on a 16^3 grid over the

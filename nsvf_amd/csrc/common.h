@@ -30,6 +30,15 @@ inline int check_launch(const char* what) {
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// Bitwise or of v over each group of 8 lanes, to all of them (DPP: lane ^ 1,
+// lane ^ 2, then the mirror of the 8).
+__device__ __forceinline__ uint32_t or8(uint32_t v) {
+  v |= uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true));
+  v |= uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true));
+  v |= uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x141, 0xF, 0xF, true));
+  return v;
+}
+
 // Makes this wavefront's earlier LDS writes visible to all its lanes (a
 // barrier for one wave; waves of a block do not wait for each other).
 __device__ __forceinline__ void wave_sync() {

@@ -195,15 +195,6 @@ constexpr int kSvoMaxLevels = 30;
 constexpr int kSvoIdBits = 27;            // node ids; the depth sits above them
 constexpr uint32_t kSvoLeaf = 31;         // depth code of a waiting leaf
 
-// Bitwise or of v over each group of 8 lanes, to all of them (DPP: lane ^ 1,
-// lane ^ 2, then the mirror of the 8).
-__device__ __forceinline__ uint32_t or8(uint32_t v) {
-  v |= uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0xB1, 0xF, 0xF, true));
-  v |= uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x4E, 0xF, 0xF, true));
-  v |= uint32_t(__builtin_amdgcn_mov_dpp(int(v), 0x141, 0xF, 0xF, true));
-  return v;
-}
-
 // Half sizes, over the scale, of the boxes an internal node is tested with:
 // the reference's loose box, twice the node's octant, or the octant with a
 // margin, where svo_check_kernel has found that it holds every leaf below.

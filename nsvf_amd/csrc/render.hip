@@ -31,6 +31,7 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kHitsBlock = 128;
+constexpr int kGroupBlock = 256;
 constexpr int kMaxLevels = 24;
 
 // ---------------------------------------------------------------------------
@@ -206,6 +207,190 @@ __global__ __launch_bounds__(kBlock) void ray_gen_kernel(nsvf_camera cam, float 
   }
 }
 
+// The walk with eight lanes per ray, each ray walking alone.  Lane s of a
+// group tests the child at place s of the child order (slot s ^ dmask); an
+// expansion is one 256-byte record read by the group.  Leaves ahead of the
+// first internal child go out at once, the rest waits in LDS, one word per
+// level and lane: the node and log2 of its scale, or, for a leaf (whose box
+// its parent's record holds), the parent and kHitsLeaf.  The next node is the
+// first that waits at the deepest level, so leaves come out depth first in
+// child order, as above.
+constexpr int kHitsIdBits = 27;
+constexpr uint32_t kHitsLeaf = 31;
+
+struct GroupLane {
+  int s;           // the lane's place in its group of eight
+  int shift;       // the group's first lane in its wave
+  uint32_t* wait;  // this lane's words, 64 apart per level
+  __device__ __forceinline__ uint32_t votes(bool p) const {
+    return uint32_t(__ballot(p) >> shift) & 0xFFu;
+  }
+};
+
+__device__ int walk_group(const GroupLane& ln, const float o[3], const float inv[3], int dmask,
+                          bool act, const float4* __restrict__ recs, int T, int n_max,
+                          HitRec* row) {
+  int cnt = 0, level = 0, psc = 0x7fffffff;
+  int node = act ? T : -1;   // -1: none, the ray is done
+  int order = 0;             // the root's record has it in slot 0
+  uint32_t pend = 0;
+  const uint32_t* group_wait = ln.wait - ln.s;
+  while (__any(node >= 0)) {
+    bool leaf = false, inner = false;
+    int id = -1, sc = 0;
+    float lo = 0.0f, hi = 0.0f;
+    if (node >= 0) {
+      const float4* piece = recs + int64_t(node) * 16 + 2 * (ln.s ^ order);
+      const float4 mn = piece[0], mx = piece[1];
+      id = __float_as_int(mx.w);
+      sc = __float_as_int(mn.w);
+      const bool hit = unsigned(id) < unsigned(T) && sc < psc && ray_box(o, inv, mn, mx, &lo, &hi);
+      leaf = hit && sc == 1;
+      inner = hit && sc > 1 && level + 1 < kMaxLevels;
+    }
+    const uint32_t leaves = ln.votes(leaf), inners = ln.votes(inner);
+    const uint32_t out = leaves & ((inners & (0u - inners)) - 1u);
+    if (out >> ln.s & 1) {
+      const int at = cnt + int(__popc(out & ((1u << ln.s) - 1)));
+      if (at < n_max) row[at] = HitRec{lo, hi, id, 0};
+    }
+    cnt = min(cnt + int(__popc(out)), n_max);
+    if (((leaves | inners) & ~out) >> ln.s & 1) {
+      ln.wait[level * 64] =
+          leaf ? uint32_t(node) | kHitsLeaf << kHitsIdBits
+               : uint32_t(id) | uint32_t(31 - __clz(sc)) << kHitsIdBits;
+      pend |= 1u << level;
+    }
+    uint32_t levels = cnt < n_max ? or8(pend) : 0;
+    order = dmask;
+    node = -1;
+    wave_sync();
+    while (__any(levels != 0 && node < 0)) {
+      const bool look = levels != 0 && node < 0;
+      const int l = look ? 31 - __clz(int(levels)) : 0;
+      const uint32_t waiting = ln.votes(look && (pend >> l & 1));
+      if (look) {
+        const int f = __builtin_ctz(waiting);
+        if (ln.s == f) pend &= ~(1u << l);
+        if ((waiting & (waiting - 1)) == 0) levels &= ~(1u << l);
+        const uint32_t w = group_wait[l * 64 + f];
+        const int k = int(w & ((1u << kHitsIdBits) - 1));
+        if (w >> kHitsIdBits != kHitsLeaf) {
+          node = k;
+          psc = int(1u << (w >> kHitsIdBits));
+          level = l + 1;
+        } else {
+          // its test again: the same operands, the same bits
+          const float4* piece = recs + int64_t(k) * 16 + 2 * (k == T ? f : f ^ dmask);
+          const float4 mn = piece[0], mx = piece[1];
+          float klo = 0.0f, khi = 0.0f;
+          ray_box(o, inv, mn, mx, &klo, &khi);
+          if (ln.s == 0) row[cnt] = HitRec{klo, khi, __float_as_int(mx.w), 0};
+          if (++cnt >= n_max) levels = 0;
+        }
+      }
+    }
+    wave_sync();
+  }
+  return cnt;
+}
+
+// Left-to-right sum of the row's segment lengths, and whether its entry depths
+// strictly increase, by the row's eight lanes: eight segments at a time, lane
+// s's running sum from lane s - 1's (DPP wave_shr:1), each rounded once.
+__device__ __forceinline__ float sum_group(const GroupLane& ln, const HitRec* row, int cnt,
+                                           bool* increasing) {
+  float tot = 0.0f, prev = 0.0f;
+  bool falls = false;
+  const auto left = [](float v) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xf, 0xf, false));
+  };
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  for (int k0 = 0; __any(k0 < cnt); k0 += 8) {
+    const int k = k0 + ln.s;
+    float lo = 0.0f, d = 0.0f;
+    if (k < cnt) {
+      const HitRec h = row[k];
+      lo = h.lo;
+      d = h.hi - h.lo;
+    }
+    const float lower = left(lo);   // by every lane: a branch would hide lane 0
+    const float before = ln.s == 0 ? prev : lower;
+    falls = falls || (k < cnt && k > 0 && !(before < lo));
+    float run = ln.s == 0 ? tot + d : d;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) {
+      const float l = left(run);
+      run = ln.s == 0 ? run : l + d;
+    }
+    tot = k0 < cnt ? __shfl(run, ln.shift + 7, 64) : tot;
+    prev = __shfl(lo, ln.shift + 7, 64);
+  }
+  *increasing = ln.votes(falls) == 0;
+  return tot;
+}
+
+// Stable sort of the row by entry depth: up to 64 hits by their ranks (eight
+// records in each lane, the depths in the group's waiting words), longer rows
+// by insertion on one lane.
+__device__ __forceinline__ void sort_group(const GroupLane& ln, HitRec* row, int cnt) {
+  constexpr int N = 8;
+  float* depths = reinterpret_cast<float*>(ln.wait - ln.s);
+  const auto depth = [depths](int k) -> float& {
+    return depths[(k >> 3) * 64 + (k & 7)];
+  };
+  const bool ranked = cnt <= 8 * N;
+  float4 h[N];
+  int rank[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int k = 8 * i + ln.s;
+    rank[i] = 0;
+    h[i] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+    if (ranked && k < cnt) {
+      h[i] = reinterpret_cast<const float4*>(row)[k];
+      depth(k) = h[i].x;
+    }
+  }
+  wave_sync();
+  if (ranked) {
+    for (int j = 0; j < cnt; ++j) {
+      const float lo = depth(j);
+#pragma unroll
+      for (int i = 0; i < N; ++i) rank[i] += j < 8 * i + ln.s ? lo <= h[i].x : lo < h[i].x;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+      if (8 * i + ln.s < cnt) reinterpret_cast<float4*>(row)[rank[i]] = h[i];
+  } else if (ln.s == 0) {
+    for (int k = 1; k < cnt; ++k) {
+      const HitRec v = row[k];
+      int j = k - 1;
+      while (j >= 0 && row[j].lo > v.lo) {
+        row[j + 1] = row[j];
+        --j;
+      }
+      row[j + 1] = v;
+    }
+  }
+}
+
+// The row of a ray that the front-to-back walk does not settle: walked in the
+// reference's child order, sorted, summed.  Returns the count.
+__device__ __forceinline__ int redo_group(const GroupLane& ln, const float o[3],
+                                          const float inv[3], bool act,
+                                          const float4* __restrict__ recs, int T, int n_max,
+                                          HitRec* row, float* tot) {
+  bool increasing;
+  const int cnt = walk_group(ln, o, inv, 7, act, recs, T, n_max, row);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  sort_group(ln, row, cnt);
+  *tot = sum_group(ln, row, cnt, &increasing);
+  wave_sync();
+  return cnt;
+}
+
 // Per ray: hits sorted by entry depth, count, and the left-to-right sum of
 // the segment lengths.  The front-to-back traversal yields the hits already
 // sorted (leaves are disjoint voxels and a ray crosses octants in increasing
@@ -286,22 +471,36 @@ __global__ __launch_bounds__(kHitsBlock) void hits_kernel(
   int cnt = hr.cnt;
   float tot = hr.tot;
   const bool redo = valid && !(cnt < n_max && hr.increasing);
-  if (__ballot(redo)) {
-    HitRow ref{row, 0, 0.0f, 0.0f, true};
-    traverse_union(o, inv, 7, redo, recs, T, n_max, lrec, ref);
-    if (redo) {
-      cnt = ref.cnt;
-      for (int k = 1; k < cnt; ++k) {  // stable insertion sort by entry depth
-        const HitRec h = row[k];
-        int j = k - 1;
-        while (j >= 0 && row[j].lo > h.lo) {
-          row[j + 1] = row[j];
-          --j;
-        }
-        row[j + 1] = h;
+  uint64_t again = __ballot(redo);
+  if (again) {
+    // eight such rays at a time, one to each group of eight lanes; the walk's
+    // words take the records' place
+    wave_sync();
+    const int lane = threadIdx.x & 63;
+    const GroupLane ln{lane & 7, lane & 56, reinterpret_cast<uint32_t*>(lrec) + lane};
+    static_assert(16 * sizeof(float4) == 64 * sizeof(uint32_t), "a level's record or words");
+    while (again) {
+      uint64_t m = again;
+      for (int i = 0; i < (lane >> 3); ++i) m &= m - 1;
+      const int src = m ? first_lane(m) : 0;
+      float ro[3], rinv[3];
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        ro[a] = __shfl(o[a], src, 64);
+        rinv[a] = __shfl(inv[a], src, 64);
       }
-      tot = 0.0f;
-      for (int k = 0; k < cnt; ++k) tot = tot + (row[k].hi - row[k].lo);
+      HitRec* rrow = hits + __shfl((long long)r, src, 64) * n_max;
+      float rtot;
+      const int rcnt = redo_group(ln, ro, rinv, m != 0, recs, T, n_max, rrow, &rtot);
+      const int place = __popcll(again & ((uint64_t(1) << lane) - 1));
+      const bool mine = (again >> lane & 1) && place < 8;
+      const int c8 = __shfl(rcnt, (place & 7) * 8, 64);
+      const float t8 = __shfl(rtot, (place & 7) * 8, 64);
+      if (mine) {
+        cnt = c8;
+        tot = t8;
+      }
+      again &= ~__ballot(mine);
     }
   }
   if (!valid) return;
@@ -311,6 +510,107 @@ __global__ __launch_bounds__(kHitsBlock) void hits_kernel(
   // at most ceil(steps) + cnt samples carry a voxel id (one per CDF step and
   // one tail per bin; the compat duplicate replaces a step sample)
   bound[r] = cnt > 0 ? int(ceilf(tot / step_size)) + cnt + 2 : 0;
+}
+
+// hits_kernel's outputs, bit for bit, with each ray walking alone.  Bound: the
+// chain of record reads of a ray (some 40 of a microsecond each), with the
+// rows that are walked again; those were sorted by one lane in global memory,
+// which alone took half of either kernel (64 x 64 rays: 86 -> 59 us here, 412
+// -> 310 us there).  Random training rays, 8,192 in shell boxes: 525 -> 63 us.
+template <bool kCamera>
+__global__ __launch_bounds__(kGroupBlock) void hits_group_kernel(
+    const float* __restrict__ ray_start, const float* __restrict__ ray_dir, int64_t R, int width,
+    nsvf_camera cam, float su, float sv, float* __restrict__ gen_start,
+    float* __restrict__ gen_dir, const float4* __restrict__ recs, int T, int n_max,
+    float step_size, HitRec* __restrict__ hits, int32_t* __restrict__ count,
+    float* __restrict__ tot_out, int32_t* __restrict__ hit_flag, int32_t* __restrict__ bound,
+    const int32_t* __restrict__ order) {
+  __shared__ uint32_t waiting_at[kGroupBlock / 64][kMaxLevels * 64];
+  const GroupLane ln{int(threadIdx.x & 7), int(threadIdx.x & 56),
+                     waiting_at[threadIdx.x >> 6] + (threadIdx.x & 63)};
+  // blocks go round the 8 XCDs; each takes one contiguous eighth of the rays
+  const int64_t per_xcd = gridDim.x / 8;
+  const int64_t blk = int64_t(blockIdx.x) < per_xcd * 8
+                          ? (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3)
+                          : int64_t(blockIdx.x);
+  const int64_t t = blk * (kGroupBlock / 8) + (threadIdx.x >> 3);
+  int64_t r = t;
+  bool valid = t < R;
+  if (order) {
+    r = valid ? order[t] : 0;
+    valid = valid && r >= 0 && r < R;
+  }
+  r = valid ? r : 0;
+  float o[3] = {0.0f, 0.0f, 0.0f}, inv[3] = {1.0f, 1.0f, 1.0f};
+  int mask = 0;
+  if (valid) {
+    float dir[3];
+    if constexpr (kCamera) {
+      camera_ray(cam, su, sv, int(r / width), int(r % width), o, dir);
+      if (ln.s == 0) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          gen_start[r * 3 + a] = o[a];
+          gen_dir[r * 3 + a] = dir[a];
+        }
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        o[a] = ray_start[r * 3 + a];
+        dir[a] = ray_dir[r * 3 + a];
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      inv[a] = 1.0f / dir[a];
+      mask |= (dir[a] < 0.0f ? 1 : 0) << a;
+    }
+  }
+  HitRec* row = hits + r * n_max;
+  int cnt = walk_group(ln, o, inv, mask, valid, recs, T, n_max, row);
+  bool increasing;
+  float tot = sum_group(ln, row, cnt, &increasing);
+  const bool redo = valid && !(cnt < n_max && increasing);
+  if (__any(redo)) {
+    wave_sync();
+    float sorted;
+    const int again = redo_group(ln, o, inv, redo, recs, T, n_max, row, &sorted);
+    if (redo) {
+      cnt = again;
+      tot = sorted;
+    }
+  }
+  if (!valid || ln.s != 0) return;
+  count[r] = cnt;
+  tot_out[r] = tot;
+  hit_flag[r] = cnt > 0 ? 1 : 0;
+  bound[r] = cnt > 0 ? int(ceilf(tot / step_size)) + cnt + 2 : 0;
+}
+
+// Rays up to which each walks alone.  The shared walk's wave takes the union
+// of 64 rays' nodes one by one, so a call has a floor (shell, image tiles:
+// 310 us for 64 x 64 rays, 235 for 200 x 200); eight lanes per ray pay for
+// every ray's own nodes (59 and 69 us) and pass it where the chip is full:
+// 149 against 159 us at 400 x 400, 247 against 233 at 566 x 566, 427 against
+// 183 at 800 x 800.
+constexpr int64_t kGroupRays = 3 << 16;
+
+template <bool kCamera>
+void launch_hits(const float* ray_start, const float* ray_dir, int64_t R, int width,
+                 const nsvf_camera& cam, float su, float sv, float* gen_start, float* gen_dir,
+                 const void* records, int T, int n_max, float step_size, void* hits,
+                 int32_t* count, float* tot, int32_t* hit_flag, int32_t* bound,
+                 const int32_t* order, void* stream) {
+  const bool group = R <= kGroupRays;
+  const int64_t threads =
+      group ? R * 8 : width > 0 ? ceil_div(R / width, 8) * ceil_div(width, 8) * 64 : R;
+  const int block = group ? kGroupBlock : kHitsBlock;
+  hipLaunchKernelGGL(group ? hits_group_kernel<kCamera> : hits_kernel<kCamera>,
+                     dim3(unsigned(ceil_div(threads, block))), dim3(block), 0, as_stream(stream),
+                     ray_start, ray_dir, R, width, cam, su, sv, gen_start, gen_dir,
+                     static_cast<const float4*>(records), T, n_max, step_size,
+                     static_cast<HitRec*>(hits), count, tot, hit_flag, bound, order);
 }
 
 // Sort key of a ray for the traversal's grouping (nsvf_ray_order_keys):
@@ -1114,15 +1414,13 @@ int nsvf_render_hits(const float* ray_start, const float* ray_dir, int64_t R, in
   if (!ray_start || !ray_dir || !records || !hits || !count || !tot || !hit_flag || !bound)
     return set_error(NSVF_EINVAL, "render_hits: null pointer");
   if (T >= (1 << 27)) return set_error(NSVF_EINVAL, "render_hits: more than 2^27 nodes");
-  const int64_t threads =
-      width > 0 ? ceil_div(R / width, 8) * ceil_div(width, 8) * 64 : R;
-  hipLaunchKernelGGL(hits_kernel<false>, dim3(unsigned(ceil_div(threads, kHitsBlock))),
-                     dim3(kHitsBlock), 0, as_stream(stream), ray_start, ray_dir, R, width,
-                     nsvf_camera{}, 0.0f, 0.0f, nullptr, nullptr,
-                     static_cast<const float4*>(records), T, n_max, step_size,
-                     static_cast<HitRec*>(hits), count, tot, hit_flag, bound, nullptr);
+  launch_hits<false>(ray_start, ray_dir, R, width, nsvf_camera{}, 0.0f, 0.0f, nullptr, nullptr,
+                     records, T, n_max, step_size, hits, count, tot, hit_flag, bound, nullptr,
+                     stream);
   return check_launch("render_hits");
 }
+
+int nsvf_render_hits_alone(int64_t R) { return R <= kGroupRays ? 1 : 0; }
 
 int nsvf_ray_order_keys(const float* ray_start, const float* ray_dir, int64_t R,
                         const float* bounds, int64_t* keys, void* stream) {
@@ -1150,11 +1448,9 @@ int nsvf_render_hits_ordered(const float* ray_start, const float* ray_dir, int64
     return set_error(NSVF_EINVAL, "render_hits_ordered: null pointer");
   if (T >= (1 << 27))
     return set_error(NSVF_EINVAL, "render_hits_ordered: more than 2^27 nodes");
-  hipLaunchKernelGGL(hits_kernel<false>, dim3(unsigned(ceil_div(R, kHitsBlock))),
-                     dim3(kHitsBlock), 0, as_stream(stream), ray_start, ray_dir, R, 0,
-                     nsvf_camera{}, 0.0f, 0.0f, nullptr, nullptr,
-                     static_cast<const float4*>(records), T, n_max, step_size,
-                     static_cast<HitRec*>(hits), count, tot, hit_flag, bound, order);
+  launch_hits<false>(ray_start, ray_dir, R, 0, nsvf_camera{}, 0.0f, 0.0f, nullptr, nullptr,
+                     records, T, n_max, step_size, hits, count, tot, hit_flag, bound, order,
+                     stream);
   return check_launch("render_hits_ordered");
 }
 
@@ -1193,12 +1489,8 @@ int nsvf_render_hits_camera(const nsvf_camera* cam, const void* records, int T, 
   if (T >= (1 << 27)) return set_error(NSVF_EINVAL, "render_hits_camera: more than 2^27 nodes");
   const float su = float(double(cam->W) / cam->w), sv = float(double(cam->H) / cam->h);
   const int64_t R = int64_t(cam->h) * cam->w;
-  const int64_t threads = ceil_div(cam->h, 8) * ceil_div(cam->w, 8) * 64;
-  hipLaunchKernelGGL(hits_kernel<true>, dim3(unsigned(ceil_div(threads, kHitsBlock))),
-                     dim3(kHitsBlock), 0, as_stream(stream), nullptr, nullptr, R, cam->w, *cam,
-                     su, sv, ray_start, ray_dir, static_cast<const float4*>(records), T, n_max,
-                     step_size, static_cast<HitRec*>(hits), count, tot, hit_flag, bound,
-                     nullptr);
+  launch_hits<true>(nullptr, nullptr, R, cam->w, *cam, su, sv, ray_start, ray_dir, records, T,
+                    n_max, step_size, hits, count, tot, hit_flag, bound, nullptr, stream);
   return check_launch("render_hits_camera");
 }
 

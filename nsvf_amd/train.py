@@ -459,10 +459,10 @@ class TrainRenderer:
     octree, shifted centres and corner ids) with a TrainableField's
     parameters: intersect + coarse samples (non-differentiable kernels), then
     gather, MLP and compositing with autograd, then the background fill
-    (nsvf.py:94-101).  coherent: the traversal takes the batch's rays
-    grouped by direction and origin (coherent_order; a batch of random
-    pixels from several views has no image rows to tile), which changes no
-    result."""
+    (nsvf.py:94-101).  coherent: where the traversal's waves share a walk
+    (large batches), it takes the batch's rays grouped by direction and
+    origin (coherent_order; a batch of random pixels from several views has
+    no image rows to tile), which changes no result."""
 
     def __init__(self, device, compat=True, deterministic_step=False, seed=0, coherent=True):
         self.device = torch.device(device)
@@ -492,7 +492,8 @@ class TrainRenderer:
         self.steps += 1
         self.last_seed = seed
         self.geometry.noise_seed = seed
-        order = coherent_order(rs, rd) if self.coherent and rs.shape[0] > 0 else None
+        shared = not lib().nsvf_render_hits_alone(rs.shape[0])
+        order = coherent_order(rs, rd) if self.coherent and shared else None
         g = self.geometry.coarse_stream(sc, rs, rd, order=order).owned()
         self.last = g
         rec = g.samples
