@@ -618,6 +618,23 @@ int nsvf_render_composite_backward(const int32_t* hit_list,
                                    const float* grad_rgb, const float* grad_depth,
                                    const float* grad_missed, float* grad_field,
                                    void* stream);
+/* The same through the background fill (nsvf_render_finish: rgb + missed bg,
+ * depth + missed bg_depth; nsvf.py:94-101): grad_rgb, grad_depth, grad_missed
+ * are those of the filled outputs, any of them NULL where there is none.    */
+int nsvf_render_over_backward(const int32_t* hit_list,
+                              const int32_t* n_hit_dev, int64_t n_hit_max,
+                              const int32_t* off, const int32_t* cnt,
+                              const void* samples, const float* field,
+                              const float* grad_rgb, const float* grad_depth,
+                              const float* grad_missed, float bg_r, float bg_g,
+                              float bg_b, float bg_depth, float* grad_field,
+                              void* stream);
+
+/* Voxel s_idx [M] and position xyz [M,3] = ray_start + ray_dir * depth of each
+ * of M sample records of R rays.                                            */
+int nsvf_stream_points(const void* samples, int64_t M, const float* ray_start,
+                       const float* ray_dir, int64_t R, int32_t* s_idx,
+                       float* xyz, void* stream);
 
 /* Early ray termination as the reference's chunked ray marching
  * (fairnr/modules/renderer.py:136-174 with --raymarching-tolerance > 0;
@@ -684,6 +701,16 @@ int64_t nsvf_mlp_train_param_floats(int D, int H, int L);
 int64_t nsvf_mlp_train_partial_floats(int D, int H, int L, int64_t M);
 int nsvf_mlp_train_pack(int D, int H, int L, const float* const* weights,
                         const float* const* biases, float* packed, void* stream);
+/* Split-BF16 operand fragments of an MLP in one launch.  index (device,
+ * n_forward then n_backward positions in [0, W_0 flat, ..., W_L flat], 0 for
+ * padding; both multiples of 512): each 512 become 1,024 bf16, the parts
+ * bf16(w), then bf16(w - hi).  bias [L H + 16]: b_0 .. b_{L-1}, then the
+ * head's 4 padded to 16.  *count_dev = count (an MLP call's sample count).  */
+int nsvf_mlp_split_pack(int D, int H, int L, const float* const* weights,
+                        const float* const* biases, const int64_t* index,
+                        int64_t n_forward, int64_t n_backward, void* forward,
+                        void* backward, float* bias, int count,
+                        int32_t* count_dev, void* stream);
 int nsvf_mlp_train_forward(int D, int H, int L, const float* packed,
                            const float* emb, int64_t M, float* out, void* stream);
 int nsvf_mlp_train_backward(int D, int H, int L, const float* packed,

@@ -79,6 +79,7 @@ SIGNATURES = {
     "nsvf_mlp_train_packed_floats": ([_I, _I, _I], _L),
     "nsvf_mlp_train_param_floats": ([_I, _I, _I], _L),
     "nsvf_mlp_train_partial_floats": ([_I, _I, _I, _L], _L),
+    "nsvf_mlp_split_pack": ([_I, _I, _I, _P, _P, _P, _L, _L, _P, _P, _P, _I, _P, _P], _I),
     "nsvf_mlp_train_pack": ([_I, _I, _I, _P, _P, _P, _P], _I),
     "nsvf_mlp_train_forward": ([_I, _I, _I, _P, _P, _L, _P, _P], _I),
     "nsvf_mlp_train_backward": ([_I, _I, _I, _P, _P, _L, _P, _P, _P, _L, _P, _P], _I),
@@ -109,6 +110,8 @@ SIGNATURES = {
     "nsvf_render_composite": ([_P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P], _I),
     "nsvf_render_composite_backward": ([_P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P], _I),
     "nsvf_track_voxel_probs": ([_P, _P, _L, _P, _P, _P, _P, _P, _L, _P], _I),
+    "nsvf_render_over_backward": ([_P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _F, _F, _F, _F, _P, _P], _I),
+    "nsvf_stream_points": ([_P, _L, _P, _P, _L, _P, _P, _P], _I),
     "nsvf_render_finish": ([_L, _P, _P, _P, _P, _F, _F, _F, _F, _P, _P, _P, _P], _I),
     "nsvf_plain_aabb_intersect": ([_P, _P, _P, _I, _I, _I, _F, _I, _P, _P, _P, _P], _I),
     "nsvf_plain_svo_intersect": ([_P, _P, _P, _P, _I, _I, _I, _F, _I, _P, _P, _P, _P], _I),

@@ -1225,6 +1225,48 @@ struct TrainLayers {
   const float* b[8];
 };
 
+// Layer l's weights are positions start[l] .. start[l + 1] - 1 of [0, W_0
+// flat, W_1 flat, ...].
+struct SplitLayers {
+  TrainLayers net;
+  int64_t start[9];
+  int H, L;
+};
+
+// Elements of the split-BF16 fragments, at the positions index[] gives (the
+// forward kernel's, then the backward's): per 512 their hi parts bf16(w), then
+// their lo parts bf16(w - hi); the biases in one row, the head's 4 padded to
+// 16; and count.  One launch: the copies, conversions and differences were 16
+// torch launches in every training step.
+__global__ __launch_bounds__(256) void split_pack_kernel(SplitLayers s,
+                                                         const int64_t* __restrict__ index,
+                                                         int64_t n_forward, int64_t n_backward,
+                                                         __bf16* __restrict__ forward,
+                                                         __bf16* __restrict__ backward,
+                                                         float* __restrict__ bias, int count,
+                                                         int32_t* __restrict__ count_dev) {
+  int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i == 0) *count_dev = count;
+  if (i < n_forward + n_backward) {
+    const int64_t p = index[i];
+    float w = 0.0f;
+    for (int l = 0; l <= s.L; ++l)
+      if (p >= s.start[l] && p < s.start[l + 1]) w = s.net.w[l][p - s.start[l]];
+    __bf16* out = i < n_forward ? forward : backward;
+    if (i >= n_forward) i -= n_forward;
+    const __bf16 hi = __bf16(w);
+    out[(i >> 9) * 1024 + (i & 511)] = hi;
+    out[(i >> 9) * 1024 + 512 + (i & 511)] = __bf16(w - float(hi));
+    return;
+  }
+  i -= n_forward + n_backward;
+  const int64_t hidden = int64_t(s.L) * s.H;
+  if (i < hidden)
+    bias[i] = s.net.b[i / s.H][i % s.H];
+  else if (i < hidden + 16)
+    bias[i] = i < hidden + 4 ? s.net.b[s.L][i - hidden] : 0.0f;
+}
+
 // Block l: layer l's largest |w|, row sum |w|, column sum |w| and |b| (not
 // finite where a value is not).
 template <int D, int H, int L>
@@ -1431,6 +1473,38 @@ int64_t nsvf_mlp_train_partial_floats(int D, int H, int L, int64_t M) {
   // the blocks' partial sums, then their flags
   const int64_t nb = backward_blocks(M, kBwdChunk);
   return nb * TrainDims<32, 128, 3>::PARAMS + (M > 0 ? nb : 0);
+}
+
+int nsvf_mlp_split_pack(int D, int H, int L, const float* const* weights,
+                        const float* const* biases, const int64_t* index, int64_t n_forward,
+                        int64_t n_backward, void* forward, void* backward, float* bias, int count,
+                        int32_t* count_dev, void* stream) {
+  clear_error();
+  if (D <= 0 || H <= 0 || L <= 0 || L > 7 || n_forward < 0 || n_backward < 0 ||
+      n_forward % 512 != 0 || n_backward % 512 != 0)
+    return set_error(NSVF_EINVAL, "mlp_split_pack: bad size");
+  if (!weights || !biases || !index || !bias || !count_dev || (n_forward > 0 && !forward) ||
+      (n_backward > 0 && !backward))
+    return set_error(NSVF_EINVAL, "mlp_split_pack: null pointer");
+  for (int l = 0; l <= L; ++l)
+    if (!weights[l] || !biases[l]) return set_error(NSVF_EINVAL, "mlp_split_pack: layer %d null", l);
+  SplitLayers net;
+  int64_t at = 1;
+  for (int l = 0; l <= L; ++l) {
+    net.net.w[l] = weights[l];
+    net.net.b[l] = biases[l];
+    net.start[l] = at;
+    at += int64_t(l < L ? H : 4) * (l == 0 ? D : H);
+  }
+  net.start[L + 1] = at;
+  net.H = H;
+  net.L = L;
+  const int64_t n = n_forward + n_backward + L * H + 16;
+  hipLaunchKernelGGL(split_pack_kernel, dim3(unsigned(ceil_div(n, 256))), dim3(256), 0,
+                     as_stream(stream), net, index, n_forward, n_backward,
+                     static_cast<__bf16*>(forward), static_cast<__bf16*>(backward), bias, count,
+                     count_dev);
+  return check_launch("mlp_split_pack");
 }
 
 int nsvf_mlp_train_pack(int D, int H, int L, const float* const* weights,

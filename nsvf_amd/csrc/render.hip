@@ -1289,12 +1289,13 @@ __global__ __launch_bounds__(kBlock) void composite_kernel(
 // ray back to front, so the suffix sums of u are accumulated directly (no
 // difference of two large prefix sums), and overwrites each record with its
 // gradient.  T_k and p_k are recomputed with the forward's exact operations.
+template <bool kOver>
 __global__ __launch_bounds__(kBlock) void composite_backward_kernel(
     const int32_t* __restrict__ hit_list, const int32_t* __restrict__ n_hit_dev,
     const int32_t* __restrict__ off_arr, const int32_t* __restrict__ cnt_arr,
     const SampleRec* __restrict__ samples, const float4* __restrict__ field,
     const float* __restrict__ g_rgb, const float* __restrict__ g_depth,
-    const float* __restrict__ g_missed, float4* __restrict__ grad_field) {
+    const float* __restrict__ g_missed, float4 bg, float4* __restrict__ grad_field) {
   const int64_t n = int64_t(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (n >= *n_hit_dev) return;
@@ -1318,9 +1319,18 @@ __global__ __launch_bounds__(kBlock) void composite_backward_kernel(
     if (k < cnt) grad_field[off + k].x = carry + (incl - fe);
     carry += __shfl(incl, 63, 64);
   }
-  const float gr = g_rgb[int64_t(r) * 3 + 0], gg = g_rgb[int64_t(r) * 3 + 1],
-              gb = g_rgb[int64_t(r) * 3 + 2];
-  const float gd = g_depth[r], gm = g_missed[r];
+  float gr = 0.0f, gg = 0.0f, gb = 0.0f;
+  if (!kOver || g_rgb) {
+    gr = g_rgb[int64_t(r) * 3 + 0];
+    gg = g_rgb[int64_t(r) * 3 + 1];
+    gb = g_rgb[int64_t(r) * 3 + 2];
+  }
+  const float gd = !kOver || g_depth ? g_depth[r] : 0.0f;
+  float gm = !kOver || g_missed ? g_missed[r] : 0.0f;
+  if constexpr (kOver) {  // through the background: rgb + missed bg, depth + missed bg.w
+    if (g_rgb) gm = gm + ((gr * bg.x + gg * bg.y) + gb * bg.z);
+    if (g_depth) gm = gm + gd * bg.w;
+  }
   float suffix = 0.0f;  // sum of u over the samples after the current chunk
   for (int base = (cnt - 1) & ~63; base >= 0; base -= 64) {
     const int k = base + lane;
@@ -1359,6 +1369,23 @@ __global__ __launch_bounds__(kBlock) void composite_backward_kernel(
 
 // Frame outputs for every ray: the hit rays' composite plus the background
 // weighted by `missed`; rays that hit nothing are pure background.
+// Voxel and position o + d z of every slot (geometry.py:160-161, each product
+// and sum rounded); a record with no ray of the batch is unused.
+__global__ __launch_bounds__(kBlock) void stream_points_kernel(
+    const SampleRec* __restrict__ samples, int64_t M, const float* __restrict__ ray_start,
+    const float* __restrict__ ray_dir, int64_t R, int32_t* __restrict__ s_idx,
+    float* __restrict__ xyz) {
+  const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+  if (i >= M) return;
+  const SampleRec s = samples[i];
+  const bool ok = s.ray >= 0 && s.ray < R;
+  s_idx[i] = ok ? s.idx : -1;
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+    xyz[i * 3 + a] =
+        ok ? ray_start[int64_t(s.ray) * 3 + a] + ray_dir[int64_t(s.ray) * 3 + a] * s.depth : 0.0f;
+}
+
 __global__ __launch_bounds__(kBlock) void finish_kernel(
     int64_t R, const int32_t* __restrict__ hit_flag, const float* __restrict__ ray_rgb,
     const float* __restrict__ ray_depth, const float* __restrict__ ray_missed, float bg_r,
@@ -1657,11 +1684,45 @@ int nsvf_render_composite_backward(const int32_t* hit_list, const int32_t* n_hit
       !grad_depth || !grad_missed || !grad_field)
     return set_error(NSVF_EINVAL, "render_composite_backward: null pointer");
   const int per_block = kBlock / 64;
-  hipLaunchKernelGGL(composite_backward_kernel, dim3(unsigned(ceil_div(n_hit_max, per_block))),
-                     dim3(kBlock), 0, as_stream(stream), hit_list, n_hit_dev, off, cnt,
+  hipLaunchKernelGGL(composite_backward_kernel<false>,
+                     dim3(unsigned(ceil_div(n_hit_max, per_block))), dim3(kBlock), 0,
+                     as_stream(stream), hit_list, n_hit_dev, off, cnt,
                      static_cast<const SampleRec*>(samples), reinterpret_cast<const float4*>(field),
-                     grad_rgb, grad_depth, grad_missed, reinterpret_cast<float4*>(grad_field));
+                     grad_rgb, grad_depth, grad_missed, float4{0.0f, 0.0f, 0.0f, 0.0f},
+                     reinterpret_cast<float4*>(grad_field));
   return check_launch("render_composite_backward");
+}
+
+int nsvf_render_over_backward(const int32_t* hit_list, const int32_t* n_hit_dev,
+                              int64_t n_hit_max, const int32_t* off, const int32_t* cnt,
+                              const void* samples, const float* field, const float* grad_rgb,
+                              const float* grad_depth, const float* grad_missed, float bg_r,
+                              float bg_g, float bg_b, float bg_depth, float* grad_field,
+                              void* stream) {
+  clear_error();
+  if (n_hit_max <= 0) return NSVF_OK;
+  if (!hit_list || !n_hit_dev || !off || !cnt || !samples || !field || !grad_field)
+    return set_error(NSVF_EINVAL, "render_over_backward: null pointer");
+  hipLaunchKernelGGL(composite_backward_kernel<true>,
+                     dim3(unsigned(ceil_div(n_hit_max, kBlock / 64))), dim3(kBlock), 0,
+                     as_stream(stream), hit_list, n_hit_dev, off, cnt,
+                     static_cast<const SampleRec*>(samples), reinterpret_cast<const float4*>(field),
+                     grad_rgb, grad_depth, grad_missed, float4{bg_r, bg_g, bg_b, bg_depth},
+                     reinterpret_cast<float4*>(grad_field));
+  return check_launch("render_over_backward");
+}
+
+int nsvf_stream_points(const void* samples, int64_t M, const float* ray_start,
+                       const float* ray_dir, int64_t R, int32_t* s_idx, float* xyz, void* stream) {
+  clear_error();
+  if (M < 0 || R < 0) return set_error(NSVF_EINVAL, "stream_points: bad size");
+  if (M == 0) return NSVF_OK;
+  if (!samples || !ray_start || !ray_dir || !s_idx || !xyz)
+    return set_error(NSVF_EINVAL, "stream_points: null pointer");
+  hipLaunchKernelGGL(stream_points_kernel, dim3(unsigned(ceil_div(M, kBlock))), dim3(kBlock), 0,
+                     as_stream(stream), static_cast<const SampleRec*>(samples), M, ray_start,
+                     ray_dir, R, s_idx, xyz);
+  return check_launch("stream_points");
 }
 
 int nsvf_render_finish(int64_t R, const int32_t* hit_flag, const float* ray_rgb,

@@ -237,10 +237,10 @@ class CoarseStream:
     def owned(self):
         """A copy whose tensors no later coarse_stream call overwrites (what
         an autograd graph keeps until its backward)."""
-        c = lambda t: t.clone()
-        return CoarseStream(self.rays, self.n_hit, self.slots, None, None, None, c(self.flag), None,
-                            c(self.hit_list), c(self.off), c(self.cnt), c(self.samples), None,
-                            c(self.scal))
+        rows = [self.flag, self.hit_list, self.off, self.cnt, self.scal]
+        flag, hit_list, off, cnt, scal = torch.cat(rows).split([t.numel() for t in rows])
+        return CoarseStream(self.rays, self.n_hit, self.slots, None, None, None, flag, None,
+                            hit_list, off, cnt, self.samples.clone(), None, scal)
 
     @property
     def c_off(self):

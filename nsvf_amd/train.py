@@ -177,6 +177,48 @@ class StreamComposite(torch.autograd.Function):
         return grad_field, None
 
 
+class _CompositeOver(torch.autograd.Function):
+    """StreamComposite over the background (nsvf.py:94-101): (rgb + missed *
+    BG_COLOR, depth + missed * BG_DEPTH, missed), the fill and its gradient
+    inside the kernels."""
+
+    @staticmethod
+    def forward(ctx, field, g: CoarseStream):
+        field = field.contiguous()
+        if field.dtype != torch.float32 or field.shape != (g.slots, 4):
+            raise RuntimeError(f"field must be float32 [{g.slots}, 4]")
+        dev, R, L = field.device, g.rays, lib()
+        hit = torch.empty((5, R), dtype=torch.float32, device=dev)   # the hit rays' rgb, depth, missed
+        rgb = torch.empty((R, 3), dtype=torch.float32, device=dev)
+        depth = torch.empty(R, dtype=torch.float32, device=dev)
+        missed = torch.empty(R, dtype=torch.float32, device=dev)
+        st = _stream(dev)
+        if g.n_hit > 0:
+            check(L.nsvf_render_composite(_p(g.hit_list), _p(g.scal[0:1]), g.n_hit, _p(g.off),
+                                          _p(g.cnt), _p(g.samples), _p(field), None, _p(hit),
+                                          _p(hit[3]), _p(hit[4]), st), "composite")
+        check(L.nsvf_render_finish(R, _p(g.flag), _p(hit), _p(hit[3]), _p(hit[4]), *BG_COLOR,
+                                   BG_DEPTH, _p(rgb), _p(depth), _p(missed), st), "finish")
+        ctx.save_for_backward(field)
+        ctx.stream = g
+        ctx.set_materialize_grads(False)
+        return rgb, depth, missed
+
+    @staticmethod
+    def backward(ctx, g_rgb, g_depth, g_missed):
+        (field,) = ctx.saved_tensors
+        g = ctx.stream
+        g_rgb, g_depth, g_missed = (None if t is None else t.contiguous().float()
+                                    for t in (g_rgb, g_depth, g_missed))
+        grad_field = torch.zeros_like(field)
+        if g.n_hit > 0:
+            check(lib().nsvf_render_over_backward(
+                _p(g.hit_list), _p(g.scal[0:1]), g.n_hit, _p(g.off), _p(g.cnt), _p(g.samples),
+                _p(field), _p(g_rgb), _p(g_depth), _p(g_missed), *BG_COLOR, BG_DEPTH,
+                _p(grad_field), _stream(field.device)), "over_backward")
+        return grad_field, None
+
+
 def _mlp_shape(weights):
     return int(weights[0].shape[1]), int(weights[0].shape[0]), len(weights) - 1
 
@@ -196,16 +238,23 @@ def pack_mlp_train(weights, biases):
     if n < 0:
         raise RuntimeError(f"training MLP: shape D={D} H={H} L={L} is not built")
     dev = weights[0].device
-    ws = [w.detach().contiguous().float() for w in weights]
-    bs = [b.detach().contiguous().float() for b in biases]
-    for w, b in zip(ws, bs):
-        _need_cuda(w, "weight")
-        _need_cuda(b, "bias")
     packed = torch.empty(n, dtype=torch.float32, device=dev)
-    wp = (ctypes.c_void_p * len(ws))(*[w.data_ptr() for w in ws])
-    bp = (ctypes.c_void_p * len(bs))(*[b.data_ptr() for b in bs])
+    wp, bp, keep = _layer_pointers(weights, biases)
     check(L_.nsvf_mlp_train_pack(D, H, L, wp, bp, _p(packed), _stream(dev)), "mlp_train_pack")
     return packed
+
+
+def _layer_pointers(weights, biases):
+    """Host arrays of the layers' device pointers (contiguous FP32), and the
+    tensors that must outlive their use."""
+    def plain(t, name):
+        _need_cuda(t, name)
+        return t if t.dtype == torch.float32 and t.is_contiguous() else t.detach().contiguous().float()
+
+    ws = [plain(w, "weight") for w in weights]
+    bs = [plain(b, "bias") for b in biases]
+    array = ctypes.c_void_p * len(ws)
+    return array(*[w.data_ptr() for w in ws]), array(*[b.data_ptr() for b in bs]), (ws, bs)
 
 
 class FieldMLP(torch.autograd.Function):
@@ -289,6 +338,9 @@ def pack_mlp_x3(weights, biases):
     field.pack_mlp's "bf16x3": per fragment its 512 hi parts bf16(w), then
     its lo parts bf16(w - hi), round to nearest even)."""
     dev = weights[0].device
+    if dev.type == "cuda":
+        frags, _, bias, _ = _pack_split(weights, biases)
+        return frags, bias
     idx = _x3_index([tuple(w.shape) for w in weights], dev)
     flat = torch.cat([torch.zeros(1, dtype=torch.float32, device=dev)]
                      + [w.detach().reshape(-1).float() for w in weights])
@@ -346,6 +398,33 @@ def pack_mlp_train_x3(weights):
     return torch.stack([hi, lo], 1).reshape(-1).view(torch.int16)
 
 
+_SPLIT_INDEX = {}
+
+
+def _pack_split(weights, biases, count=0, backward=False):
+    """pack_mlp_x3's fragments and biases, with backward=True also
+    pack_mlp_train_x3's fragments (else None), and `count` as an int32 [1],
+    in one launch."""
+    dev = weights[0].device
+    shapes = [tuple(w.shape) for w in weights]
+    D, H, L = _mlp_shape(weights)
+    key = (tuple(shapes), str(dev), backward)
+    got = _SPLIT_INDEX.get(key)
+    if got is None:
+        f = _x3_index(shapes, dev)
+        b = _x3_train_index(shapes, dev) if backward else f[:0]
+        got = _SPLIT_INDEX[key] = (torch.cat([f, b]), f.numel(), b.numel())
+    idx, nf, nb = got
+    frags = torch.empty(2 * (nf + nb), dtype=torch.int16, device=dev)
+    bias = torch.empty(L * H + 16, dtype=torch.float32, device=dev)
+    m_dev = torch.empty(1, dtype=torch.int32, device=dev)
+    wp, bp, keep = _layer_pointers(weights, biases)
+    check(lib().nsvf_mlp_split_pack(D, H, L, wp, bp, _p(idx), nf, nb, _p(frags),
+                                    _p(frags[2 * nf:]) if backward else None, _p(bias), count,
+                                    _p(m_dev), _stream(dev)), "mlp_split_pack")
+    return frags[:2 * nf], frags[2 * nf:] if backward else None, bias, m_dev
+
+
 class FieldMLPx3(FieldMLP):
     """FieldMLP with its forward on the renderer's split-BF16 MLP kernel
     (three BF16 MFMAs per product on hi / lo operand parts, FP32
@@ -369,17 +448,16 @@ class FieldMLPx3(FieldMLP):
             raise RuntimeError(f"split-BF16 MLP not built for D={D} H={H} L={L}")
         dev, M = emb.device, emb.shape[0]
         out = torch.empty((M, 4), dtype=torch.float32, device=dev)
+        frags, x3w, bias, m_dev = _pack_split(weights, biases, M, backward=True)
         if M > 0:
-            frags, bias = pack_mlp_x3(weights, biases)
             ws_bytes = int(L_.nsvf_field_workspace_bytes(2, D, H, L, M))
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            m_dev = torch.full((1,), M, dtype=torch.int32, device=dev)
             st = _stream(dev)
             check(L_.nsvf_field_tiles_bf16x3(D, H, L, _p(emb), M, _p(ws), ws_bytes, st),
                   "field_tiles_bf16x3")
             check(L_.nsvf_field_mlp_bf16x3(D, H, L, _p(ws), ws_bytes, _p(m_dev), M, _p(frags),
                                            _p(bias), _p(out), None, st), "field_mlp_bf16x3")
-        ctx.save_for_backward(emb, pack_mlp_train(weights, biases), pack_mlp_train_x3(weights))
+        ctx.save_for_backward(emb, pack_mlp_train(weights, biases), x3w)
         ctx.shape = (D, H, L)
         ctx.param_shapes = [tuple(t.shape) for t in params]
         return out
@@ -496,20 +574,18 @@ class TrainRenderer:
         order = coherent_order(rs, rd) if self.coherent and shared else None
         g = self.geometry.coarse_stream(sc, rs, rd, order=order).owned()
         self.last = g
-        rec = g.samples
-        s_idx = rec[:, 0]
-        depth = rec[:, 1].view(torch.float32)
-        ray = rec[:, 3].long()
         # sample points x = o + d * z, each operation rounded (geometry.py:160-161)
-        xyz = rs.index_select(0, ray) + rd.index_select(0, ray) * depth[:, None]
+        rec = g.samples
+        s_idx = torch.empty(rec.shape[0], dtype=torch.int32, device=rec.device)
+        xyz = torch.empty((rec.shape[0], 3), dtype=torch.float32, device=rec.device)
+        check(lib().nsvf_stream_points(_p(rec), rec.shape[0], _p(rs), _p(rd), rs.shape[0],
+                                       _p(s_idx), _p(xyz), _stream(rec.device)), "stream_points")
         if sc.gather_plan is None:  # the scene's incidence order, once per scene
             sc.gather_plan = gather_backward_plan(sc.feats, field.values.shape[0])
         emb = trilinear_gather(field.values, s_idx, xyz, sc.centers, sc.feats, sc.voxel_size,
                                sc.gather_plan)
         out = field.mlp(emb)
-        rgb, dep, missed = StreamComposite.apply(out, g)
-        bg = torch.tensor(BG_COLOR, dtype=torch.float32, device=rgb.device)
-        return rgb + missed[:, None] * bg, dep + missed * BG_DEPTH, missed
+        return _CompositeOver.apply(out, g)
 
 
 def mse_loss(rgb, target):
