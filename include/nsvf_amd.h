@@ -368,6 +368,17 @@ int nsvf_render_hits_camera(const nsvf_camera* cam, const void* records, int T,
                             int32_t* count, float* tot, int32_t* hit_flag,
                             int32_t* bound, void* stream);
 
+/* What lies between a view's traversal and its coarse samples: rank and off
+ * (exclusive sums of hit_flag (0 or 1) and bound over the R rays), list (the
+ * hit rays), scalars = {hit rays, sum of bound, 0, ...} (nscalars >= 2 of
+ * them), and zero [R] cleared.  workspace: int32[
+ * nsvf_render_offsets_workspace_ints(R)].                                   */
+int64_t nsvf_render_offsets_workspace_ints(int64_t R);
+int nsvf_render_offsets(const int32_t* hit_flag, const int32_t* bound,
+                        int64_t R, int32_t* rank, int32_t* list, int32_t* off,
+                        int32_t* zero, int32_t* scalars, int nscalars,
+                        int32_t* workspace, void* stream);
+
 /* list[rank[r]] = r for every ray with hit_flag[r] != 0.                  */
 int nsvf_render_compact(const int32_t* hit_flag, const int32_t* rank,
                         int64_t R, int32_t* list, void* stream);

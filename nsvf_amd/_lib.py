@@ -65,6 +65,8 @@ SIGNATURES = {
     "nsvf_ray_order_keys": ([_P, _P, _L, _P, _P, _P], _I),
     "nsvf_generate_rays": ([_CAM, _P, _P, _P], _I),
     "nsvf_render_hits_camera": ([_CAM, _P, _I, _I, _I, _F, _P, _P, _P, _P, _P, _P, _P, _P], _I),
+    "nsvf_render_offsets_workspace_ints": ([_L], _L),
+    "nsvf_render_offsets": ([_P, _P, _L, _P, _P, _P, _P, _P, _I, _P, _P], _I),
     "nsvf_render_compact": ([_P, _P, _L, _P, _P], _I),
     "nsvf_render_sample_coarse": ([_P, _P, _L, _P, _P, _P, _P, _P, _I, _F, _I, _F, _P, _P, _P,
                                    _P, _P, _I, _P, _L, _P], _I),

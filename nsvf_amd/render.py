@@ -499,7 +499,7 @@ class Renderer:
         return {"hits": (R * P * 4, i32), "count": (R, i32), "tot": (R, f32), "flag": (R, i32),
                 "c_bound": (R, i32), "scalars": (8, i32), "f_bound": (R, i32), "rank": (R, i32),
                 "hit_list": (R, i32), "c_off": (R, i32),
-                "scan_ws": (int(lib().nsvf_scan_workspace_ints(R)), i32),
+                "scan_ws": (int(lib().nsvf_render_offsets_workspace_ints(R)), i32),
                 "ray_rgb": (R * 3, f32), "ray_depth": (R, f32), "ray_missed": (R, f32),
                 "c_cnt": (R, i32), "f_off": (R, i32), "f_cnt": (R, i32),
                 "out": (R * 5, f32), "seg_bounds": (17, i32), "seg_max": (16, i32)}
@@ -630,15 +630,11 @@ class Renderer:
         intersect(sc, P, hits, count, tot, flag, c_bound, st)
         self._mark("intersect")
         scal = self._buf("scalars", 8, torch.int32)   # [n_hit, slots_c, max_c, slots_f]
-        scal.zero_()
-        f_bound = self._buf("f_bound", R, torch.int32)
-        f_bound.zero_()
-        rank = self._buf("rank", R, torch.int32)
-        self._scan(flag, rank, R, scal[0:1])
-        hit_list = self._buf("hit_list", R, torch.int32)
-        check(L.nsvf_render_compact(_p(flag), _p(rank), R, _p(hit_list), st), "render_compact")
-        c_off = self._buf("c_off", R, torch.int32)
-        self._scan(c_bound, c_off, R, scal[1:2])
+        ws = self._buf("scan_ws", int(L.nsvf_render_offsets_workspace_ints(R)), torch.int32)
+        check(L.nsvf_render_offsets(
+            _p(flag), _p(c_bound), R, _p(self._buf("rank", R, torch.int32)),
+            _p(self._buf("hit_list", R, torch.int32)), _p(self._buf("c_off", R, torch.int32)),
+            _p(self._buf("f_bound", R, torch.int32)), _p(scal), 8, _p(ws), st), "render_offsets")
         if self._host is None:
             self._host = torch.zeros(2, dtype=torch.int32, pin_memory=True)
         # the one device-to-host read of the view: hit rays and slot total
