@@ -49,6 +49,11 @@ def _ptr(t):
 
 
 def _stream(dev):
+    """The device's current stream, as a C handle.  A device with an index
+    asks for the handle itself: 0.4 us against 5 for a Stream object, of which
+    a training step makes eleven."""
+    if isinstance(dev, torch.device) and dev.index is not None:
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(dev.index))
     return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 

@@ -24,6 +24,7 @@ import numpy as np
 import torch
 
 from . import geometry
+from ._ext import _stream
 from ._lib import check, lib
 from .field import pack_mlp
 from .scene import VoxelScene
@@ -38,10 +39,6 @@ _WEIGHTS = {0: "bf16", 1: "f32", 2: "bf16x3"}
 
 def _p(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
-
-
-def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
 def node_boxes(centers, children, half_voxel):

@@ -21,12 +21,14 @@ as in the reference, on request).
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from ._ext import _stream
 from ._lib import check, lib
 from .field import pack_layer_bf16
 from .render import BG_COLOR, BG_DEPTH, CoarseStream, DeviceScene, Renderer, coherent_order
@@ -35,10 +37,6 @@ from .scene import VoxelScene
 
 def _p(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
-
-
-def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
 def _need_cuda(t, name):
@@ -300,12 +298,8 @@ class FieldMLP(torch.autograd.Function):
         check(L_.nsvf_mlp_train_backward(D, H, L, _p(packed), _p(emb), M, _p(dout), _p(demb),
                                          _p(partial), n_part, _p(dparams), _stream(dev)),
               "mlp_train_backward")
-        grads, o = [], 0
-        for shp in ctx.param_shapes:
-            n = int(np.prod(shp))
-            grads.append(dparams[o:o + n].view(shp))
-            o += n
-        return (demb, *grads)
+        sizes = [math.prod(s) for s in ctx.param_shapes]
+        return (demb, *(g.view(s) for g, s in zip(dparams.split(sizes), ctx.param_shapes)))
 
 
 _X3_INDEX = {}
@@ -478,12 +472,8 @@ class FieldMLPx3(FieldMLP):
         check(L_.nsvf_mlp_train_backward_x3(D, H, L, _p(packed), _p(x3w), _p(emb), M, _p(dout),
                                             _p(demb), _p(partial), n_part, _p(dparams),
                                             _stream(dev)), "mlp_train_backward_x3")
-        grads, o = [], 0
-        for shp in ctx.param_shapes:
-            n = int(np.prod(shp))
-            grads.append(dparams[o:o + n].view(shp))
-            o += n
-        return (demb, *grads)
+        sizes = [math.prod(s) for s in ctx.param_shapes]
+        return (demb, *(g.view(s) for g, s in zip(dparams.split(sizes), ctx.param_shapes)))
 
 
 class TrainableField(nn.Module):

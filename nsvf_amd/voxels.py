@@ -20,6 +20,7 @@ from dataclasses import replace
 import numpy as np
 import torch
 
+from ._ext import _stream
 from ._lib import check, lib
 from .render import DeviceScene
 from .scene import VoxelScene
@@ -29,10 +30,6 @@ PRECISIONS = {"bf16": 0, "fp32": 1, "bf16x3": 2}
 
 def _p(t):
     return ctypes.c_void_p(t.data_ptr())
-
-
-def _stream(dev):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
 
 
 def prune_scores(sc: DeviceScene, precision="fp32", bits=16, chunk=65536, x3_chunk=None):
