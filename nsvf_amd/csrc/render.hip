@@ -756,22 +756,20 @@ struct SampleBinsT {
 };
 using SampleBins = SampleBinsT<false>;
 
-__device__ __forceinline__ void grouped_neighbours(int64_t n, int64_t N, int64_t* ray0,
+__device__ __forceinline__ void grouped_neighbours(uint32_t n, uint32_t N, int64_t* ray0,
                                                    int64_t* next) {
-  constexpr int G = 200, chunk = 800;  // clib/__init__.py:234,259
-  const int64_t Kc = (N + G - 1) / G;
-  const int64_t g = n / Kc, c = n - g * Kc;
-  const int64_t c0 = (c / chunk) * chunk;
-  const int64_t W = min(int64_t(chunk), Kc - c0);
-  const int64_t n0 = g * Kc + c0;
+  constexpr uint32_t G = 200, chunk = 800;  // clib/__init__.py:234,259
+  const uint32_t Kc = (N + G - 1) / G;
+  const uint32_t g = n / Kc, c = n - g * Kc;
+  const uint32_t c0 = (c / chunk) * chunk;
+  const uint32_t W = min(chunk, Kc - c0);
+  const uint32_t n0 = g * Kc + c0;
   *ray0 = n0 < N ? n0 : 0;
-  int64_t nn;
-  if (c - c0 < W - 1)
-    nn = n + 1;
-  else if (g < G - 1)
-    nn = (g + 1) * Kc + c0;
-  else
-    nn = -1;
+  if (c - c0 + 1 >= W && g + 1 >= G) {
+    *next = -1;
+    return;
+  }
+  const uint32_t nn = c - c0 + 1 < W ? n + 1 : n0 + Kc;
   *next = nn >= N ? 0 : nn;
 }
 
@@ -818,7 +816,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
   __shared__ int32_t lds_id[kSampleWaves][kCoarseBins];
   __shared__ int block_max;
   __shared__ int block_seg_max[kMaxSegments];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t N = *n_hit_dev;
   if (threadIdx.x == 0) block_max = 0;
   if (threadIdx.x < kMaxSegments) block_seg_max[threadIdx.x] = 0;
@@ -828,7 +826,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
        n += int64_t(gridDim.x) * kSampleWaves) {
     const int32_t r = hit_list[n];
     int64_t n0, nn;
-    grouped_neighbours(n, N, &n0, &nn);
+    grouped_neighbours(uint32_t(n), uint32_t(N), &n0, &nn);
     const int32_t r0 = hit_list[n0];
     const int cnt = count[r];
     HitBins bins{hits + int64_t(r) * n_max, cnt, tot[r], hits + int64_t(r0) * n_max, count[r0],
@@ -939,7 +937,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
   __shared__ float lds_c[kSampleWaves][kFineBins], lds_lo[kSampleWaves][kFineBins],
       lds_hi[kSampleWaves][kFineBins];
   __shared__ int32_t lds_id[kSampleWaves][kFineBins];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int64_t N = *n_hit_dev;
   const int P_frame = *c_max_dev;  // bin columns = longest coarse row
   for (int64_t n = int64_t(blockIdx.x) * kSampleWaves + wave; n < N;
@@ -952,7 +950,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(6))) voi
     FieldReuse reuse{src ? src + f_off[r] : nullptr};
     if (P > 0) {
       int64_t n0, nn;
-      grouped_neighbours(n, N, &n0, &nn);
+      grouped_neighbours(uint32_t(n), uint32_t(N), &n0, &nn);
       const int32_t r0 = hit_list[n0];
       const int64_t off = c_off[r];
       const int cnt = c_cnt[r];

@@ -42,22 +42,22 @@ struct FlatNoise {
 };
 
 // Bins of hit ray n of [N,P] rows under the reference's regrouping.
-__device__ __forceinline__ void grouped_neighbours(int64_t n, int64_t N, int G, int chunk,
-                                                   int64_t* ray0, int64_t* next) {
-  const int64_t Kc = (N + G - 1) / G;  // columns per group row (H / G)
-  const int64_t g = n / Kc, c = n - g * Kc;
-  const int64_t c0 = (c / chunk) * chunk;
-  const int64_t W = min(int64_t(chunk), Kc - c0);
-  int64_t n0 = g * Kc + c0;
+__device__ __forceinline__ void grouped_neighbours(uint32_t n, uint32_t N, uint32_t G,
+                                                   uint32_t chunk, int64_t* ray0, int64_t* next) {
+  const uint32_t Kc = (N - 1) / G + 1;  // columns per group row (H / G)
+  const uint32_t g = n / Kc, c = n - g * Kc;
+  const uint32_t c0 = (c / chunk) * chunk;
+  const uint32_t W = min(chunk, Kc - c0);
+  const uint32_t n0 = g * Kc + c0;
   *ray0 = n0 < N ? n0 : 0;  // rows past N are copies of row 0
-  int64_t nn;
-  if (c - c0 < W - 1)
-    nn = n + 1;
-  else if (g < G - 1)
-    nn = (g + 1) * Kc + c0;
-  else
-    nn = -1;  // one past the chunk buffer
-  *next = (nn >= N) ? 0 : nn;
+  if (c - c0 + 1 >= W && g + 1 >= G) {
+    *next = -1;  // one past the chunk buffer
+    return;
+  }
+  // the next column, or the next group row's first of this chunk (64 bits: a
+  // group count near 2^31 has rows of one column)
+  const int64_t nn = c - c0 + 1 < W ? int64_t(n) + 1 : int64_t(n0) + Kc;
+  *next = nn >= int64_t(N) ? 0 : nn;
 }
 
 // RowSink that also counts the samples with a voxel id.
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void icdf_rows_kernel(
        n += int64_t(gridDim.x) * kRowWaves) {
     int64_t ray0, next;
     if constexpr (kGrouped) {
-      grouped_neighbours(n, N, G, chunk, &ray0, &next);
+      grouped_neighbours(uint32_t(n), uint32_t(N), G, chunk, &ray0, &next);
     } else {
       ray0 = n / R * R;
       next = n + 1 < N ? n + 1 : -1;
