@@ -30,6 +30,13 @@ inline int check_launch(const char* what) {
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// atomicMax for a maximum that thousands of blocks raise: atomics on one
+// address go one after another, so those that would change nothing are left
+// out (a stale value read here only costs the atomic).
+__device__ __forceinline__ void raise_max(int32_t* p, int32_t v) {
+  if (v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, v);
+}
+
 // Bitwise or of v over each group of 8 lanes, to all of them (DPP: lane ^ 1,
 // lane ^ 2, then the mirror of the 8).
 __device__ __forceinline__ uint32_t or8(uint32_t v) {

@@ -848,9 +848,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
   }
   if (lane == 0) atomicMax(&block_max, wave_max);
   __syncthreads();
-  if (threadIdx.x == 0 && block_max > 0) atomicMax(max_count, block_max);
+  if (threadIdx.x == 0 && block_max > 0) raise_max(max_count, block_max);
   if (int(threadIdx.x) < n_seg && block_seg_max[threadIdx.x] > 0)
-    atomicMax(&seg_max[threadIdx.x], block_seg_max[threadIdx.x]);
+    raise_max(&seg_max[threadIdx.x], block_seg_max[threadIdx.x]);
 }
 
 // Column sum of (p + 1e-5) over the P bin columns of a fine-pass ray

@@ -330,7 +330,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void icdf_rows_kernel(
   if (max_valid) {
     if (lane == 0) atomicMax(&best, most);
     __syncthreads();
-    if (threadIdx.x == 0 && best > 0) atomicMax(max_valid, best);
+    if (threadIdx.x == 0 && best > 0) raise_max(max_valid, best);
   }
 }
 
