@@ -600,7 +600,7 @@ def rows(args, dev, sc, dsc):
     # one training step: forward, MSE against U(0,1) targets, backward --
     # with the HIP training MLP, and with torch's Linear layers for reference
     target = torch.rand((R, 3), device=dev)
-    mlp_names = {"hip": "HIP FP32 MFMA",
+    mlp_names = {"hip": "HIP FP32 (FP16 pairs)",
                  "hip_x3": "HIP split BF16 (the backward's head in FP32)",
                  "torch": "torch FP32 nn.Linear"}
     for key, impl in (("train_step", "hip"), ("train_step_split_bf16", "hip_x3"),
@@ -683,17 +683,18 @@ def rows(args, dev, sc, dsc):
                         "backward_split_bf16_ms": round(ms_fb3 - ms_f3, 3), "samples": M,
                         "forward_TFLOPs": round(M * fl / (ms_f * 1e-3) / 1e12, 1),
                         "backward_TFLOPs": round(bw_flops / (ms_b * 1e-3) / 1e12, 1),
-                        "peak_TFLOPs": 157.3}
+                        # three FP16 MFMAs per product
+                        "peak_TFLOPs": round(PEAK_BF16_TFLOPS / 3, 1)}
     del tf, prm, emb, dout
     torch.cuda.empty_cache()
     # pruning: 16^3 lattice per voxel through the field MLP, max relu(sigma)
     flops = sc.num_voxels * 4096 * sc.mlp.flops_per_sample()
     for prec, peak in (("bf16", PEAK_BF16_TFLOPS), ("bf16x3", PEAK_BF16_TFLOPS),
-                       ("fp32", 157.3)):
+                       ("fp32", PEAK_BF16_TFLOPS)):
         ms = _time_ms(lambda: prune_scores(dsc, prec), 2)
         tf_s = flops / (ms * 1e-3) / 1e12
-        # split BF16 runs three BF16 MFMAs per product
-        mfma_tf = tf_s * (3 if prec == "bf16x3" else 1)
+        # split BF16 and FP32 (FP16 pairs) run three 16-bit MFMAs per product
+        mfma_tf = tf_s * (1 if prec == "bf16" else 3)
         res[f"prune_{prec}"] = {"ms": round(ms, 2), "lattice_points": sc.num_voxels * 4096,
                                 "achieved_TFLOPs": round(tf_s, 1), "peak_TFLOPs": peak,
                                 "frac": round(mfma_tf / peak, 4)}

@@ -173,7 +173,7 @@ int nsvf_inverse_cdf_sampling_rows_max(const int32_t* pts_idx,
  * each voxel (offsets (2i+1-bits)/(bits-1) * vs/2 per axis, corners
  * included) evaluated with the field MLP, into vmax [n].  The reference keeps
  * a voxel when 1 - min exp(-relu sigma) > th, i.e. 1 - exp(-vmax) > th.
- * precision 0 = BF16 MFMA, 1 = FP32 MFMA (the reference computes in FP32);
+ * precision 0 = BF16 MFMA, 1 = FP32 (the reference computes in FP32);
  * wfrag/bias as for nsvf_field_eval; centers are the x-shifted centres.
  * bits a multiple of 4 (the reference uses 16).
  * ---------------------------------------------------------------------- */

@@ -31,7 +31,7 @@ from .scene import VoxelScene
 
 BG_DEPTH = 5.0              # fairnr/modules/implicit.py:19
 BG_COLOR = (1.0, 1.0, 1.0)  # fairnr/modules/field.py:69 (transparent background)
-# field MLP arithmetic: BF16 MFMA, FP32 MFMA, or split BF16 (three BF16 MFMAs
+# field MLP arithmetic: BF16 MFMA, FP32, or split BF16 (three BF16 MFMAs
 # per product on hi / lo operand parts, about 16 significant bits)
 PRECISIONS = {"bf16": 0, "fp32": 1, "bf16x3": 2}
 _WEIGHTS = {0: "bf16", 1: "f32", 2: "bf16x3"}

@@ -34,7 +34,7 @@ def _p(t):
 
 def prune_scores(sc: DeviceScene, precision="fp32", bits=16, chunk=65536, x3_chunk=None):
     """[N] float32: max over each voxel's bits^3 lattice of relu(sigma)
-    (encoder.py:620-646).  FP32 MFMA by default, as the reference evaluates
+    (encoder.py:620-646).  FP32 by default, as the reference evaluates
     the field in FP32; "bf16" is faster and may flip voxels whose max is
     within about 1% of the threshold; "bf16x3" (split BF16, the renderer's
     served precision) keeps FP32-level accuracy at a fraction of the FP32
