@@ -71,8 +71,9 @@ struct CountedRowSink {
 };
 
 constexpr int kRowWaves = 4;
-constexpr int kRowBins = 256;     // bins of a row staged in LDS
-constexpr int kRowBlocks = 8192;  // 16 KB of LDS each: more than the chip holds at once
+constexpr int kRowBins = 256;     // bins of a row staged in LDS: 16 KB per block,
+constexpr int kWideBins = 1024;   // or 64 KB (two blocks per CU) where rows have more
+constexpr int kRowBlocks = 8192;  // more than the chip holds at once
 
 __device__ __forceinline__ int first_set(uint64_t mask) {
   return mask ? __ffsll(static_cast<unsigned long long>(mask)) - 1 : 64;
@@ -84,7 +85,7 @@ __device__ __forceinline__ int first_set(uint64_t mask) {
 // left-to-right prefix of the probabilities), but every sample is written,
 // also one without a voxel id, its distance as it is.  Rows the closed form
 // does not cover run icdf_ray on lane 0: no valid first bin or more than
-// kRowBins, a negative or NaN probability (C must not fall), a step count or
+// bins_cap, a negative or NaN probability (C must not fall), a step count or
 // size that is not positive and within the row, noise outside [0, 1] (the
 // steps' cdf must not fall).  Returns the number of samples written with a
 // voxel id; *count: the samples made, *dropped: those that found no slot
@@ -92,8 +93,8 @@ __device__ __forceinline__ int first_set(uint64_t mask) {
 template <bool kNoise, bool kCount>
 __device__ int icdf_row_wave(const OpBins& bins, int P, float steps, float fixed_step,
                              const FlatNoise& noise, int compat, int S, const RowSink& out,
-                             float* C, float* lo, float* hi, int32_t* id, int* count,
-                             int* dropped) {
+                             int bins_cap, float* C, float* lo, float* hi, int32_t* id,
+                             int* count, int* dropped) {
   const int lane = threadIdx.x & 63;
   const auto u_at = [&](int i) { return kNoise ? noise.at(i) : 0.5f; };
   const auto put = [&](int pos, int32_t v, float d, float mid) {
@@ -123,7 +124,7 @@ __device__ int icdf_row_wave(const OpBins& bins, int P, float steps, float fixed
     const int32_t v = k < P ? bins.id(k) : -1;
     const int here = first_set(__ballot(v == -1));
     if (here > 0) {
-      if (t0 + here > kRowBins) {
+      if (t0 + here > bins_cap) {
         seq = true;
         break;
       }
@@ -287,14 +288,16 @@ __global__ __launch_bounds__(64 * kRowWaves) void icdf_rows_kernel(
     int P, int S, int G, int chunk, float fixed_step_size, int compat,
     int32_t* __restrict__ out_idx, float* __restrict__ out_depth,
     float* __restrict__ out_dists, int32_t* __restrict__ max_valid,
-    unsigned long long* __restrict__ flags) {
-  __shared__ float C[kRowWaves][kRowBins], lo[kRowWaves][kRowBins], hi[kRowWaves][kRowBins];
-  __shared__ int32_t id[kRowWaves][kRowBins];
+    unsigned long long* __restrict__ flags, int bins_cap) {
+  extern __shared__ float staged[];   // [wave][C, lo, hi, id][bins_cap]
   __shared__ int best;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (threadIdx.x == 0) best = 0;
   __syncthreads();
+  float* C = staged + w * 4 * bins_cap;
+  float *lo = C + bins_cap, *hi = lo + bins_cap;
+  int32_t* id = reinterpret_cast<int32_t*>(hi + bins_cap);
   int most = 0;
   for (int64_t n = int64_t(blockIdx.x) * kRowWaves + w; n < N;
        n += int64_t(gridDim.x) * kRowWaves) {
@@ -313,7 +316,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void icdf_rows_kernel(
     const float st = steps[n];
     int count, dropped;
     const int valid = icdf_row_wave<kNoise, kCount>(bins, P, st, fixed_step_size, nz, compat, S,
-                                                    row, C[w], lo[w], hi[w], id[w], &count,
+                                                    row, bins_cap, C, lo, hi, id, &count,
                                                     &dropped);
     most = max(most, valid);
     for (int t = min(count, S) + lane; t < S; t += 64) {
@@ -341,12 +344,14 @@ static void launch_icdf(const int32_t* pts_idx, const float* min_depth, const fl
                         int32_t* out_idx, float* out_depth, float* out_dists, int32_t* max_valid,
                         int64_t* flags, void* stream) {
   const dim3 grid(unsigned(std::min<int64_t>(ceil_div(N, kRowWaves), kRowBlocks)));
+  const int cap = P <= kRowBins ? kRowBins : kWideBins;
   hipLaunchKernelGGL((flags ? icdf_rows_kernel<kNoise, kGrouped, true>
                             : icdf_rows_kernel<kNoise, kGrouped, false>),
-                     grid, dim3(64 * kRowWaves), 0, as_stream(stream), pts_idx, min_depth,
+                     grid, dim3(64 * kRowWaves), size_t(kRowWaves) * 4 * cap * sizeof(float),
+                     as_stream(stream), pts_idx, min_depth,
                      max_depth, noise, probs, steps, N, R, P, S, G, chunk, fixed_step_size, compat,
                      out_idx, out_depth, out_dists, max_valid,
-                     reinterpret_cast<unsigned long long*>(flags));
+                     reinterpret_cast<unsigned long long*>(flags), cap);
 }
 
 // Uniform sampling of one ray (fairnr/clib/src/sample_gpu.cu:42-105) into a

@@ -37,8 +37,8 @@ def prune_scores(sc: DeviceScene, precision="fp32", bits=16, chunk=65536, x3_chu
     (encoder.py:620-646).  FP32 by default, as the reference evaluates
     the field in FP32; "bf16" is faster and may flip voxels whose max is
     within about 1% of the threshold; "bf16x3" (split BF16, the renderer's
-    served precision) keeps FP32-level accuracy at a fraction of the FP32
-    time.  chunk: voxels per launch of the FP32 / BF16 kernels; x3_chunk:
+    served precision) keeps FP32-level accuracy in about the FP32 time (and is
+    much faster for shapes whose FP32 runs on the FP32 MFMAs).  chunk: voxels per launch of the FP32 / BF16 kernels; x3_chunk:
     voxels per chunk of the split-BF16 path (default 2048)."""
     if precision == "bf16x3":
         return _prune_scores_x3(sc, bits, **({} if x3_chunk is None else {"chunk_voxels": x3_chunk}))

@@ -1,5 +1,5 @@
 """The inverse-CDF ops give a wavefront a row: bit-equal to the oracle's walk
-at the edges of its 64-lane passes and 256 staged bins, and on the rows that
+at the edges of its 64-lane passes and 256 or 1,024 staged bins, and on the rows that
 the closed form does not cover."""
 import ctypes
 
@@ -54,7 +54,7 @@ def spoil(kind, a, noise):
         lo[idx == -1], hi[idx == -1] = 1.0, 2.0
 
 
-CASES = [(p, "plain") for p in (1, 2, 63, 64, 65, 128, 255, 256, 257, 300)] + [
+CASES = [(p, "plain") for p in (1, 2, 63, 64, 65, 128, 255, 256, 257, 300, 1024, 1025)] + [
     (20, k) for k in ("negative", "nan", "short", "long", "noise_ends", "noise_out", "no_steps",
                       "no_bins", "pads")]
 
