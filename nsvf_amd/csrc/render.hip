@@ -333,7 +333,7 @@ __device__ __forceinline__ float sum_group(const GroupLane& ln, const HitRec* ro
 
 // Stable sort of the row by entry depth: up to 64 hits by their ranks (eight
 // records in each lane, the depths in the group's waiting words), longer rows
-// by insertion on one lane.
+// by insertion, eight hits shifted at a time.
 __device__ __forceinline__ void sort_group(const GroupLane& ln, HitRec* row, int cnt) {
   constexpr int N = 8;
   float* depths = reinterpret_cast<float*>(ln.wait - ln.s);
@@ -363,16 +363,23 @@ __device__ __forceinline__ void sort_group(const GroupLane& ln, HitRec* row, int
 #pragma unroll
     for (int i = 0; i < N; ++i)
       if (8 * i + ln.s < cnt) reinterpret_cast<float4*>(row)[rank[i]] = h[i];
-  } else if (ln.s == 0) {
+  } else {
     for (int k = 1; k < cnt; ++k) {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
       const HitRec v = row[k];
-      int j = k - 1;
-      while (j >= 0 && row[j].lo > v.lo) {
-        row[j + 1] = row[j];
-        --j;
+      int end = k;   // the place for v: after the last hit that is not deeper
+      uint32_t deeper = 0xFFu;
+      while (deeper == 0xFFu && end > 0) {
+        const int i = end - 8 + ln.s;
+        const HitRec h = row[max(i, 0)];
+        const bool d = i >= 0 && h.lo > v.lo;
+        if (d) row[i + 1] = h;
+        deeper = ln.votes(d);
+        end -= __popc(deeper);
       }
-      row[j + 1] = v;
+      if (ln.s == 0) row[end] = v;
     }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
   }
 }
 
