@@ -406,7 +406,7 @@ __device__ __forceinline__ int redo_group(const GroupLane& ln, const float o[3],
 // depths are not strictly increasing (equal entries: the tie order must be
 // the reference's), is traversed again in the reference's order -- child
 // slots 7..0 (intersect_gpu.cu:201-230), which is slot = i ^ 7 -- and stably
-// insertion-sorted, which is exactly the reference pipeline's result: the
+// sorted, which is exactly the reference pipeline's result: the
 // exact boxes prune only subtrees without a hit, so both traversals emit the
 // same leaves in the same order and stop at the same n_max-th hit.
 template <bool kCamera>
