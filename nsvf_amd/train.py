@@ -302,28 +302,39 @@ class FieldMLP(torch.autograd.Function):
         return (demb, *(g.view(s) for g, s in zip(dparams.split(sizes), ctx.param_shapes)))
 
 
-_X3_INDEX = {}
+def _x3_positions(shapes):
+    """For weights of the given [out, in] shapes: the position, in
+    [0, W_0 flat, W_1 flat, ...] (0: zero padding), of every element of the
+    split-BF16 kernel's fragments in their order, int64 [fragments * 512]
+    (pack_layer_bf16 applied to the positions; they stay below 2^24, so
+    its float32 arrays carry them exactly)."""
+    parts, base = [], 1
+    for O, K in shapes:
+        pos = (np.arange(O * K, dtype=np.float64) + base).reshape(O, K).astype(np.float32)
+        parts.append(pack_layer_bf16(pos, ((K + 31) // 32) * 32).reshape(-1))
+        base += O * K
+    if base >= 1 << 24:
+        raise ValueError("split-BF16 training MLP: too many weights")
+    return np.concatenate(parts).astype(np.int64)
+
+
+_POSITIONS = {}
+
+
+def _on_device(key, make, device):
+    """make()'s array as a tensor on the device, kept under (key, device).  One
+    blocking copy from the host: complete when the entry is visible, so calls
+    on other streams need no order with the first one."""
+    key = (key, str(device))
+    got = _POSITIONS.get(key)
+    if got is None:
+        got = _POSITIONS[key] = torch.from_numpy(make()).to(device)
+    return got
 
 
 def _x3_index(shapes, device):
-    """For weights of the given [out, in] shapes: the position, in
-    [0, W_0 flat, W_1 flat, ...] (0: zero padding), of every element of the
-    split-BF16 kernel's fragments in their order, [fragments * 512] int64
-    (pack_layer_bf16 applied to the positions; they stay below 2^24, so
-    its float32 arrays carry them exactly)."""
-    key = (tuple(shapes), str(device))
-    idx = _X3_INDEX.get(key)
-    if idx is None:
-        parts, base = [], 1
-        for O, K in shapes:
-            pos = (np.arange(O * K, dtype=np.float64) + base).reshape(O, K).astype(np.float32)
-            parts.append(pack_layer_bf16(pos, ((K + 31) // 32) * 32).reshape(-1))
-            base += O * K
-        if base >= 1 << 24:
-            raise ValueError("split-BF16 training MLP: too many weights")
-        idx = torch.from_numpy(np.concatenate(parts).astype(np.int64)).to(device)
-        _X3_INDEX[key] = idx
-    return idx
+    """_x3_positions on the device."""
+    return _on_device(("forward", tuple(shapes)), lambda: _x3_positions(shapes), device)
 
 
 def pack_mlp_x3(weights, biases):
@@ -348,30 +359,27 @@ def pack_mlp_x3(weights, biases):
     return frags, bias
 
 
-_X3T_INDEX = {}
-
-
-def _x3_train_index(shapes, device):
+def _x3_train_positions(shapes):
     """For weights of the given [out, in] shapes (hidden layers, then the
     head): the position, in [0, W_0 flat, W_1 flat, ...] (0: zero padding),
     of every element of the split-BF16 backward's fragments in their order
-    -- W_0 .. W_{L-1}, then their transposes -- [fragments * 512] int64."""
-    key = (tuple(shapes), str(device))
-    idx = _X3T_INDEX.get(key)
-    if idx is None:
-        pos, base = [], 1
-        for O, K in shapes:
-            pos.append((np.arange(O * K, dtype=np.float64) + base).reshape(O, K).astype(np.float32))
-            base += O * K
-        if base >= 1 << 24:
-            raise ValueError("split-BF16 training MLP: too many weights")
-        hidden = pos[:-1]
-        parts = [pack_layer_bf16(q, ((q.shape[1] + 31) // 32) * 32).reshape(-1) for q in hidden]
-        parts += [pack_layer_bf16(np.ascontiguousarray(q.T), ((q.shape[0] + 31) // 32) * 32)
-                  .reshape(-1) for q in hidden]
-        idx = torch.from_numpy(np.concatenate(parts).astype(np.int64)).to(device)
-        _X3T_INDEX[key] = idx
-    return idx
+    -- W_0 .. W_{L-1}, then their transposes -- int64 [fragments * 512]."""
+    pos, base = [], 1
+    for O, K in shapes:
+        pos.append((np.arange(O * K, dtype=np.float64) + base).reshape(O, K).astype(np.float32))
+        base += O * K
+    if base >= 1 << 24:
+        raise ValueError("split-BF16 training MLP: too many weights")
+    hidden = pos[:-1]
+    parts = [pack_layer_bf16(q, ((q.shape[1] + 31) // 32) * 32).reshape(-1) for q in hidden]
+    parts += [pack_layer_bf16(np.ascontiguousarray(q.T), ((q.shape[0] + 31) // 32) * 32)
+              .reshape(-1) for q in hidden]
+    return np.concatenate(parts).astype(np.int64)
+
+
+def _x3_train_index(shapes, device):
+    """_x3_train_positions on the device."""
+    return _on_device(("backward", tuple(shapes)), lambda: _x3_train_positions(shapes), device)
 
 
 def pack_mlp_train_x3(weights):
@@ -392,7 +400,16 @@ def pack_mlp_train_x3(weights):
     return torch.stack([hi, lo], 1).reshape(-1).view(torch.int16)
 
 
-_SPLIT_INDEX = {}
+def _split_index(shapes, backward, device):
+    """_x3_positions, with backward also _x3_train_positions after them, in one
+    tensor on the device; and the length of each."""
+    def both():
+        f = _x3_positions(shapes)
+        return np.concatenate([f, _x3_train_positions(shapes)]) if backward else f
+
+    idx = _on_device(("both" if backward else "forward", tuple(shapes)), both, device)
+    nf = 512 * sum((O + 15) // 16 * ((K + 31) // 32) for O, K in shapes)
+    return idx, nf, idx.numel() - nf
 
 
 def _pack_split(weights, biases, count=0, backward=False):
@@ -402,13 +419,7 @@ def _pack_split(weights, biases, count=0, backward=False):
     dev = weights[0].device
     shapes = [tuple(w.shape) for w in weights]
     D, H, L = _mlp_shape(weights)
-    key = (tuple(shapes), str(dev), backward)
-    got = _SPLIT_INDEX.get(key)
-    if got is None:
-        f = _x3_index(shapes, dev)
-        b = _x3_train_index(shapes, dev) if backward else f[:0]
-        got = _SPLIT_INDEX[key] = (torch.cat([f, b]), f.numel(), b.numel())
-    idx, nf, nb = got
+    idx, nf, nb = _split_index(shapes, backward, dev)
     frags = torch.empty(2 * (nf + nb), dtype=torch.int16, device=dev)
     bias = torch.empty(L * H + 16, dtype=torch.float32, device=dev)
     m_dev = torch.empty(1, dtype=torch.int32, device=dev)
