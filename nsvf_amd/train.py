@@ -343,7 +343,7 @@ def pack_mlp_x3(weights, biases):
     field.pack_mlp's "bf16x3": per fragment its 512 hi parts bf16(w), then
     its lo parts bf16(w - hi), round to nearest even)."""
     dev = weights[0].device
-    if dev.type == "cuda":
+    if dev.type == "cuda" and _split_packable(weights, biases):
         frags, _, bias, _ = _pack_split(weights, biases)
         return frags, bias
     idx = _x3_index([tuple(w.shape) for w in weights], dev)
@@ -412,11 +412,22 @@ def _split_index(shapes, backward, device):
     return idx, nf, idx.numel() - nf
 
 
+def _split_packable(weights, biases):
+    """Whether the packing kernel takes these layers: up to 7 hidden ones of one
+    width H, a 4-wide head, a bias per output."""
+    D, H, L = _mlp_shape(weights)
+    shapes = [(H, D)] + [(H, H)] * (L - 1) + [(4, H)]
+    return (1 <= L <= 7 and [tuple(w.shape) for w in weights] == shapes
+            and [tuple(b.shape) for b in biases] == [(o,) for o, _ in shapes])
+
+
 def _pack_split(weights, biases, count=0, backward=False):
     """pack_mlp_x3's fragments and biases, with backward=True also
     pack_mlp_train_x3's fragments (else None), and `count` as an int32 [1],
     in one launch."""
     dev = weights[0].device
+    if not _split_packable(weights, biases):
+        raise RuntimeError("split-BF16 packing: hidden layers of one width and a 4-wide head")
     shapes = [tuple(w.shape) for w in weights]
     D, H, L = _mlp_shape(weights)
     idx, nf, nb = _split_index(shapes, backward, dev)

@@ -49,6 +49,31 @@ def test_no_queued_operation_makes_the_table(monkeypatch, backward):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("widths", [[32] + [64] * 9 + [4], [32, 64, 48, 4], [32, 64, 64, 3],
+                                    [32, 64, 64, 9], [20, 4], [48, 256, 256, 256, 256, 4]])
+def test_any_layers_are_packed(device, widths):
+    """Layers that the packing kernel does not take (many, of several widths,
+    another head) have the same fragments as on the CPU, as those that it does."""
+    g = torch.Generator().manual_seed(6)
+    ws = [torch.randn(o, i, generator=g) for i, o in zip(widths, widths[1:])]
+    bs = [torch.randn(o, generator=g) for o in widths[1:]]
+    want, want_bias = train.pack_mlp_x3(ws, bs)
+    frags, bias = train.pack_mlp_x3([w.to(device) for w in ws], [b.to(device) for b in bs])
+    assert torch.equal(frags.cpu(), want) and torch.equal(bias.cpu(), want_bias)
+
+
+def test_the_kernel_takes_equal_layers_only():
+    make = lambda *widths: ([torch.zeros(o, i) for i, o in zip(widths, widths[1:])],
+                            [torch.zeros(o) for o in widths[1:]])
+    assert train._split_packable(*make(32, 128, 128, 128, 4))
+    assert train._split_packable(*make(20, 64, 4))
+    for widths in ([32] + [64] * 8 + [4], [32, 64, 48, 4], [32, 64, 64, 3], [20, 4]):
+        assert not train._split_packable(*make(*widths))
+    ws, bs = make(32, 64, 64, 4)
+    assert not train._split_packable(ws, bs[:1] + [torch.zeros(63)] + bs[2:])
+
+
+@pytest.mark.gpu
 def test_first_calls_on_two_streams(device):
     """The first call of a shape on a busy stream, the second on another one."""
     g = torch.Generator().manual_seed(4)
