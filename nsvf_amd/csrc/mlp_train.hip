@@ -1273,12 +1273,11 @@ template <int D, int H, int L>
 __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
                                                          float* __restrict__ stats) {
   __shared__ int best[4];
-  __shared__ float cols[H];
+  __shared__ float cols[16][H];   // each wave's column sums
   const int l = blockIdx.x, rows = l < L ? H : 4, in = l == 0 ? D : H;
   const float* W = net.w[l];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (threadIdx.x < 4) best[threadIdx.x] = 0;
-  if (threadIdx.x < H) cols[threadIdx.x] = 0.0f;
   __syncthreads();
   // |x| as integer bits order as the values do, NaN and infinity on top
   const auto up = [&](int k, float v) {
@@ -1315,13 +1314,19 @@ __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
   up(1, widest);
   up(0, top);
 #pragma unroll
-  for (int q = 0; q < H / 64; ++q) atomicAdd(&cols[lane + 64 * q], mine[q]);
+  for (int q = 0; q < H / 64; ++q) cols[wave][lane + 64 * q] = mine[q];
   float b = 0.0f;
   for (int i = threadIdx.x; i < rows; i += 1024)
     b = __int_as_float(max(__float_as_int(b), __float_as_int(net.b[l][i]) & 0x7FFFFFFF));
   up(3, b);
   __syncthreads();
-  up(2, threadIdx.x < H ? cols[threadIdx.x] : 0.0f);
+  // the waves' sums in order: the sums choose scales, so their last bits must
+  // not depend on timing
+  float col = 0.0f;
+  if (threadIdx.x < H)
+#pragma unroll
+    for (int w = 0; w < 16; ++w) col += cols[w][threadIdx.x];
+  up(2, col);
   __syncthreads();
   // row and column sums a little above their rounding
   if (threadIdx.x < 4) {
