@@ -36,6 +36,7 @@
 // hi = bf16(f), lo = bf16(f - hi), a product Wl Xh + Wh Xl + Wh Xh in FP32
 // accumulators.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "mlp_f16x3.h"
@@ -482,7 +483,8 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 // two below their largest, everything behind them is linear in it, and the
 // bounds of dz are then the same for every sample; the input gradient is
 // multiplied back.  In the weight gradients, sums over samples, each sample's
-// factor multiplies dz when it is read, relative to the chunk's largest.
+// factor multiplies dz when it is read, in bands of samples of like size
+// (BwdBands).
 // The FP16 matrix unit's sums come out low on average (measured: every bias
 // gradient's error negative, whatever its own sign).  That is below FP32's
 // rounding in one product, but a parameter's gradient adds a million: so every second sample's normalised gradient, and
@@ -516,10 +518,10 @@ struct BwdLds {
   unsigned short head[2][4][4][4][8];        // head weights hi / lo: [kt][g][logit][i]
   float back[4][kBwdChunk];                  // accumulator -> sum, layers 0..2 and head
   float scale[3][kBwdChunk];                 // sum -> parts, h0, h1, h2
-  _Float16 factor[3][kBwdChunk];             // weight gradients' sample factors: x0, h0, h1
+  _Float16 factor[kBwdWaves][kBwdChunk];     // each wave's sample factors of a weight gradient
   float unit[kBwdChunk];                     // 2^k of the normalised gradients (0: none)
-  float factor2[kBwdChunk];                  // the head's weight gradient's sample factors
   int top0[kBwdChunk];                       // largest h0 (float bits)
+  short dz_top[3][kBwdWaves][4];             // largest |dz| of each wave's lane groups (upper 16 bits)
   int wild;
 };
 static_assert(sizeof(BwdLds) <= 160 * 1024, "LDS");
@@ -627,16 +629,65 @@ __device__ __forceinline__ void bwd_layer(const unsigned short* p, const int (&a
   }
 }
 
-// sum[a][b] += 2^e x the sum over the chunk's samples of rows A (dz, NA tiles
+// Largest of the 16 lanes of a group, to its lane 15 (DPP row shifts; v >= 0).
+__device__ __forceinline__ int row_max15(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
+  return max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
+}
+
+// The samples of a chunk in bands of like size, for a sum over samples whose
+// terms are 2^q[lane] x operands of one scale: each step takes those within
+// 2^-width of the largest that are left, leaves their factors +-2^(q - top) in
+// the wave's row of LDS (0 for the others) and top in `top`; false when none
+// are left.  u: the samples' units (0: no gradient), us: their signs.
+// A factor multiplies the FP16 parts of an operand, whose low parts lose bits
+// to FP16's subnormals where it is small; in one band for the whole chunk, a
+// sample 2^-25 of the largest would vanish, also from the rows of a weight
+// gradient that the larger samples do not reach.  Gradients fall along a ray
+// with its transmittance, so samples that far apart are common.
+// Rows of dW that only samples 2^-k of their neighbours' reach, error against
+// 64 bits: 1.2e-6 for every k with 16 (up to 2.3e-6 at k = 15 .. 18 with 18,
+// 4.6e-6 with 20; all of the row from k = 25 on with one band).  A million
+// samples whose gradients spread over four decades, the whole call: 1,385 us
+// with one band, 1,407 with 18, 1,519 with 16.
+constexpr int kBand = 16, kHeadBand = 16;
+struct BwdBands {
+  int q;
+  float us;
+  bool left;
+  int top;
+  __device__ __forceinline__ BwdBands(int q_, float u, float sign)
+      : q(q_), us(copysignf(sign, u * sign)), left(u != 0.0f), top(0) {}
+  __device__ __forceinline__ bool next(_Float16* factor, int lane, int width) {
+    if (!__any(left)) return false;
+    const int m = row_max15(left ? q : 0);   // exponents are positive
+    top = __builtin_amdgcn_readlane(m, 15);
+#pragma unroll
+    for (int r = 1; r < 4; ++r) top = max(top, __builtin_amdgcn_readlane(m, 16 * r + 15));
+    const int d = q - top;
+    const bool in = left && d > -width;
+    wave_sync();   // the band before has been read
+    factor[lane] = in ? _Float16(us * __int_as_float((127 + d) << 23)) : _Float16(0.0f);
+    wave_sync();
+    left = left && !in;
+    return true;
+  }
+};
+
+// sum[a][b] += 2^e x the sum over a band's samples of rows A (dz, NA tiles
 // of 16) and B (the layer's input, NB tiles): rows from pa / pb on, the lane's
 // at[ks] halves on (row c, sample 32 ks + 8 g), lo planes `lo_a` / `lo_b` halves
-// on; factor: the samples' factors; by: their sign in this chunk.  A chunk's products start from 0 and are added by the vector unit:
+// on; factor: the samples' factors, multiplied by 2^up (what the rows leave of
+// FP16's range: the bound that dz was scaled by is loose, by some 2^10 for dz0);
+// by: their sign in this chunk.  A chunk's products start from 0 and are added by the vector unit:
 // the matrix unit rounds its accumulations toward zero, which over a block's
 // hundreds of steps into one accumulator cost 4e-6 of the gradient (1e-6 so).
 template <bool F16, int NA, int NB>
 __device__ __forceinline__ void bwd_dw(const unsigned short* pa, int lo_a,
                                        const unsigned short* pb, int lo_b, const int (&at)[2],
-                                       const _Float16* factor, int g, int e, float by,
+                                       const _Float16* factor, int up, int g, int e, float by,
                                        f32x4 (&sum)[NA][NB]) {
   constexpr int KS = kBwdChunk / 32;
   u32x4 ah[KS][NA], al[KS][NA];
@@ -646,12 +697,19 @@ __device__ __forceinline__ void bwd_dw(const unsigned short* pa, int lo_a,
     for (int a = 0; a < NA; ++a) {
       ah[ks][a] = lds128(pa + at[ks] + a * 16 * kBwdRow);
       al[ks][a] = lds128(pa + at[ks] + a * 16 * kBwdRow + lo_a);
-      if constexpr (F16) {
-        const f16x8 f = *reinterpret_cast<const f16x8*>(factor + 32 * ks + 8 * g);
+    }
+  if constexpr (F16) {
+    const _Float16 raise = _Float16(__int_as_float((127 + up) << 23));
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const f16x8 f = *reinterpret_cast<const f16x8*>(factor + 32 * ks + 8 * g) * raise;
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
         ah[ks][a] = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, ah[ks][a]) * f);
         al[ks][a] = __builtin_bit_cast(u32x4, __builtin_bit_cast(f16x8, al[ks][a]) * f);
       }
     }
+  }
 #pragma unroll
   for (int b = 0; b < NB; ++b) {
     f32x4 acc[NA];
@@ -680,14 +738,6 @@ __device__ __forceinline__ void bwd_dw(const unsigned short* pa, int lo_a,
 #pragma unroll
     for (int a = 0; a < NA; ++a) asm volatile("" : "+v"(sum[a][b]));
   }
-}
-
-// Largest of the 16 lanes of a group, to its lane 15 (DPP row shifts; v >= 0).
-__device__ __forceinline__ int row_max15(int v) {
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
-  return max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
 }
 
 // Exponent window of the FP16 form's operands, 2^-40 to 2^60 (or 0): every
@@ -990,40 +1040,39 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
     }
     __syncthreads();
 
-    // the samples' factors (lane = sample): exponents q of the normalised
-    // gradient times a layer's input, the chunk's largest, and the factors
-    // relative to it -- every wave the head's, one wave each of the others
-    int top[4] = {0, 0, 0, 0};
-    if constexpr (F16) {
+    // a layer's weight gradient (k = 0 .. 2) or the head's (3): the samples'
+    // exponents are those of the normalised gradient times the layer's input
+    const auto bands = [&](int k) {
       const float u = S.unit[lane];
       const int e = (__float_as_int(u) & 0x7FFFFFFF) >> 23;
-      const float us = copysignf(sign, u * sign);   // the sample's sign times the chunk's
-      int q[4];
-      q[0] = e + feature_exponent(S.back[0][lane], ew[0]);
+      return BwdBands(e + (k == 0 ? feature_exponent(S.back[0][lane], ew[0])
+                                  : 268 - (__float_as_int(S.scale[k > 0 ? k - 1 : 0][lane]) >> 23)),
+                      u, sign);
+    };
+    const auto weight_gradient = [&](auto layer, const unsigned short* pa,
+                                     const unsigned short* pb, int lo_b, auto& sum) {
+      constexpr int k = layer();
+      constexpr int NA = std::extent<std::remove_reference_t<decltype(sum)>, 0>::value;
+      constexpr int NB = std::extent<std::remove_reference_t<decltype(sum)>, 1>::value;
+      if constexpr (F16) {
+        BwdBands b = bands(k);
+        // the rows' headroom: those of two waves, or (dz0) of this one
+        const short* t = k == 0 ? S.dz_top[0][w] : S.dz_top[k][2 * (w & 3)];
+        int top = 0;
 #pragma unroll
-      for (int k = 0; k < 3; ++k) q[k + 1] = e + 268 - (__float_as_int(S.scale[k][lane]) >> 23);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int m = u == 0.0f ? 0 : q[k];   // exponents are positive
-        top[k] = __builtin_amdgcn_readlane(row_max15(m), 15);
-#pragma unroll
-        for (int r = 1; r < 4; ++r)
-          top[k] = max(top[k], __builtin_amdgcn_readlane(row_max15(m), 16 * r + 15));
-        const int d = q[k] - top[k];
-        if (k < 3) {
-          if (w == k)
-            S.factor[k][lane] =
-                u == 0.0f ? _Float16(0.0f)
-                          : _Float16(us * __int_as_float((127 + max(d, -40)) << 23));
-        } else {   // 2^(13 + d), 0 far below
-          S.factor2[lane] = u == 0.0f ? 0.0f : us * __int_as_float(max(140 + d, 0) << 23);
-        }
+        for (int i = 0; i < (k == 0 ? 4 : 8); ++i) top = max(top, int(t[i]));
+        const int up = min(max(ez[2 - k] - (__builtin_amdgcn_readfirstlane(top) >> 7), 0), 15);
+        while (b.next(S.factor[w], lane, kBand))
+          bwd_dw<true, NA, NB>(pa, kBwdPlane, pb, lo_b, at_row, S.factor[w], up, g,
+                               b.top + ez[2 - k] - 409 - up, sign, sum);
+      } else {
+        bwd_dw<false, NA, NB>(pa, kBwdPlane, pb, lo_b, at_row, nullptr, 0, g, 0, sign, sum);
       }
-      wave_sync();   // factor2: every wave writes the same values and reads them
-    }
+    };
     // ---- dz of a layer's accumulator (values v, sample 16 m + 4 g + r) into
     // plane set `to`; the bias gradient in true units
     const auto dz_out = [&](float (&v)[4][4], unsigned int bits, int to, int l, float sz) {
+      [[maybe_unused]] float largest = 0.0f;
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         f32x4 u = {1.0f, 1.0f, 1.0f, 1.0f};
@@ -1033,6 +1082,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         for (int r = 0; r < 4; ++r) {
           v[m][r] = (bits >> (4 * m + r)) & 1u ? v[m][r] : 0.0f;
           gb[l] = F16 ? __fmaf_rn(v[m][r], u[r], gb[l]) : gb[l] + v[m][r];
+          if constexpr (F16) largest = fmaxf(largest, fabsf(v[m][r]));
         }
         asm volatile("" : "+v"(gb[l]));
 #pragma unroll
@@ -1045,6 +1095,10 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         *reinterpret_cast<u32x2*>(&S.t[to][at_out[m]]) = hi;
         *reinterpret_cast<u32x2*>(&S.t[to][kBwdPlane + at_out[m]]) = lo;
         tile_fence();
+      }
+      if constexpr (F16) {
+        const int m = row_max15(__float_as_int(largest));
+        if (c == 15) S.dz_top[l][w][g] = short(m >> 16);
       }
     };
     // ---- dz2 = mask (W_head^T dl) in FP32, and dW_head
@@ -1060,31 +1114,42 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         }
       dz_out(v, mask[2], 3, 2, F16 ? f16_scale(ez[0]) : 1.0f);
     }
-    f32x4 ghc = zero4;
+    const auto head_gradient = [&]([[maybe_unused]] const _Float16* factor) {
+      f32x4 ghc = zero4;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      // dl of logit c (lanes c < 4) for samples 32 ks + 8 g + i, with their factors
-      unsigned int hw[4], lw[4];
+      for (int ks = 0; ks < 2; ++ks) {
+        // dl of logit c (lanes c < 4) for samples 32 ks + 8 g + i, with their
+        // factors: at 2^14, a band's smallest keep their 22 bits
+        unsigned int hw[4], lw[4];
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        float v[2], s[2] = {1.0f, 1.0f};
+        for (int p = 0; p < 4; ++p) {
+          float v[2], s[2] = {1.0f, 1.0f};
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int i = 32 * ks + 8 * g + 2 * p + k;
-          v[k] = c < 4 ? S.dl[i][c & 3] : 0.0f;
-          if constexpr (F16) s[k] = S.factor2[i];
+          for (int k = 0; k < 2; ++k) {
+            const int i = 32 * ks + 8 * g + 2 * p + k;
+            v[k] = c < 4 ? S.dl[i][c & 3] : 0.0f;
+            if constexpr (F16) s[k] = float(factor[i]) * 0x1p14f;
+          }
+          parts2<F16>(v[0], v[1], s[0], s[1], hw[p], lw[p]);
         }
-        parts2<F16>(v[0], v[1], s[0], s[1], hw[p], lw[p]);
+        const unsigned short* pb = &S.t[2][16 * w * kBwdRow + at_row[ks]];
+        ghc = mm16x3<F16>(u32x4{hw[0], hw[1], hw[2], hw[3]}, u32x4{lw[0], lw[1], lw[2], lw[3]},
+                          lds128(pb), lds128(pb + kBwdPlane), ghc);
+        tile_fence();
       }
-      const unsigned short* pb = &S.t[2][16 * w * kBwdRow + at_row[ks]];
-      ghc = mm16x3<F16>(u32x4{hw[0], hw[1], hw[2], hw[3]}, u32x4{lw[0], lw[1], lw[2], lw[3]},
-                        lds128(pb), lds128(pb + kBwdPlane), ghc);
-      tile_fence();
-    }
+      return ghc;
+    };
+    if constexpr (F16) {
+      BwdBands b = bands(3);
+      while (b.next(S.factor[w], lane, kHeadBand)) {
+        const f32x4 ghc = head_gradient(S.factor[w]);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      gh[r] = F16 ? __fmaf_rn(__builtin_amdgcn_ldexpf(ghc[r], top[3] + 128 - 409), sign, gh[r])
-                  : gh[r] + ghc[r];
+        for (int r = 0; r < 4; ++r)
+          gh[r] = __fmaf_rn(__builtin_amdgcn_ldexpf(ghc[r], b.top + 127 - 409), sign, gh[r]);
+      }
+    } else {
+      gh = gh + head_gradient(nullptr);
+    }
     asm volatile("" : "+v"(gh));
     __syncthreads();
     if (threadIdx.x < kBwdChunk) S.top0[threadIdx.x] = 0;
@@ -1095,8 +1160,6 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
     for (int m = 0; m < 4; ++m) acc[m] = zero4;
     bwd_layer<F16, 4>(S.t[3], at_tr, kBwdPlane, f, acc);
     f.load(F + 128 * (T::X_THIDDEN + w * T::KXH), lane);
-    bwd_dw<F16, 2, 4>(&S.t[3][row2], kBwdPlane, &S.t[1][col2], kBwdPlane, at_row, S.factor[2], g,
-                      top[2] + ez[0] - 409, sign, gw2);
     {
       const float bk = F16 ? f16_unscale(ez[0]) * f16_unscale(ew[2]) : 1.0f;
       float v[4][4];
@@ -1106,6 +1169,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         for (int r = 0; r < 4; ++r) v[m][r] = F16 ? acc[m][r] * bk : acc[m][r];
       dz_out(v, mask[1], 2, 1, F16 ? f16_scale(ez[1]) : 1.0f);
     }
+    weight_gradient(std::integral_constant<int, 2>{}, &S.t[3][row2], &S.t[1][col2], kBwdPlane, gw2);
     __syncthreads();
     // ---- dW_1 (dz1 x h0); dz0 = mask (W_1^T dz1) into dz2's planes
 #pragma unroll
@@ -1113,8 +1177,6 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
     bwd_layer<F16, 4>(S.t[2], at_tr, kBwdPlane, f, acc);
     // W_0^T: the input gradient's tile w & 1 (features) of samples 16 (w / 2)..
     f.load(F + 128 * (T::X_T0 + (w & 1) * T::KXH), lane);
-    bwd_dw<F16, 2, 4>(&S.t[2][row2], kBwdPlane, &S.t[0][col2], kBwdPlane, at_row, S.factor[1], g,
-                      top[1] + ez[1] - 409, sign, gw1);
     {
       const float bk = F16 ? f16_unscale(ez[1]) * f16_unscale(ew[1]) : 1.0f;
       float v[4][4];
@@ -1124,6 +1186,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         for (int r = 0; r < 4; ++r) v[m][r] = F16 ? acc[m][r] * bk : acc[m][r];
       dz_out(v, mask[0], 3, 0, F16 ? f16_scale(ez[2]) : 1.0f);
     }
+    weight_gradient(std::integral_constant<int, 1>{}, &S.t[2][row2], &S.t[0][col2], kBwdPlane, gw1);
     __syncthreads();
     // ---- dW_0 (dz0 x features) and the input gradient W_0^T dz0, whose
     // products run as W X so that a lane holds 4 features of a sample
@@ -1141,8 +1204,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
       if (s0 + i < M)
         *reinterpret_cast<f32x4*>(demb + (s0 + i) * D + 16 * (w & 1) + 4 * g) = d;
     }
-    bwd_dw<F16, 1, 2>(&S.t[3][16 * w * kBwdRow], kBwdPlane, S.x0, kBwdPlane0, at_row, S.factor[0], g,
-                      top[0] + ez[2] - 409, sign, gw0);
+    weight_gradient(std::integral_constant<int, 0>{}, &S.t[3][16 * w * kBwdRow], S.x0, kBwdPlane0, gw0);
     __syncthreads();
   }
 

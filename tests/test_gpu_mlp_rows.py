@@ -1,0 +1,92 @@
+"""The training backward where a tensor's largest entry says nothing: rows of
+the weight gradients that only samples with far smaller gradients than their
+neighbours' reach.
+
+Tolerance: the training tests' bar for FP32, 2e-5 of a tensor's largest entry,
+for each row (or column) by itself."""
+import numpy as np
+import pytest
+import torch
+
+from nsvf_amd import scene as S
+from nsvf_amd.train import FieldMLP
+
+pytestmark = pytest.mark.gpu
+
+BAR = 2e-5
+
+
+def _grads(fn, emb, params, dout, device):
+    leaves = [torch.from_numpy(x).to(device).requires_grad_() for x in (emb, *params)]
+    out = fn.apply(*leaves)
+    return [g.cpu().double() for g in
+            torch.autograd.grad(out, leaves, torch.from_numpy(dout).to(device))]
+
+
+def _grads64(emb, params, dout, margin=1e-5):
+    """float64 autograd; samples near a ReLU kink lose their gradient (dout is
+    changed)."""
+    leaves = [torch.from_numpy(x).double().requires_grad_() for x in (emb, *params)]
+    h, near = leaves[0], torch.zeros(len(emb), dtype=torch.bool)
+    for i in range(1, len(leaves), 2):
+        z = h @ leaves[i].T + leaves[i + 1]
+        if i + 2 < len(leaves):
+            scale = h.detach().abs() @ leaves[i].detach().abs().T
+            near |= (z.detach().abs() < margin * scale).any(1)
+            h = torch.relu(z)
+    dout[near.numpy()] = 0
+    out = torch.cat([z[:, :1], torch.sigmoid(z[:, 1:])], 1)
+    return torch.autograd.grad(out, leaves, torch.from_numpy(dout).double())
+
+
+def _rows_close(got, want, what):
+    err, size = (got - want).abs().amax(-1), want.abs().amax(-1)
+    assert (size > 0).any()
+    assert (err <= BAR * size).all(), (what, float((err / size.clamp(min=1e-300)).max()))
+
+
+def _params(seed):
+    mlp = S.make_mlp(32, 128, 3, seed)
+    return [x.copy() for wb in zip(mlp.weights, mlp.biases) for x in wb]
+
+
+@pytest.mark.parametrize("ratio", [1e-2, 1e-4, 1e-6, 1e-7, 1e-8, 1e-9, 1e-12, 1e-20])
+def test_rows_of_small_samples(device, ratio):
+    """Unit 5 of the first layer, 7 of the second and 9 of the third are active
+    on every fourth sample only, whose gradients are `ratio` of the others'."""
+    M = 64 * 5 + 9
+    rng = np.random.default_rng(21)
+    ps = _params(21)
+    for l, unit, source in ((0, 5, 0), (1, 7, 5), (2, 9, 7)):
+        ps[2 * l][unit], ps[2 * l + 1][unit] = 0, 0
+        ps[2 * l][unit, source] = 1
+    emb = (rng.standard_normal((M, 32)) * 0.1).astype(np.float32)
+    small = np.arange(M) % 4 == 1
+    emb[:, 0] = np.where(small, 0.5, -0.5)
+    dout = rng.standard_normal((M, 4)).astype(np.float32)
+    dout[small] *= np.float32(ratio)
+    want = _grads64(emb, ps, dout)
+    got = _grads(FieldMLP, emb, ps, dout, device)
+    for l, unit in ((0, 5), (1, 7), (2, 9)):
+        _rows_close(got[1 + 2 * l][unit][None], want[1 + 2 * l][unit][None], f"dW_{l} row")
+        _rows_close(got[3 + 2 * l][:, unit][None], want[3 + 2 * l][:, unit][None],
+                    f"dW_{l + 1} column")
+        _rows_close(got[2 + 2 * l][unit].reshape(1, 1), want[2 + 2 * l][unit].reshape(1, 1),
+                    f"db_{l}")
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a - b).abs().max() <= BAR * b.abs().max(), i
+
+
+def test_every_sample_of_another_size(device):
+    """Gradients that fall by a factor of 2 from sample to sample, 2^-62 in a
+    chunk of 64."""
+    M = 64 * 3
+    rng = np.random.default_rng(22)
+    ps = _params(22)
+    emb = (rng.standard_normal((M, 32)) * 0.1).astype(np.float32)
+    dout = (rng.standard_normal((M, 4)) * 2.0 ** -(np.arange(M) % 63)[:, None]).astype(np.float32)
+    want = _grads64(emb, ps, dout)
+    got = _grads(FieldMLP, emb, ps, dout, device)
+    _rows_close(got[0], want[0], "demb")
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a - b).abs().max() <= BAR * b.abs().max(), i
