@@ -118,7 +118,7 @@ struct TrainDims {
   static constexpr int64_t T_BASE = int64_t(F_FRAGS) * 64;
   static constexpr int64_t BIAS_BASE = T_BASE + int64_t(T_FRAGS) * 64;
   // per layer: largest |w|, largest row sum |w|, largest column sum |w|,
-  // largest |b| (L + 1 of each)
+  // largest b (0 at least) (L + 1 of each)
   static constexpr int64_t STATS_BASE = BIAS_BASE + int64_t(L) * H + 4;
   // parameter gradients in torch order: W_0 [H][D], b_0 [H], ..., W_L [4][H], b_L [4]
   static constexpr int64_t P_W0 = 0, P_B0 = int64_t(H) * D;
@@ -1329,8 +1329,9 @@ __global__ __launch_bounds__(256) void split_pack_kernel(SplitLayers s,
     bias[i] = i < hidden + 4 ? s.net.b[s.L][i - hidden] : 0.0f;
 }
 
-// Block l: layer l's largest |w|, row sum |w|, column sum |w| and |b| (not
-// finite where a value is not).
+// Block l: layer l's largest |w|, row sum |w|, column sum |w| and b, the last 0
+// at least (not finite where a value is not; a bias of -inf is a unit switched
+// off).
 template <int D, int H, int L>
 __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
                                                          float* __restrict__ stats) {
@@ -1378,8 +1379,10 @@ __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
 #pragma unroll
   for (int q = 0; q < H / 64; ++q) cols[wave][lane + 64 * q] = mine[q];
   float b = 0.0f;
-  for (int i = threadIdx.x; i < rows; i += 1024)
-    b = __int_as_float(max(__float_as_int(b), __float_as_int(net.b[l][i]) & 0x7FFFFFFF));
+  for (int i = threadIdx.x; i < rows; i += 1024) {
+    const float bi = net.b[l][i];   // one below 0 only lowers its unit
+    b = __int_as_float(max(__float_as_int(b), bi < 0.0f ? 0 : __float_as_int(bi) & 0x7FFFFFFF));
+  }
   up(3, b);
   __syncthreads();
   // the waves' sums in order: the sums choose scales, so their last bits must

@@ -1,6 +1,6 @@
 """The training backward where a tensor's largest entry says nothing: rows of
 the weight gradients that only samples with far smaller gradients than their
-neighbours' reach.
+neighbours' reach, and units with a large negative bias.
 
 Tolerance: the training tests' bar for FP32, 2e-5 of a tensor's largest entry,
 for each row (or column) by itself."""
@@ -88,5 +88,22 @@ def test_every_sample_of_another_size(device):
     want = _grads64(emb, ps, dout)
     got = _grads(FieldMLP, emb, ps, dout, device)
     _rows_close(got[0], want[0], "demb")
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a - b).abs().max() <= BAR * b.abs().max(), i
+
+
+@pytest.mark.parametrize("bias", [-1e3, -1e6, -1e9, -1e20, -np.inf])
+def test_units_switched_off(device, bias):
+    """A large negative bias in each layer switches its unit off and is no bound
+    of what the others give."""
+    M = 150
+    rng = np.random.default_rng(23)
+    ps = _params(23)
+    for l in range(3):
+        ps[2 * l + 1][11 * l + 3] = bias
+    emb = (rng.standard_normal((M, 32)) * 0.1).astype(np.float32)
+    dout = rng.standard_normal((M, 4)).astype(np.float32)
+    want = _grads64(emb, ps, dout)
+    got = _grads(FieldMLP, emb, ps, dout, device)
     for i, (a, b) in enumerate(zip(got, want)):
         assert (a - b).abs().max() <= BAR * b.abs().max(), i
