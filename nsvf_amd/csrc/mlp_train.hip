@@ -513,9 +513,12 @@ typedef __attribute__((ext_vector_type(4))) short s16x4;
 
 struct BwdLds {
   unsigned short x0[2 * kBwdPlane0];         // input: hi plane, lo plane
-  unsigned short t[4][2 * kBwdPlane];        // h0, h1, h2, dz2
+  unsigned short t[4][2 * kBwdPlane];        // h0, h1, h2, dz2 (split BF16: h2 in FP32 before)
   float dl[kBwdChunk][4];                    // logits' gradients (normalised)
-  unsigned short head[2][4][4][4][8];        // head weights hi / lo: [kt][g][logit][i]
+  union {
+    unsigned short head[2][4][4][4][8];      // head weights hi / lo: [kt][g][logit][i]
+    float head32[32][4][4];                  // split BF16: FP32, [k-tile of 4][g][logit]
+  };
   float back[4][kBwdChunk];                  // accumulator -> sum, layers 0..2 and head
   float scale[3][kBwdChunk];                 // sum -> parts, h0, h1, h2
   _Float16 factor[kBwdWaves][kBwdChunk];     // each wave's sample factors of a weight gradient
@@ -791,22 +794,24 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
       ez[k] = tame_exponent(bound);
     }
   }
-  // the head's weights: parts in LDS (operand of the logits), FP32 columns of
-  // this lane's feature (its input gradient)
-  for (int i = threadIdx.x; i < 4 * 4 * 4 * 4; i += kBwdBlock) {
+  // the head's weights in LDS (operand of the logits; packed head fragment mt,
+  // lane (o, c) = W[o][16 mt + c])
+  const float* WT = packed + T::T_BASE + T::T_HEAD * 64;
+  const auto head_weight = [WT](int o, int f) { return WT[(f >> 4) * 64 + o * 16 + (f & 15)]; };
+  for (int i = threadIdx.x; F16 && i < 4 * 4 * 4 * 4; i += kBwdBlock) {
     // pair p of logit o, k-tile kt, group gg: features 32 kt + {4 gg + ..}
     const int p = i & 3, o = (i >> 2) & 3, gg = (i >> 4) & 3, kt = i >> 6;
     const int j = 2 * p, f = 32 * kt + (j < 4 ? 4 * gg + j : 16 + 4 * gg + j - 4);
-    // packed head fragment mt, lane (o, c) = W[o][16 mt + c]
-    const float* WT = packed + T::T_BASE + T::T_HEAD * 64;
-    const float a = WT[(f >> 4) * 64 + o * 16 + (f & 15)];
-    const float b = WT[((f + 1) >> 4) * 64 + o * 16 + ((f + 1) & 15)];
-    const float s = F16 ? f16_scale(ew[3]) : 1.0f;
+    const float s = f16_scale(ew[3]);
     unsigned int hi, lo;
-    parts2<F16>(a, b, s, s, hi, lo);
+    parts2<F16>(head_weight(o, f), head_weight(o, f + 1), s, s, hi, lo);
     *reinterpret_cast<unsigned int*>(&S.head[0][kt][gg][o][j]) = hi;
     *reinterpret_cast<unsigned int*>(&S.head[1][kt][gg][o][j]) = lo;
   }
+  for (int i = threadIdx.x; !F16 && i < 32 * 4 * 4; i += kBwdBlock)
+    // k-tile kt = 4 t + r: feature 16 t + 4 g + r
+    S.head32[i >> 4][(i >> 2) & 3][i & 3] =
+        head_weight(i & 3, 16 * (i >> 6) + 4 * ((i >> 2) & 3) + ((i >> 4) & 3));
   // this lane's biases (feature c of the wave's, logit c of the head) and head
   // weights
   float bl[3], bh;
@@ -947,6 +952,9 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         }
         *reinterpret_cast<u32x2*>(&S.t[l][at_out[m]]) = hi;
         *reinterpret_cast<u32x2*>(&S.t[l][kBwdPlane + at_out[m]]) = lo;
+        if (!F16 && l == 2)
+          *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(S.t[3]) + at_out[m]) =
+              f32x4{h[0], h[1], h[2], h[3]};
         if constexpr (F16) {
           if (l == 0) {
 #pragma unroll
@@ -1001,21 +1009,30 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
     // samples 4 g + r
     if (w < 4) {
       f32x4 z = zero4;
-      if constexpr (!F16) {
-        z = f32x4{bh, bh, bh, bh};
-      }
-      const int at_w = bwd_at(4 * g + (c >> 2), 16 * w + 4 * (c & 3));
-#pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        const unsigned short* p = &S.t[2][at_w + kt * 32 * kBwdRow];
-        const u32x4 ah = lds_tr(p), al = lds_tr(p + kBwdPlane);
-        const u32x4 bh = lds128(S.head[0][kt][g][c & 3]), bl = lds128(S.head[1][kt][g][c & 3]);
-        z = mm16x3<F16>(ah, al, bh, bl, z);
-      }
       if constexpr (F16) {
+        const int at_w = bwd_at(4 * g + (c >> 2), 16 * w + 4 * (c & 3));
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+          const unsigned short* p = &S.t[2][at_w + kt * 32 * kBwdRow];
+          const u32x4 ah = lds_tr(p), al = lds_tr(p + kBwdPlane);
+          const u32x4 bh = lds128(S.head[0][kt][g][c & 3]), bl = lds128(S.head[1][kt][g][c & 3]);
+          z = mm16x3<F16>(ah, al, bh, bl, z);
+        }
         const f32x4 bk = *reinterpret_cast<const f32x4*>(&S.back[3][16 * w + 4 * g]);
 #pragma unroll
         for (int r = 0; r < 4; ++r) z[r] = __fmaf_rn(z[r], bk[r], bh);
+      } else {
+        // in FP32: logits from parts of h2 and the weights put 2-10% on the
+        // error of every gradient against 64 bits (FP32 costs 45 us per million
+        // samples more, of 1,180 forward and backward)
+        const float* h2 = reinterpret_cast<const float*>(S.t[3]);
+#pragma unroll
+        for (int kt = 0; kt < 32; ++kt) {
+          z = mfma4(h2[bwd_at(16 * (kt >> 2) + 4 * g + (kt & 3), 16 * w + c)],
+                    S.head32[kt][g][c & 3], z);
+          if (kt % 8 == 7) tile_fence();
+        }
+        z = z + f32x4{bh, bh, bh, bh};
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {

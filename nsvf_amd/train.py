@@ -448,8 +448,8 @@ class FieldMLPx3(FieldMLP):
     features written as its operand tiles, the weights packed on the device
     each call -- and the backward kernel with the activations'
     recomputation, the input gradients and the parameter gradients in split
-    BF16 too (the head's input gradient in FP32), deterministic like
-    FieldMLP's."""
+    BF16 too (the head's recomputed logits and their input gradient in
+    FP32), deterministic like FieldMLP's."""
 
     @staticmethod
     def forward(ctx, emb, *params):
@@ -505,7 +505,8 @@ class TrainableField(nn.Module):
     mlp="hip": the MLP runs forward and backward on the hand-written FP32
     kernels (FieldMLP; built for D=32, H=128, L=3 -- other shapes raise);
     mlp="hip_x3": forward and backward in split BF16 (FieldMLPx3: outputs
-    within about 1e-5 of FP32, gradients about as close);
+    within about 1e-5 of FP32, gradients about as close; the backward's head
+    -- recomputed logits and their input gradient -- in FP32);
     mlp="torch": torch.nn.functional.linear with torch autograd, as in the
     reference."""
 

@@ -1,6 +1,7 @@
 """The training backward where a tensor's largest entry says nothing: rows of
 the weight gradients that only samples with far smaller gradients than their
-neighbours' reach, and units with a large negative bias.
+neighbours' reach, units with a large negative bias, and the split-BF16
+backward's logits.
 
 Tolerance: the training tests' bar for FP32, 2e-5 of a tensor's largest entry,
 for each row (or column) by itself."""
@@ -9,7 +10,7 @@ import pytest
 import torch
 
 from nsvf_amd import scene as S
-from nsvf_amd.train import FieldMLP
+from nsvf_amd.train import FieldMLP, FieldMLPx3
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +108,33 @@ def test_units_switched_off(device, bias):
     got = _grads(FieldMLP, emb, ps, dout, device)
     for i, (a, b) in enumerate(zip(got, want)):
         assert (a - b).abs().max() <= BAR * b.abs().max(), i
+
+
+def test_split_bf16_backward_logits(device):
+    """Two head weights of opposite sign on two outputs that agree in their
+    first 16 bits: the logit is a difference that FP32 holds exactly and a pair
+    of BF16 parts does not hold at all.  Every other product is of whole
+    numbers within 24 bits, so the gradients have FP32's error."""
+    M = 200
+    rng = np.random.default_rng(25)
+    emb = np.zeros((M, 32), np.float32)
+    emb[:, :5] = rng.integers(1, 256, (M, 5))
+    w = [np.zeros(s, np.float32) for s in ((128, 32), (128, 128), (128, 128), (4, 128))]
+    b = [np.zeros(s, np.float32) for s in (128, 128, 128, 4)]
+    w[0][range(5), range(5)] = 1
+    w[1][0, 0], w[1][0, 1] = 256, 1          # 16 bits
+    w[1][1, 2], w[1][1, 3] = 256, 1
+    w[1][2, 4] = 1
+    w[2][0, 0], w[2][0, 1] = 128, 1          # 23 bits, nearly equal
+    w[2][1, 0], w[2][1, 2] = 128, 1
+    w[3][0, 0] = 2.0 ** -20
+    w[3][1:, 0], w[3][1:, 1] = 2.0 ** -15, -2.0 ** -15
+    ps = [x for wb in zip(w, b) for x in wb]
+    dout = rng.standard_normal((M, 4)).astype(np.float32)
+    want = _grads64(emb, ps, dout, margin=0.0)
+    got = _grads(FieldMLPx3, emb, ps, dout, device)
+    assert ((got[8] - want[8]).abs() <= BAR * want[8].abs().max()).all()
+    # the gradients behind the head are split BF16: 2^-16 of a product's parts
+    # each, three layers
+    for i, (x, y) in enumerate(zip(got, want)):
+        assert (x - y).abs().max() <= 2e-4 * y.abs().max(), i
