@@ -507,12 +507,13 @@ int nsvf_field_eval(int precision, int D, int H, int L, const float* centers,
                     const float* bias, float* out, void* workspace,
                     int64_t workspace_bytes, void* stream);
 
-/* nsvf_field_eval at precision 1 on the FP32 matrix units for every shape, in
- * the order of FP32 sums that this library has always had.  Both kernels are
- * within FP32 rounding of the exact field, but where samples are placed by
- * probabilities computed from the field (hierarchical views), a last bit can
- * move a ray's last step across the end of its bins and change the sample
- * list, so those views keep the one order.                                  */
+/* nsvf_field_eval at precision 1 on the FP32 matrix units for every shape: the
+ * embedding's corners added in corner order, each product and sum rounded, and
+ * the MLP's sums on the FP32 units.  Both kernels are within FP32 rounding of
+ * the exact field, but where a decision is taken from the field's last bits
+ * (hierarchical views place their fine samples by probabilities computed from
+ * it, early termination ends a ray by it), another rounding changes the sample
+ * list, so those views keep this one.                                       */
 int nsvf_field_eval_f32(int D, int H, int L, const float* centers,
                         const int32_t* feats, const float* values,
                         float voxel_size, const float* ray_start,

@@ -55,25 +55,29 @@ struct FieldRays {
   const float* dir;    // [R,3]
 };
 
-// Trilinear weights of a point x in voxel v (corner order 4x + 2y + z).
+// Trilinear weights of a point x in voxel v (corner order 4x + 2y + z); the
+// division by the voxel size is an exact multiplication where the size is a
+// power of two.
 __device__ __forceinline__ void corner_weights(const FieldScene& sc, int32_t v, const float x[3],
                                                float w[8], int32_t key[8]) {
   float p[3];
 #pragma unroll
-  for (int a = 0; a < 3; ++a) p[a] = (x[a] - sc.centers[int64_t(v) * 3 + a]) / sc.voxel_size + 0.5f;
+  for (int a = 0; a < 3; ++a) {
+    const float d = x[a] - sc.centers[int64_t(v) * 3 + a];
+    p[a] = (sc.voxel_pow2 ? d * sc.inv_voxel : d / sc.voxel_size) + 0.5f;
+  }
   const float q[3] = {1.0f - p[0], 1.0f - p[1], 1.0f - p[2]};
+  const float xy[4] = {q[0] * q[1], q[0] * p[1], p[0] * q[1], p[0] * p[1]};
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
-    const float wx = (c & 4) ? p[0] : q[0];
-    const float wy = (c & 2) ? p[1] : q[1];
-    const float wz = (c & 1) ? p[2] : q[2];
-    w[c] = (wx * wy) * wz;
+    w[c] = xy[c >> 1] * ((c & 1) ? p[2] : q[2]);
     key[c] = sc.feats[int64_t(v) * 8 + c];
   }
 }
 
 // The 8 features {32kt + 4g + 0..3, 32kt + 16 + 4g + 0..3} of one sample's
-// embedding (zero past D).
+// embedding (zero past D), each product and sum rounded: the order of the
+// plain evaluation, for the kernels whose last bits place samples.
 template <int D>
 __device__ __forceinline__ void gather8(const FieldScene& sc, const float w[8],
                                         const int32_t key[8], int kt, int g, float out[8]) {
@@ -95,28 +99,8 @@ __device__ __forceinline__ void gather8(const FieldScene& sc, const float w[8],
   }
 }
 
-// Corner weights for the BF16 field kernel: the same formula, with the
-// division by the voxel size done as an exact multiply when the size is a
-// power of two.
-__device__ __forceinline__ void corner_weights_fast(const FieldScene& sc, int32_t v,
-                                                    const float x[3], float w[8],
-                                                    int32_t key[8]) {
-  float p[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const float d = x[a] - sc.centers[int64_t(v) * 3 + a];
-    p[a] = (sc.voxel_pow2 ? d * sc.inv_voxel : d / sc.voxel_size) + 0.5f;
-  }
-  const float q[3] = {1.0f - p[0], 1.0f - p[1], 1.0f - p[2]};
-  const float xy[4] = {q[0] * q[1], q[0] * p[1], p[0] * q[1], p[0] * p[1]};
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    w[c] = xy[c >> 1] * ((c & 1) ? p[2] : q[2]);
-    key[c] = sc.feats[int64_t(v) * 8 + c];
-  }
-}
-
-// gather8 with fused multiply-adds (the BF16 path rounds to bf16 afterwards).
+// gather8 with fused multiply-adds (half the instructions, one rounding less
+// per corner).
 template <int D>
 __device__ __forceinline__ void gather8_fma(const FieldScene& sc, const float w[8],
                                             const int32_t key[8], int kt, int g, float out[8]) {
@@ -206,7 +190,6 @@ struct StreamSource {
   FieldRays rays;
   const SampleRec* samples;
   const int32_t* list;
-  template <bool kFast>
   __device__ __forceinline__ bool weights(int64_t s, float w[8], int32_t key[8]) const {
     const SampleRec rec = samples[list ? list[s] : s];
     if (rec.idx < 0) return false;  // an unused slot of a ray's range
@@ -214,10 +197,7 @@ struct StreamSource {
 #pragma unroll
     for (int a = 0; a < 3; ++a)
       x[a] = rays.start[int64_t(rec.ray) * 3 + a] + rays.dir[int64_t(rec.ray) * 3 + a] * rec.depth;
-    if (kFast)
-      corner_weights_fast(sc, rec.idx, x, w, key);
-    else
-      corner_weights(sc, rec.idx, x, w, key);
+    corner_weights(sc, rec.idx, x, w, key);
     return true;
   }
 };
@@ -231,7 +211,6 @@ struct LatticeSource {
   int64_t voxel0;
   int bits;
   float half_voxel;
-  template <bool kFast>
   __device__ __forceinline__ bool weights(int64_t s, float w[8], int32_t key[8]) const {
     const int64_t per = int64_t(bits) * bits * bits;
     const int64_t v = voxel0 + s / per;
@@ -243,10 +222,7 @@ struct LatticeSource {
       const float off = float(2 * ijk[a] + 1 - bits) / float(bits - 1);
       x[a] = sc.centers[v * 3 + a] + off * half_voxel;
     }
-    if (kFast)
-      corner_weights_fast(sc, int32_t(v), x, w, key);
-    else
-      corner_weights(sc, int32_t(v), x, w, key);
+    corner_weights(sc, int32_t(v), x, w, key);
     return true;
   }
 };
@@ -254,7 +230,7 @@ struct LatticeSource {
 // The sources as the FP16-split kernel reads them, a wave's 32-sample tiles
 // one after another: next(base, M) starts on the tile at `base` (its loads are
 // in flight until weights() needs them), then weights(j, w, key) gives its
-// samples 16 j + lane % 16, as Source::weights<true> does.
+// samples 16 j + lane % 16, as Source::weights does.
 template <class Src>
 struct TileReader;
 
@@ -279,7 +255,7 @@ struct TileReader<StreamSource> {
     for (int a = 0; a < 3; ++a)
       x[a] = src.rays.start[int64_t(rec[j].ray) * 3 + a] +
              src.rays.dir[int64_t(rec[j].ray) * 3 + a] * rec[j].depth;
-    corner_weights_fast(src.sc, rec[j].idx, x, w, key);
+    corner_weights(src.sc, rec[j].idx, x, w, key);
     return true;
   }
 };
@@ -316,7 +292,7 @@ struct TileReader<LatticeSource> {
 #pragma unroll
     for (int a = 0; a < 3; ++a)
       x[a] = src.sc.centers[v * 3 + a] + __shfl(plane, int(ijk[a]), 64);
-    corner_weights_fast(src.sc, int32_t(v), x, w, key);
+    corner_weights(src.sc, int32_t(v), x, w, key);
     return t < left;
   }
 };
@@ -593,7 +569,7 @@ __global__ __launch_bounds__(kFieldBlock) void field_bf16_kernel(
       const int64_t s = base + 16 * j + col;
       float w[8];
       int32_t key[8];
-      const bool valid = s < M && src.template weights<true>(s, w, key);
+      const bool valid = s < M && src.weights(s, w, key);
 #pragma unroll
       for (int kt = 0; kt < Dm::KT0; ++kt) {
         float f[8];
@@ -720,7 +696,7 @@ __global__ __launch_bounds__(256) void embed_bf16_kernel(FieldScene sc, FieldRay
     }
     if (!have_w) {
       // corner weights: x = o + d * z, p = (x - c) / vs + 0.5 (the fused
-      // kernel's corner_weights_fast arithmetic)
+      // corner_weights' arithmetic)
       float p[3];
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
@@ -1416,7 +1392,8 @@ __global__ __launch_bounds__(64 * kFusedWaves, 1) void field_fused_kernel(
 // 16 t + 4 g + i.
 constexpr int kF32NT = 2;
 
-template <int D, class Weights>
+// kFused: with gather8_fma (kernels that do not keep FP32's order of sums).
+template <int D, bool kFused, class Weights>
 __device__ __forceinline__ void gather_f32_tile(const FieldScene& sc, int g,
                                                 float (&x)[kF32NT][4 * ((D + 15) / 16)],
                                                 Weights weights) {
@@ -1430,7 +1407,10 @@ __device__ __forceinline__ void gather_f32_tile(const FieldScene& sc, int g,
     for (int kt32 = 0; kt32 < (KT0 + 7) / 8; ++kt32) {
       float f[8];
       if (valid) {
-        gather8_fma<D>(sc, w, key, kt32, g, f);
+        if constexpr (kFused)
+          gather8_fma<D>(sc, w, key, kt32, g, f);
+        else
+          gather8<D>(sc, w, key, kt32, g, f);
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) f[i] = 0.0f;
@@ -1550,9 +1530,9 @@ __global__ __launch_bounds__(kFieldBlock) void field_f32_kernel(
     const int64_t base = t * 16 * kF32NT;
     sink.begin_tile(base, M, 16 * kF32NT);
     float x[kF32NT][4 * ((D + 15) / 16)];
-    gather_f32_tile<D>(src.sc, g, x, [&](int j, float w[8], int32_t key[8]) {
+    gather_f32_tile<D, false>(src.sc, g, x, [&](int j, float w[8], int32_t key[8]) {
       const int64_t s = base + 16 * j + col;
-      return s < M && src.template weights<true>(s, w, key);
+      return s < M && src.weights(s, w, key);
     });
     f32x4 out[kF32NT];
     mlp_f32_tile<D, H, L>(x, wfrag, bias, lane, g, out);
@@ -1590,12 +1570,10 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void field_f16x3_kernel(
     const int64_t base = t * kF16Samples;
     sink.begin_tile(base, M, kF16Samples);
     float x[kF32NT][D / 4];
-    const auto gather = [&] {
-      gather_f32_tile<D>(src.sc, g, x, [&](int j, float w[8], int32_t key[8]) {
-        return reader.weights(j, w, key);
-      });
+    const auto weights = [&](int j, float w[8], int32_t key[8]) {
+      return reader.weights(j, w, key);
     };
-    gather();
+    gather_f32_tile<D, true>(src.sc, g, x, weights);
     f32x4 out[kF32NT];
     const bool done = mlp.tile(x, lane, g, out, [&](int l) {
       if (l == 1 && t + 1 < last) reader.next(base + kF16Samples, M);
@@ -1606,7 +1584,7 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void field_f16x3_kernel(
       const float* wf = wfrag;
       asm volatile("" : "+s"(wf));
       reader.next(base, M);
-      gather();
+      gather_f32_tile<D, false>(src.sc, g, x, weights);
       mlp_f32_tile<D, H, L>(x, wf, bias, lane, g, out);
       if (t + 1 < last) reader.next(base + kF16Samples, M);
     }
