@@ -361,11 +361,13 @@ class Renderer:
     def _field(self, sc, ray_start, ray_dir, samples, m_dev, m, out, slots=None):
         """Field of the m_dev samples of a stream (slots: optional evaluation
         list of stream slots; then only those slots of out are written).
-        FP32 hierarchical views stay on the FP32 matrix units: the coarse
-        pass places the fine samples, and its last bits decide on which side
-        of its bins' end a ray's last step falls (one ray of the shell's 64 x
-        64 view moves by 6.5e-3 in colour otherwise); the fine pass takes
-        fields from the coarse one, so both are of one kind."""
+        FP32 views that take decisions from the field's last bits stay on the
+        FP32 matrix units.  Hierarchical ones: the coarse pass places the fine
+        samples, and its last bits decide on which side of its bins' end a
+        ray's last step falls (one ray of the shell's 64 x 64 view moves by
+        6.5e-3 in colour otherwise); the fine pass takes fields from the
+        coarse one, so both are of one kind.  Early termination: a ray stops
+        where its sum passes the threshold."""
         L = lib()
         prec = PRECISIONS[self.precision]
         w = sc.mlp[_WEIGHTS[prec]]
@@ -413,7 +415,7 @@ class Renderer:
         args = (sc.D, sc.H, sc.L, _p(sc.centers), _p(sc.feats), _p(sc.values), sc.voxel_size,
                 _p(ray_start), _p(ray_dir), _p(samples), _p(slots), _p(m_dev), m, _p(w),
                 _p(sc.mlp["bias"]), _p(out))
-        if prec == 1 and self.hierarchical:
+        if prec == 1 and (self.hierarchical or self.tolerance > 0):
             check(L.nsvf_field_eval_f32(*args, st), "field_eval_f32")
         else:
             check(L.nsvf_field_eval(prec, *args, None, 0, st), "field_eval")
