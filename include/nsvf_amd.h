@@ -693,10 +693,14 @@ int nsvf_march_end(const int32_t* hit_list, int64_t n_hit, const int32_t* off,
  * ReLU layers of width H over D inputs, a 4-wide head; output (sigma,
  * sigmoid(r, g, b)), which the reference differentiates with torch
  * autograd), forward and backward at FP32 accuracy: FP16 hi / lo parts of
- * scaled FP32 operands, or the FP32 MFMAs for the tiles (forward) and calls
- * (backward) with a value that is not finite or, in the backward, a weight or
- * a sample's largest feature outside 2^-40 .. 2^60.  Built for D=32, H=128,
- * L=3 (nsvf_mlp_train_supported); other shapes return NSVF_EINVAL and the
+ * scaled FP32 operands (22 significant bits, and an absolute error of 2^-39
+ * of the layer's largest weight and of the sample's largest activation: what
+ * is further below them has fewer bits), or the FP32 MFMAs for the tiles of 32
+ * (forward) and chunks of 64 samples (backward) with a value that is not
+ * finite or, in the backward, a sample's largest feature outside 2^-40 ..
+ * 2^60 or a gradient above 2^60, and for all where a weight is.  Built for
+ * D=32, H=128, L=3 (nsvf_mlp_train_supported); other shapes return
+ * NSVF_EINVAL and the
  * size queries -1.
  * Parameters in torch layout: weights[l] [out][in] and biases[l] [out] for
  * l = 0..L (device pointers, host arrays of L + 1).  nsvf_mlp_train_pack

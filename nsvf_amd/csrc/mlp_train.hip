@@ -49,6 +49,8 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int kTrainWaves = 8;
 constexpr int kTrainBlock = 64 * kTrainWaves;
 constexpr int kTrainChunk = 16 * kTrainWaves;  // samples per block step
+constexpr int kBwdChunk = 64;                  // of the 16-bit backward kernel
+static_assert(kTrainChunk == 2 * kBwdChunk, "the FP32 kernel's steps are two of its chunks");
 constexpr int kLdsRow = 144;  // floats per LDS row: 144 = 16 mod 64 banks
 constexpr int kMaxTrainBlocks = 256;
 
@@ -272,13 +274,14 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void mlp_train_forward_kernel(
 // Backward: demb [M][D] and this block's partial parameter gradients
 // (partial + blockIdx.x * PARAMS, torch order), from dout [M][4] = the
 // gradient of (sigma, r, g, b) after the sigmoid.  Needs H == 16 * waves.
-// On the FP32 MFMAs: runs where one of the nflags flags is set, the whole
-// call again (grids differ: the sum over partials looks at the same flags).
+// On the FP32 MFMAs, for the chunks of 64 samples that the 16-bit kernel left
+// (chunk_flags): returns at once where none of the nflags blocks' flags is set
+// (the sum over partials looks at the same flags).
 template <int D, int H, int L>
 __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
     const float* __restrict__ emb, int64_t M, const float* __restrict__ packed,
     const float* __restrict__ dout, float* __restrict__ demb, float* __restrict__ partial,
-    const int32_t* __restrict__ flags, int nflags) {
+    const int32_t* __restrict__ flags, int nflags, const int32_t* __restrict__ chunk_flags) {
   using T = TrainDims<D, H, L>;
   static_assert(T::MT == kTrainWaves, "one hidden m-tile per wave");
   static_assert(D % 16 == 0 && D <= H, "input width");
@@ -309,17 +312,23 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
   if (!__syncthreads_or(flagged)) return;
   const int64_t chunks = (M + kTrainChunk - 1) / kTrainChunk;
   for (int64_t ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
+    const int64_t half = ch * kTrainChunk + kBwdChunk;   // the second chunk's first sample
+    const bool first = chunk_flags[2 * ch] != 0;
+    const bool second = half < M && chunk_flags[2 * ch + 1] != 0;
+    if (!first && !second) continue;
+    // the samples below `end` are this wave's to do: none of a chunk done before
+    const int64_t end = (w < kTrainWaves / 2 ? first : second) ? M : 0;
     const int64_t s = ch * kTrainChunk + w * 16 + col;
     const float* pk = opaque(packed);
     const float* At = pk + T::T_BASE;
     float x0[T::KT0];
     float h[L][T::KTH];
     f32x4 z;
-    forward_tile<D, H, L>(emb, M, pk, s, x0, h, z, lane, g);
+    forward_tile<D, H, L>(emb, end, pk, s, x0, h, z, lane, g);
     // dlogits on the lanes of group 0: d sigma as given, d rgb through the
     // sigmoid's derivative y (1 - y)
     f32x4 dl = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (g == 0 && s < M) {
+    if (g == 0 && s < end) {
       const float4 d = *reinterpret_cast<const float4*>(dout + s * 4);
       const float4 bb = *reinterpret_cast<const float4*>(bias + L * H);
       const float y1 = logistic(z[1] + bb.y), y2 = logistic(z[2] + bb.z),
@@ -417,7 +426,7 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 #pragma unroll
         for (int mt = 0; mt < T::MT0; ++mt) {
           const f32x4 acc = mfma_chain<T::KTH>(At + mt * T::KTH * 64, dz, lane);
-          if (s < M) *reinterpret_cast<f32x4*>(demb + s * D + 16 * mt + 4 * g) = acc;
+          if (s < end) *reinterpret_cast<f32x4*>(demb + s * D + 16 * mt + 4 * g) = acc;
           tile_fence();
         }
       }
@@ -491,8 +500,11 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 // every second chunk's weight gradient, is computed with the other sign.  (With
 // one sign the bias gradients were 3e-6 off on a million samples, FP32 MFMAs
 // 1e-6.)
-// An operand that is not finite or outside 2^-40 .. 2^60 raises the block's
-// flag, and the FP32 kernel below then computes the whole call.
+// A chunk with an operand that is not finite or outside 2^-40 .. 2^60 is found
+// out before its weight gradients and left to the FP32 kernel above, which adds
+// partial sums of its own (all chunks, if it is a weight).  Repeating the whole
+// call there, a million samples with one such sample took 4,376 us where all on
+// the FP32 MFMAs had taken 3,975.
 //
 // Bound: LDS reads (about 15 k cycles per 64 samples at 128 B per cycle)
 // beside 12.5 k of MFMAs, and the phases' barriers.
@@ -503,7 +515,6 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 // before.
 constexpr int kBwdWaves = 8;
 constexpr int kBwdBlock = 64 * kBwdWaves;
-constexpr int kBwdChunk = 64;                // samples per block step
 constexpr int kBwdRow = 72;                  // halves per plane row
 constexpr int kBwdPlane = 128 * kBwdRow;     // halves per hidden plane
 constexpr int kBwdPlane0 = 32 * kBwdRow;     // halves per input plane
@@ -762,7 +773,8 @@ template <int D, int H, int L, bool F16>
 __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
     const float* __restrict__ emb, int64_t M, const float* __restrict__ packed,
     const u32x4* __restrict__ frags, const float* __restrict__ dout, float* __restrict__ demb,
-    float* __restrict__ partial, int32_t* __restrict__ flags) {
+    float* __restrict__ partial, int32_t* __restrict__ flags,
+    int32_t* __restrict__ chunk_flags) {
   using T = TrainDims<D, H, L>;
   static_assert(D == 32 && H == 128 && L == 3, "the phases below");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -775,13 +787,13 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
   [[maybe_unused]] int ew[4] = {0, 0, 0, 0};
   [[maybe_unused]] float rowsum[4], maxb[4];
   [[maybe_unused]] int ez[3] = {0, 0, 0};   // exponents of dz2, dz1, dz0
-  bool wild = false;
+  bool wild_weights = false;
   if constexpr (F16) {
     const float* st = packed + T::STATS_BASE;
     float bound = 2.0f;   // of the normalised logits' gradients
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
-      wild = wild || !tame(st[l]) || !tame(st[4 + l]) || !tame(st[8 + l]) ||
+      wild_weights = wild_weights || !tame(st[l]) || !tame(st[4 + l]) || !tame(st[8 + l]) ||
              !(st[12 + l] <= 0x1p60f);
       ew[l] = tame_exponent(st[l]);
       rowsum[l] = st[4 + l];
@@ -790,7 +802,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
 #pragma unroll
     for (int k = 0; k < 3; ++k) {   // dz2 through the head, dz1 through W_2, dz0 through W_1
       bound = bound * st[8 + 3 - k];
-      wild = wild || !tame(bound);
+      wild_weights = wild_weights || !tame(bound);
       ez[k] = tame_exponent(bound);
     }
   }
@@ -822,7 +834,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
 #pragma unroll
   for (int o = 0; o < 4; ++o)
     wh[o] = packed[T::T_BASE + (T::T_HEAD + w) * 64 + o * 16 + c];
-  if (threadIdx.x == 0) S.wild = 0;
+  bool flagged = F16 && wild_weights;   // a chunk was left to the FP32 kernel
   for (int i = threadIdx.x; i < kBwdChunk; i += kBwdBlock) S.top0[i] = 0;
 
   const f32x4 zero4 = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -846,7 +858,12 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
   load_x(blockIdx.x);
   __syncthreads();
 
-  for (int64_t ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
+  // weights beyond the window leave every chunk
+  for (int64_t ch = blockIdx.x + int64_t(threadIdx.x) * gridDim.x; flagged && ch < chunks;
+       ch += int64_t(gridDim.x) * kBwdBlock)
+    chunk_flags[ch] = 1;
+  for (int64_t ch = flagged ? chunks : blockIdx.x; ch < chunks; ch += gridDim.x) {
+    [[maybe_unused]] bool wild = false;
     const int64_t s0 = ch * kBwdChunk;
     const float sign = (ch / gridDim.x) & 1 ? -1.0f : 1.0f;   // of the chunk's weight gradients
     // the lane index as a value of this step: the addresses formed from it
@@ -921,6 +938,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
     }
     BwdFrags<4> f;
     __syncthreads();
+    if (threadIdx.x == 0) S.wild = 0;   // read by all before, set at the head
 
     // relu(z) of an accumulator into plane set l, the mask bits, and (F16) the
     // samples' largest value for layer 0
@@ -1007,6 +1025,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
 
     // ---- the head: wave m takes samples 16 m..; lanes c < 4 hold logit c of
     // samples 4 g + r
+    [[maybe_unused]] float hb = 0.0f;   // of the chunk
     if (w < 4) {
       f32x4 z = zero4;
       if constexpr (F16) {
@@ -1040,7 +1059,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         const float d = dy[r];
         const float y = logistic(z[r]);
         float v = (c & 3) == 0 ? d : d * (y * (1.0f - y));
-        if (c < 4) ghb += v;
+        if (c < 4) (F16 ? hb : ghb) += v;
         if constexpr (F16) {
           int m = __float_as_int(v) & 0x7FFFFFFF;
           m = max(m, __builtin_amdgcn_mov_dpp(m, 0xB1, 0xF, 0xF, true));
@@ -1055,7 +1074,21 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         if (c < 4) S.dl[i][c] = v;
       }
     }
+    if constexpr (F16) {
+      if (wild) S.wild = 1;
+    }
     __syncthreads();
+    if constexpr (F16) {
+      // the chunk to the FP32 kernel; nothing of it is in the sums yet
+      const bool skip = __builtin_amdgcn_readfirstlane(S.wild) != 0;
+      if (threadIdx.x == 0) chunk_flags[ch] = skip;
+      if (skip) {
+        flagged = true;
+        if (threadIdx.x < kBwdChunk) S.top0[threadIdx.x] = 0;
+        continue;
+      }
+      ghb += hb;
+    }
 
     // a layer's weight gradient (k = 0 .. 2) or the head's (3): the samples'
     // exponents are those of the normalised gradient times the layer's input
@@ -1226,7 +1259,6 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
   }
 
   // ---- the block's partial sums, in torch order
-  if (wild) S.wild = 1;
   float* P = partial + int64_t(blockIdx.x) * T::PARAMS;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -1259,12 +1291,13 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
   if (threadIdx.x < 4)
     P[T::P_HEAD + 4 * H + threadIdx.x] =
         ((S.dl[0][threadIdx.x] + S.dl[1][threadIdx.x]) + S.dl[2][threadIdx.x]) + S.dl[3][threadIdx.x];
-  if (F16 && threadIdx.x == 0) flags[blockIdx.x] = S.wild;
+  if (F16 && threadIdx.x == 0) flags[blockIdx.x] = flagged;
 }
 
 // dparams[p] = the sum over blocks of partial[b][p], in a fixed order: lane
 // group j of a block's 16 adds blocks j, j + 16, ..., four loads in flight, and
-// the 16 sums are added in order.  nb16 partials, or nb32 where a flag is set.
+// the 16 sums are added in order.  nb16 partials, then nb32 more where one of
+// the nb16 flags is set.
 // A thread per parameter waited for nb loads one by one: 61 us for 256
 // partials, now 16.
 constexpr int kSumCols = 16;   // parameters per block
@@ -1276,7 +1309,7 @@ __global__ __launch_bounds__(256) void sum_partials_kernel(const float* __restri
   int flagged = 0;
   if (flags)
     for (int i = threadIdx.x; i < nb16; i += 256) flagged |= flags[i];
-  const int nb = __syncthreads_or(flagged) ? nb32 : nb16;
+  const int nb = nb16 + (__syncthreads_or(flagged) ? nb32 : 0);
   const int j = threadIdx.x / kSumCols, q = threadIdx.x % kSumCols;
   const int64_t p = int64_t(blockIdx.x) * kSumCols + q;
   float acc = 0.0f;
@@ -1557,9 +1590,12 @@ int64_t nsvf_mlp_train_param_floats(int D, int H, int L) {
 
 int64_t nsvf_mlp_train_partial_floats(int D, int H, int L, int64_t M) {
   if (!train_shape_ok(D, H, L) || M < 0) return -1;
-  // the blocks' partial sums, then their flags
+  // the partial sums of the 16-bit kernel's blocks and of the FP32 one's, the
+  // first's flags and the chunks'
   const int64_t nb = backward_blocks(M, kBwdChunk);
-  return nb * TrainDims<32, 128, 3>::PARAMS + (M > 0 ? nb : 0);
+  constexpr int64_t P = TrainDims<32, 128, 3>::PARAMS;
+  return M == 0 ? nb * P
+                : (nb + backward_blocks(M, kTrainChunk)) * P + nb + ceil_div(M, kBwdChunk);
 }
 
 int nsvf_mlp_split_pack(int D, int H, int L, const float* const* weights,
@@ -1646,21 +1682,24 @@ static int train_backward(const char* name, int D, int H, int L, const float* pa
                      static_cast<long long>(partial_floats), static_cast<long long>(need));
   hipStream_t st = as_stream(stream);
   const int nb = backward_blocks(M, kBwdChunk), nb32 = backward_blocks(M, kTrainChunk);
+  float* partial32 = partial + int64_t(nb) * T::PARAMS;
   int32_t* flags = x3w || M == 0 ? nullptr
-                                 : reinterpret_cast<int32_t*>(partial + int64_t(nb) * T::PARAMS);
+                                 : reinterpret_cast<int32_t*>(partial32 + int64_t(nb32) * T::PARAMS);
   if (x3w || M == 0) {
     hipLaunchKernelGGL((mlp_train_backward_kernel<32, 128, 3, false>), dim3(nb), dim3(kBwdBlock),
                        sizeof(BwdLds), st, emb, M, packed, reinterpret_cast<const u32x4*>(x3w),
-                       dout, demb, partial, flags);
+                       dout, demb, partial, flags, nullptr);
     if (check_launch(name) != NSVF_OK) return NSVF_ELAUNCH;
   } else {
+    int32_t* chunk_flags = flags + nb;
     hipLaunchKernelGGL((mlp_train_backward_kernel<32, 128, 3, true>), dim3(nb), dim3(kBwdBlock),
                        sizeof(BwdLds), st, emb, M, packed,
                        reinterpret_cast<const u32x4*>(packed + T::F16_BASE), dout, demb, partial,
-                       flags);
+                       flags, chunk_flags);
     if (check_launch(name) != NSVF_OK) return NSVF_ELAUNCH;
     hipLaunchKernelGGL((mlp_train_backward_f32_kernel<32, 128, 3>), dim3(nb32), dim3(kTrainBlock),
-                       kBackwardLds, st, emb, M, packed, dout, demb, partial, flags, nb);
+                       kBackwardLds, st, emb, M, packed, dout, demb, partial32, flags, nb,
+                       chunk_flags);
     if (check_launch(name) != NSVF_OK) return NSVF_ELAUNCH;
   }
   hipLaunchKernelGGL(sum_partials_kernel, dim3(unsigned(ceil_div(T::PARAMS, kSumCols))), dim3(256),

@@ -138,3 +138,27 @@ def test_split_bf16_backward_logits(device):
     # each, three layers
     for i, (x, y) in enumerate(zip(got, want)):
         assert (x - y).abs().max() <= 2e-4 * y.abs().max(), i
+
+
+@pytest.mark.parametrize("wild", [(0,), (63,), (64,), (127, 128), (70, 400), (588,), "all"])
+def test_chunks_beyond_the_window(device, wild):
+    """Samples whose largest feature is below 2^-40 send their chunk of 64 to
+    the FP32 MFMAs, and no other: the others' input gradients keep their bits."""
+    M = 64 * 9 + 13
+    wild = list(range(0, M, 64)) if wild == "all" else list(wild)
+    rng = np.random.default_rng(26)
+    ps = _params(26)
+    emb = (rng.standard_normal((M, 32)) * 0.1).astype(np.float32)
+    emb[wild] = 0
+    dout = rng.standard_normal((M, 4)).astype(np.float32)
+    want = _grads64(emb, ps, dout)
+    tame = _grads(FieldMLP, emb, ps, dout, device)
+    emb[wild] = (rng.standard_normal((len(wild), 32)) * 1e-14).astype(np.float32)
+    got = _grads(FieldMLP, emb, ps, dout, device)
+    there = np.isin(np.arange(M) // 64, np.array(wild) // 64)
+    assert torch.equal(got[0][~there], tame[0][~there])
+    assert not torch.equal(got[0][there], tame[0][there])
+    for i, (a, b) in enumerate(zip(got, want)):   # 1e-14 moves nothing by 2e-5
+        assert (a - b).abs().max() <= BAR * b.abs().max(), i
+    again = _grads(FieldMLP, emb, ps, dout, device)
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
