@@ -80,8 +80,9 @@ int nsvf_svo_intersect(const float* ray_start, const float* ray_dir,
  * that each node's octant holds the leaves below it, as in every tree of
  * nsvf_build_octree, and the traversal then prunes with the octants instead
  * of the reference's boxes of twice their size: the same outputs, in about
- * half the time.  A tree that does not pass, or a tree per ray batch, is
- * traversed as by nsvf_svo_intersect.                                      */
+ * half the time.  A tree that does not pass, a tree per ray batch, or a large
+ * one for a few rays that seem to miss it is traversed as by
+ * nsvf_svo_intersect.                                                      */
 int64_t nsvf_svo_workspace_bytes(void);
 int nsvf_svo_intersect_ws(const float* ray_start, const float* ray_dir,
                           const float* points, const int32_t* children, int B,
