@@ -27,6 +27,10 @@ __device__ __forceinline__ bool ray_voxel(const float o[3], const float inv[3], 
   return ray_box(o, inv, mn, mx, lo, hi);
 }
 
+// Threads of one launch, at most: HIP takes fewer than 2^32, which batches of
+// a ray each (a block of 1,024 threads) or 2^29 octree rays would pass.
+constexpr int64_t kLaunchThreads = int64_t(1) << 31;
+
 constexpr int kAabbWaves = 16;
 constexpr int kAabbBlock = 64 * kAabbWaves;
 constexpr int kAabbTiles = 1024;   // 64-voxel tiles whose boxes a block holds at once
@@ -89,13 +93,13 @@ __device__ __forceinline__ bool ray_may_hit(const float o[3], const float inv[3]
 __global__ __launch_bounds__(kAabbBlock) void aabb_intersect_kernel(
     const float* __restrict__ ray_start, const float* __restrict__ ray_dir,
     const float* __restrict__ points, int M, int N, int64_t points_bstride,
-    int blocks_per_batch, int rays_per_block, float half_voxel, int n_max,
+    int first_block, int blocks_per_batch, int rays_per_block, float half_voxel, int n_max,
     int32_t* __restrict__ idx, float* __restrict__ min_depth,
     float* __restrict__ max_depth) {
   __shared__ float box[6][kAabbTiles];
   __shared__ int32_t counts[kAabbRays];
-  const int b = blockIdx.x / blocks_per_batch;
-  const int j0 = (blockIdx.x % blocks_per_batch) * rays_per_block;
+  const int b = (first_block + blockIdx.x) / blocks_per_batch;
+  const int j0 = (first_block + blockIdx.x) % blocks_per_batch * rays_per_block;
   const int rays = min(rays_per_block, M - j0);
   const float* pts = points + b * points_bstride;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -310,8 +314,9 @@ template <bool kShared>
 __global__ __launch_bounds__(kSvoBlock) void svo_intersect_kernel(
     const float* __restrict__ ray_start, const float* __restrict__ ray_dir,
     const float* __restrict__ centers, const int32_t* __restrict__ children,
-    int64_t B_M, int M, int T, int64_t centers_bstride, int64_t children_bstride,
-    float half_voxel, int n_max, const int32_t* __restrict__ flags, int nflags,
+    int64_t first_ray, int64_t B_M, int M, int T, int64_t centers_bstride,
+    int64_t children_bstride, float half_voxel, int n_max, const int32_t* __restrict__ flags,
+    int nflags,
     int32_t* __restrict__ idx, float* __restrict__ min_depth, float* __restrict__ max_depth) {
   __shared__ uint32_t waiting_at[kSvoMaxLevels][kSvoBlock];
   // blocks go round the 8 XCDs; each takes one contiguous eighth of the rays,
@@ -320,7 +325,7 @@ __global__ __launch_bounds__(kSvoBlock) void svo_intersect_kernel(
   const int64_t blk = int64_t(blockIdx.x) < per_xcd * 8
                           ? (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3)
                           : int64_t(blockIdx.x);
-  const int64_t r = blk * kSvoRays + (threadIdx.x >> 3);
+  const int64_t r = first_ray + blk * kSvoRays + (threadIdx.x >> 3);
   const int s = threadIdx.x & 7;
   const int shift = threadIdx.x & 56;   // this group's first lane in its wave
   const uint32_t before = (1u << s) - 1;
@@ -490,9 +495,12 @@ int nsvf_aabb_intersect(const float* ray_start, const float* ray_dir,
   const int64_t blocks = int64_t(bpb) * B;
   if (blocks > INT32_MAX) return set_error(NSVF_EINVAL, "aabb_intersect: too many rays");
   const int64_t pstride = points_shared ? 0 : int64_t(N) * 3;
-  hipLaunchKernelGGL(aabb_intersect_kernel, dim3(unsigned(blocks)), dim3(kAabbBlock), 0,
-                     as_stream(stream), ray_start, ray_dir, points, M, N, pstride, bpb, int(rpb),
-                     voxelsize * 0.5f, n_max, idx, min_depth, max_depth);
+  for (int64_t first = 0; first < blocks; first += kLaunchThreads / kAabbBlock) {
+    const int64_t n = std::min<int64_t>(blocks - first, kLaunchThreads / kAabbBlock);
+    hipLaunchKernelGGL(aabb_intersect_kernel, dim3(unsigned(n)), dim3(kAabbBlock), 0,
+                       as_stream(stream), ray_start, ray_dir, points, M, N, pstride, int(first),
+                       bpb, int(rpb), voxelsize * 0.5f, n_max, idx, min_depth, max_depth);
+  }
   return check_launch("aabb_intersect");
 }
 
@@ -536,9 +544,12 @@ int nsvf_svo_intersect_ws(const float* ray_start, const float* ray_dir,
   const auto kernel = tree_shared && int64_t(T) * 36 < (int64_t(1) << 32)
                           ? svo_intersect_kernel<true>
                           : svo_intersect_kernel<false>;
-  hipLaunchKernelGGL(kernel, dim3(unsigned(blocks)), dim3(kSvoBlock), 0, st, ray_start, ray_dir,
-                     points, children, BM, M, T, cstride, hstride, voxelsize * 0.5f, n_max, flags,
-                     nflags, idx, min_depth, max_depth);
+  for (int64_t first = 0; first < blocks; first += kLaunchThreads / kSvoBlock) {
+    const int64_t n = std::min<int64_t>(blocks - first, kLaunchThreads / kSvoBlock);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(n)), dim3(kSvoBlock), 0, st, ray_start, ray_dir,
+                       points, children, first * kSvoRays, BM, M, T, cstride, hstride,
+                       voxelsize * 0.5f, n_max, flags, nflags, idx, min_depth, max_depth);
+  }
   return check_launch("svo_intersect");
 }
 
