@@ -75,6 +75,16 @@ constexpr int kRowBins = 256;     // bins of a row staged in LDS: 16 KB per bloc
 constexpr int kWideBins = 1024;   // or 64 KB (two blocks per CU) where rows have more
 constexpr int kRowBlocks = 8192;  // more than the chip holds at once
 
+// Rows that a lane walks rather than a wavefront.  A wavefront costs some 0.65
+// ns per row however short it is; a lane a walk of its slots, 64 rows side by
+// side.  Lane against wavefront, us: 8 slots 16 and 16 for 4,096 rows, 17 and 56
+// for 65,536, 151 and 677 for 1,048,576; 16 slots 25 and 16, 31 and 58, 360 and
+// 721; 24 slots 33 and 16, 43 and 59, 593 and 782; 32 slots 44 and 17, 55 and 62,
+// 897 and 820.
+__host__ inline bool lane_per_row(int64_t rows, int slots) {
+  return slots <= 8 || (slots <= 24 && rows >= (1 << 16));
+}
+
 __device__ __forceinline__ int first_set(uint64_t mask) {
   return mask ? __ffsll(static_cast<unsigned long long>(mask)) - 1 : 64;
 }
@@ -280,6 +290,7 @@ __device__ int icdf_row_wave(const OpBins& bins, int P, float steps, float fixed
 // Bound: the padded rows' stores (12 S bytes per row) and the serial prefix
 // chain of up to 60 sums per row.  A lane per row walked its samples one by
 // one, every store to another line: 65,537 rows of up to 60 bins, 778 -> 174 us.
+// Rows of few slots keep that form (icdf_lanes_kernel).
 template <bool kNoise, bool kGrouped, bool kCount>
 __global__ __launch_bounds__(64 * kRowWaves) void icdf_rows_kernel(
     const int32_t* __restrict__ pts_idx, const float* __restrict__ min_depth,
@@ -337,12 +348,69 @@ __global__ __launch_bounds__(64 * kRowWaves) void icdf_rows_kernel(
   }
 }
 
+// A lane per row, each walking its samples: rows of few slots (lane_per_row).
+// Arguments as icdf_rows_kernel's.
+template <bool kNoise, bool kGrouped, bool kCount>
+__global__ __launch_bounds__(kSampleBlock) void icdf_lanes_kernel(
+    const int32_t* __restrict__ pts_idx, const float* __restrict__ min_depth,
+    const float* __restrict__ max_depth, const float* __restrict__ noise,
+    const float* __restrict__ probs, const float* __restrict__ steps, int64_t N, int R,
+    int P, int S, int G, int chunk, float fixed_step_size, int compat,
+    int32_t* __restrict__ out_idx, float* __restrict__ out_depth,
+    float* __restrict__ out_dists, int32_t* __restrict__ max_valid,
+    unsigned long long* __restrict__ flags) {
+  __shared__ int best;
+  if (threadIdx.x == 0) best = 0;
+  __syncthreads();
+  const int64_t n = int64_t(blockIdx.x) * kSampleBlock + threadIdx.x;
+  if (n < N) {
+    int64_t ray0, next;
+    if constexpr (kGrouped) {
+      grouped_neighbours(uint32_t(n), uint32_t(N), G, chunk, &ray0, &next);
+    } else {
+      ray0 = n / R * R;
+      next = n + 1 < N ? n + 1 : -1;
+    }
+    const int64_t H = n * P;
+    const OpBins bins{pts_idx + H, min_depth + H, max_depth + H, probs + H, pts_idx + ray0 * P,
+                      next < 0 ? -1 : pts_idx[next * P]};
+    CountedRowSink sink{RowSink{out_idx + n * S, out_depth + n * S, out_dists + n * S, S, 0}, 0};
+    const FlatNoise nz{kNoise ? noise + n * S : nullptr, kGrouped ? S : (N - n) * S};
+    const float st = steps[n];
+    int s;
+    if (kNoise)
+      s = icdf_ray(bins, P, st, fixed_step_size, nz, compat, S, sink);
+    else
+      s = icdf_ray(bins, P, st, fixed_step_size, ConstNoise{0.5f}, compat, S, sink);
+    sink.row.pad_from(min(s, S));
+    if (kCount) {
+      if (sink.row.dropped) atomicAdd(&flags[1], (unsigned long long)sink.row.dropped);
+      if (!kGrouped && int64_t(int(ceilf(st))) > nz.avail) atomicAdd(&flags[2], 1ull);
+    }
+    if (max_valid && sink.valid > 0) atomicMax(&best, sink.valid);
+  }
+  if (max_valid) {
+    __syncthreads();
+    if (threadIdx.x == 0 && best > 0) raise_max(max_valid, best);
+  }
+}
+
 template <bool kNoise, bool kGrouped>
 static void launch_icdf(const int32_t* pts_idx, const float* min_depth, const float* max_depth,
                         const float* noise, const float* probs, const float* steps, int64_t N,
                         int R, int P, int S, int G, int chunk, float fixed_step_size, int compat,
                         int32_t* out_idx, float* out_depth, float* out_dists, int32_t* max_valid,
                         int64_t* flags, void* stream) {
+  auto* fl = reinterpret_cast<unsigned long long*>(flags);
+  if (lane_per_row(N, S)) {
+    hipLaunchKernelGGL((flags ? icdf_lanes_kernel<kNoise, kGrouped, true>
+                              : icdf_lanes_kernel<kNoise, kGrouped, false>),
+                       dim3(unsigned(ceil_div(N, kSampleBlock))), dim3(kSampleBlock), 0,
+                       as_stream(stream), pts_idx, min_depth, max_depth, noise, probs, steps, N, R,
+                       P, S, G, chunk, fixed_step_size, compat, out_idx, out_depth, out_dists,
+                       max_valid, fl);
+    return;
+  }
   const dim3 grid(unsigned(std::min<int64_t>(ceil_div(N, kRowWaves), kRowBlocks)));
   const int cap = P <= kRowBins ? kRowBins : kWideBins;
   hipLaunchKernelGGL((flags ? icdf_rows_kernel<kNoise, kGrouped, true>
@@ -350,8 +418,7 @@ static void launch_icdf(const int32_t* pts_idx, const float* min_depth, const fl
                      grid, dim3(64 * kRowWaves), size_t(kRowWaves) * 4 * cap * sizeof(float),
                      as_stream(stream), pts_idx, min_depth,
                      max_depth, noise, probs, steps, N, R, P, S, G, chunk, fixed_step_size, compat,
-                     out_idx, out_depth, out_dists, max_valid,
-                     reinterpret_cast<unsigned long long*>(flags), cap);
+                     out_idx, out_depth, out_dists, max_valid, fl, cap);
 }
 
 // Uniform sampling of one ray (fairnr/clib/src/sample_gpu.cu:42-105) into a
