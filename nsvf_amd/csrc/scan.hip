@@ -149,7 +149,9 @@ __global__ __launch_bounds__(kScanBlock) void offsets_reduce_kernel(
 }
 
 // ... then every ray's rank among the hit rays, the list of these, and every
-// ray's slot offset; scalars = {hit rays, slots, 0, ...}.
+// ray's slot offset; scalars = {hit rays, slots, 0, ...}.  kDirect: as
+// scan_apply_kernel's, for both halves of partial.
+template <bool kDirect>
 __global__ __launch_bounds__(kScanBlock) void offsets_apply_kernel(
     const int32_t* __restrict__ flag, const int32_t* __restrict__ bound, int64_t R,
     const int32_t* __restrict__ partial, int32_t* __restrict__ rank, int32_t* __restrict__ list,
@@ -159,8 +161,11 @@ __global__ __launch_bounds__(kScanBlock) void offsets_apply_kernel(
   int f[kScanItems], v[kScanItems];
   const int sf = load_tile(flag, base, R, f);
   const int sv = load_tile(bound, base, R, v);
-  int hit = tiles_before(partial, smem) + block_incl_scan(sf, smem) - sf;
-  int slot = tiles_before(partial + gridDim.x, smem) + block_incl_scan(sv, smem) - sv;
+  const int32_t* slots = partial + gridDim.x;
+  int hit = (kDirect ? tiles_before(partial, smem) : partial[blockIdx.x]) +
+            block_incl_scan(sf, smem) - sf;
+  int slot = (kDirect ? tiles_before(slots, smem) : slots[blockIdx.x]) +
+             block_incl_scan(sv, smem) - sv;
 #pragma unroll
   for (int i = 0; i < kScanItems; ++i) {
     if (base + i < R) {
@@ -234,12 +239,21 @@ int nsvf_render_offsets(const int32_t* hit_flag, const int32_t* bound, int64_t R
     return set_error(NSVF_EINVAL, "render_offsets: bad size");
   if (!scalars || (R > 0 && (!hit_flag || !bound || !rank || !list || !off || !zero || !workspace)))
     return set_error(NSVF_EINVAL, "render_offsets: null pointer");
-  const dim3 grid(unsigned(std::max<int64_t>(ceil_div(R, kScanTile), 1)));
+  const int64_t tiles = ceil_div(R, kScanTile);
+  if (tiles > kMaxPartials)
+    return set_error(NSVF_EINVAL, "render_offsets: too many rays (%lld)", (long long)R);
+  const dim3 grid(unsigned(std::max<int64_t>(tiles, 1)));
+  hipStream_t st = as_stream(stream);
   if (R > 0)
-    hipLaunchKernelGGL(offsets_reduce_kernel, grid, dim3(kScanBlock), 0, as_stream(stream),
-                       hit_flag, bound, R, workspace, zero);
-  hipLaunchKernelGGL(offsets_apply_kernel, grid, dim3(kScanBlock), 0, as_stream(stream), hit_flag,
-                     bound, R, workspace, rank, list, off, scalars, nscalars);
+    hipLaunchKernelGGL(offsets_reduce_kernel, grid, dim3(kScanBlock), 0, st, hit_flag, bound, R,
+                       workspace, zero);
+  const bool direct = tiles <= kDirectTiles;
+  for (int k = 0; k < 2 && !direct; ++k)
+    hipLaunchKernelGGL(scan_partials_kernel, dim3(1), dim3(kScanBlock), 0, st,
+                       workspace + k * tiles, int(tiles), nullptr);
+  hipLaunchKernelGGL(direct ? offsets_apply_kernel<true> : offsets_apply_kernel<false>, grid,
+                     dim3(kScanBlock), 0, st, hit_flag, bound, R, workspace, rank, list, off,
+                     scalars, nscalars);
   return check_launch("render_offsets");
 }
 
