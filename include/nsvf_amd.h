@@ -372,7 +372,7 @@ int nsvf_render_hits_camera(const nsvf_camera* cam, const void* records, int T,
 /* What lies between a view's traversal and its coarse samples: rank and off
  * (exclusive sums of hit_flag (0 or 1) and bound over the R rays), list (the
  * hit rays), scalars = {hit rays, sum of bound, 0, ...} (nscalars >= 2 of
- * them), and zero [R] cleared.  workspace: int32[
+ * them), and zero [R] cleared; R up to 2^25.  workspace: int32[
  * nsvf_render_offsets_workspace_ints(R)].                                   */
 int64_t nsvf_render_offsets_workspace_ints(int64_t R);
 int nsvf_render_offsets(const int32_t* hit_flag, const int32_t* bound,
@@ -380,7 +380,8 @@ int nsvf_render_offsets(const int32_t* hit_flag, const int32_t* bound,
                         int32_t* zero, int32_t* scalars, int nscalars,
                         int32_t* workspace, void* stream);
 
-/* list[rank[r]] = r for every ray with hit_flag[r] != 0.                  */
+/* list[rank[r]] = r for every ray with hit_flag[r] != 0: the list alone, for
+ * ranks from elsewhere (nsvf_scan_exclusive_i32).                           */
 int nsvf_render_compact(const int32_t* hit_flag, const int32_t* rank,
                         int64_t R, int32_t* list, void* stream);
 
@@ -701,8 +702,7 @@ int nsvf_march_end(const int32_t* hit_list, int64_t n_hit, const int32_t* off,
  * finite or, in the backward, a sample's largest feature outside 2^-40 ..
  * 2^60 or a gradient above 2^60, and for all where a weight is.  Built for
  * D=32, H=128, L=3 (nsvf_mlp_train_supported); other shapes return
- * NSVF_EINVAL and the
- * size queries -1.
+ * NSVF_EINVAL and the size queries -1.
  * Parameters in torch layout: weights[l] [out][in] and biases[l] [out] for
  * l = 0..L (device pointers, host arrays of L + 1).  nsvf_mlp_train_pack
  * writes the kernels' operand fragments into `packed` (packed_floats).

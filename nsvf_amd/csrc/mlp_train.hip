@@ -1,7 +1,9 @@
-// The field MLP for training: forward and backward on v_mfma_f32_16x16x4_f32
-// (FP32 operands, FP32 accumulation), the differentiable counterpart of
+// The field MLP for training, the differentiable counterpart of
 // fairnr/modules/field.py:217-279 (Linear + ReLU layers, then sigma and
-// sigmoid RGB) that the reference trains through torch autograd.
+// sigmoid RGB) that the reference trains through torch autograd: forward and
+// backward on the 16-bit matrix units (mlp_f16x3.h and
+// mlp_train_backward_kernel below), and on v_mfma_f32_16x16x4_f32 (FP32
+// operands, FP32 accumulation) where those do not reach.  First the latter.
 //
 // Layout.  As in the field kernels, a layer runs transposed, Y^T = W X^T:
 // weight fragments are operand A (rows = output features), activations
@@ -28,13 +30,11 @@
 // order for a given sample count: the gradients are deterministic, with no
 // atomics.
 //
-// That is the FP32 kernel, which now runs for inputs that are not finite (or
-// far outside FP16's reach) only; the forward and backward otherwise run on
-// the 16-bit matrix units at FP32 accuracy (mlp_f16x3.h and
-// mlp_train_backward_kernel below), and the split-BF16 form (FieldMLPx3) is
-// the same backward kernel on BF16 parts: an FP32 operand f is hi + lo with
-// hi = bf16(f), lo = bf16(f - hi), a product Wl Xh + Wh Xl + Wh Xh in FP32
-// accumulators.
+// That is the FP32 kernel, which runs for the samples beside an input that is
+// not finite (or far outside FP16's reach) only; the others run on FP16 parts at
+// FP32 accuracy, and the split-BF16 form (FieldMLPx3) is the same backward
+// kernel on BF16 parts: an FP32 operand f is hi + lo with hi = bf16(f), lo =
+// bf16(f - hi), a product Wl Xh + Wh Xl + Wh Xh in FP32 accumulators.
 #include <algorithm>
 #include <type_traits>
 
@@ -494,12 +494,14 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 // multiplied back.  In the weight gradients, sums over samples, each sample's
 // factor multiplies dz when it is read, in bands of samples of like size
 // (BwdBands).
-// The FP16 matrix unit's sums come out low on average (measured: every bias
-// gradient's error negative, whatever its own sign).  That is below FP32's
-// rounding in one product, but a parameter's gradient adds a million: so every second sample's normalised gradient, and
-// every second chunk's weight gradient, is computed with the other sign.  (With
-// one sign the bias gradients were 3e-6 off on a million samples, FP32 MFMAs
-// 1e-6.)
+// The matrix unit's long sums come out low on average (measured: every bias
+// gradient's error negative, whatever its own sign; one accumulation by itself
+// rounds to nearest).  That is below FP32's rounding in one product, but a
+// parameter's gradient adds a million: so a chunk's sums are added by the
+// vector unit, and every second sample's normalised gradient, and every second
+// chunk's weight gradient, is computed with the other sign.  (In one accumulator
+// the weight gradients were 4e-6 off on a million samples, with one sign the
+// bias gradients 3e-6, FP32 MFMAs 1e-6.)
 // A chunk with an operand that is not finite or outside 2^-40 .. 2^60 is found
 // out before its weight gradients and left to the FP32 kernel above, which adds
 // partial sums of its own (all chunks, if it is a weight).  Repeating the whole
@@ -508,11 +510,11 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 //
 // Bound: LDS reads (about 15 k cycles per 64 samples at 128 B per cycle)
 // beside 12.5 k of MFMAs, and the phases' barriers.
-// Per million samples, against the form before (each wave its own 16 samples,
-// all weights from L2 for each): FP32 2,970 -> 1,170 us, split BF16 about
-// 1,900 -> 1,250 us (686 -> 460 us in the training step of 8,192 rays); 4,093
-// samples 109 -> 31 us.  The FP32 gradients are 4.9e-7 off 64 bits at most, 1.3e-6
-// before.
+// Against the form before (each wave its own 16 samples, all weights from L2 for
+// each): FP32 2,970 -> 1,426 us per million samples whose gradients spread over
+// four decades, 4,093 samples 109 -> 37 us; split BF16 686 -> 475 us for the
+// 0.51 M samples of a training step of 8,192 rays.  The FP32 gradients are
+// 6.7e-7 off 64 bits at most (300,003 samples), 1.1e-6 before.
 constexpr int kBwdWaves = 8;
 constexpr int kBwdBlock = 64 * kBwdWaves;
 constexpr int kBwdRow = 72;                  // halves per plane row
@@ -695,9 +697,7 @@ struct BwdBands {
 // at[ks] halves on (row c, sample 32 ks + 8 g), lo planes `lo_a` / `lo_b` halves
 // on; factor: the samples' factors, multiplied by 2^up (what the rows leave of
 // FP16's range: the bound that dz was scaled by is loose, by some 2^10 for dz0);
-// by: their sign in this chunk.  A chunk's products start from 0 and are added by the vector unit:
-// the matrix unit rounds its accumulations toward zero, which over a block's
-// hundreds of steps into one accumulator cost 4e-6 of the gradient (1e-6 so).
+// by: their sign in this chunk.
 template <bool F16, int NA, int NB>
 __device__ __forceinline__ void bwd_dw(const unsigned short* pa, int lo_a,
                                        const unsigned short* pb, int lo_b, const int (&at)[2],
@@ -1042,8 +1042,9 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         for (int r = 0; r < 4; ++r) z[r] = __fmaf_rn(z[r], bk[r], bh);
       } else {
         // in FP32: logits from parts of h2 and the weights put 2-10% on the
-        // error of every gradient against 64 bits (FP32 costs 45 us per million
-        // samples more, of 1,180 forward and backward)
+        // error of every gradient against 64 bits (FP32 costs 45 us more per
+        // million samples, of 1,150 forward and backward; as FMAs of the vector
+        // unit, a lane a quarter of a sample's features, 54)
         const float* h2 = reinterpret_cast<const float*>(S.t[3]);
 #pragma unroll
         for (int kt = 0; kt < 32; ++kt) {

@@ -3,7 +3,8 @@
 //
 //   hits      octree traversal + depth sort + segment-length sum per ray
 //             (encoder.py:498-535 with nsvf.py:65-74 folded in)
-//   compact   ray ranks -> list of hit rays (fairnr_model.py:157-162)
+//   (offsets  ranks and list of the hit rays, slot offsets: scan.hip;
+//             fairnr_model.py:157-162)
 //   sample    inverse-CDF sampling of a ray's bins into a sample stream
 //             (encoder.py:538-556, clib/__init__.py:231-300); coarse bins are
 //             the sorted hits, fine bins are the coarse samples
@@ -655,6 +656,8 @@ __global__ __launch_bounds__(kBlock) void ray_key_kernel(const float* __restrict
   keys[r] = (oct << 42) | (cell << 30) | morton;
 }
 
+// nsvf_render_compact: for callers of the C ABI with ranks of their own
+// (nsvf_render_offsets, which the renderer calls, makes the list too).
 __global__ __launch_bounds__(kBlock) void compact_kernel(const int32_t* __restrict__ flag,
                                                          const int32_t* __restrict__ rank,
                                                          int64_t R, int32_t* __restrict__ list) {
@@ -1372,8 +1375,6 @@ __global__ __launch_bounds__(kBlock) void composite_backward_kernel(
   }
 }
 
-// Frame outputs for every ray: the hit rays' composite plus the background
-// weighted by `missed`; rays that hit nothing are pure background.
 // Voxel and position o + d z of every slot (geometry.py:160-161, each product
 // and sum rounded); a record with no ray of the batch is unused.
 __global__ __launch_bounds__(kBlock) void stream_points_kernel(
@@ -1391,6 +1392,8 @@ __global__ __launch_bounds__(kBlock) void stream_points_kernel(
         ok ? ray_start[int64_t(s.ray) * 3 + a] + ray_dir[int64_t(s.ray) * 3 + a] * s.depth : 0.0f;
 }
 
+// Frame outputs for every ray: the hit rays' composite plus the background
+// weighted by `missed`; rays that hit nothing are pure background.
 __global__ __launch_bounds__(kBlock) void finish_kernel(
     int64_t R, const int32_t* __restrict__ hit_flag, const float* __restrict__ ray_rgb,
     const float* __restrict__ ray_depth, const float* __restrict__ ray_missed, float bg_r,
