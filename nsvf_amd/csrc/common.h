@@ -95,9 +95,12 @@ __device__ __forceinline__ bool ray_aabb(const float o[3], const float inv[3],
 // f_low > f_high at the end, and without one the running values are the
 // reference's.  The swap is a compare-and-select, as the reference's
 // ternaries, so an axis whose bounds come out NaN (direction 0 and origin on
-// the slab plane) is not swapped (a min / max pair would drop its NaN); the
-// running bounds then ignore a NaN as the reference's failed comparisons do,
-// since fmaxf / fminf return the other operand.  No branches: the traversals
+// the slab plane) is not swapped (a min / max pair would drop its NaN).  The
+// running bounds then ignore a NaN as the reference's failed comparisons do:
+// fmaxf returns the other operand, and the exit depth is a compare-and-select
+// again, since fminf takes -0 for less than +0, the reference's comparison does
+// not, and an exit depth of 0 keeps the sign of the first axis (0.5% of the
+// traversals' time).  No branches: the traversals
 // run one test per child and lane without divergence, and the three axes'
 // loads are in flight together.
 __device__ __forceinline__ bool ray_box(const float o[3], const float inv[3], const float mn[3],
@@ -112,7 +115,7 @@ __device__ __forceinline__ bool ray_box(const float o[3], const float inv[3], co
     const float lo = sw ? h0 : l0;
     const float hi = sw ? l0 : h0;
     f_low = fmaxf(f_low, lo);
-    f_high = fminf(f_high, hi);
+    f_high = hi < f_high ? hi : f_high;
   }
   *out_lo = f_low;
   *out_hi = f_high;
