@@ -655,7 +655,7 @@ __device__ __forceinline__ int row_max15(int v) {
 
 // The samples of a chunk in bands of like size, for a sum over samples whose
 // terms are 2^q[lane] x operands of one scale: each step takes those within
-// 2^-width of the largest that are left, leaves their factors +-2^(q - top) in
+// 2^-kBand of the largest that are left, leaves their factors +-2^(q - top) in
 // the wave's row of LDS (0 for the others) and top in `top`; false when none
 // are left.  u: the samples' units (0: no gradient), us: their signs.
 // A factor multiplies the FP16 parts of an operand, whose low parts lose bits
@@ -668,7 +668,7 @@ __device__ __forceinline__ int row_max15(int v) {
 // 4.6e-6 with 20; all of the row from k = 25 on with one band).  A million
 // samples whose gradients spread over four decades, the whole call: 1,385 us
 // with one band, 1,407 with 18, 1,519 with 16.
-constexpr int kBand = 16, kHeadBand = 16;
+constexpr int kBand = 16;
 struct BwdBands {
   int q;
   float us;
@@ -676,14 +676,14 @@ struct BwdBands {
   int top;
   __device__ __forceinline__ BwdBands(int q_, float u, float sign)
       : q(q_), us(copysignf(sign, u * sign)), left(u != 0.0f), top(0) {}
-  __device__ __forceinline__ bool next(_Float16* factor, int lane, int width) {
+  __device__ __forceinline__ bool next(_Float16* factor, int lane) {
     if (!__any(left)) return false;
     const int m = row_max15(left ? q : 0);   // exponents are positive
     top = __builtin_amdgcn_readlane(m, 15);
 #pragma unroll
     for (int r = 1; r < 4; ++r) top = max(top, __builtin_amdgcn_readlane(m, 16 * r + 15));
     const int d = q - top;
-    const bool in = left && d > -width;
+    const bool in = left && d > -kBand;
     wave_sync();   // the band before has been read
     factor[lane] = in ? _Float16(us * __int_as_float((127 + d) << 23)) : _Float16(0.0f);
     wave_sync();
@@ -1091,8 +1091,8 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
       ghb += hb;
     }
 
-    // a layer's weight gradient (k = 0 .. 2) or the head's (3): the samples'
-    // exponents are those of the normalised gradient times the layer's input
+    // the samples' exponents in layer k's weight gradient: those of the
+    // normalised gradient times the layer's input
     const auto bands = [&](int k) {
       const float u = S.unit[lane];
       const int e = (__float_as_int(u) & 0x7FFFFFFF) >> 23;
@@ -1113,7 +1113,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
 #pragma unroll
         for (int i = 0; i < (k == 0 ? 4 : 8); ++i) top = max(top, int(t[i]));
         const int up = min(max(ez[2 - k] - (__builtin_amdgcn_readfirstlane(top) >> 7), 0), 15);
-        while (b.next(S.factor[w], lane, kBand))
+        while (b.next(S.factor[w], lane))
           bwd_dw<true, NA, NB>(pa, kBwdPlane, pb, lo_b, at_row, S.factor[w], up, g,
                                b.top + ez[2 - k] - 409 - up, sign, sum);
       } else {
@@ -1165,41 +1165,48 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         }
       dz_out(v, mask[2], 3, 2, F16 ? f16_scale(ez[0]) : 1.0f);
     }
-    const auto head_gradient = [&]([[maybe_unused]] const _Float16* factor) {
+    if constexpr (F16) {
+      // in FP32 on the vector unit: lane (g, c) adds its 16 samples of feature
+      // c, for the four logits in gh.  A logit's gradients can lie far below
+      // its sample's largest, which is what the parts' scale would follow
+      const unsigned short* ph = &S.t[2][16 * w * kBwdRow + bwd_at(c, 16 * g)];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const f16x8 h = __builtin_bit_cast(f16x8, lds128(ph + 8 * q));
+        const f16x8 l = __builtin_bit_cast(f16x8, lds128(ph + 8 * q + kBwdPlane));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          const int k = 16 * g + 8 * q + i;
+          // the sample's unit over h2's scale (a power of two: its inverse)
+          const float f = S.unit[k] * __int_as_float((254 << 23) - __float_as_int(S.scale[2][k]));
+          const float x = __fmaf_rn(float(h[i]), f, float(l[i]) * f);
+          const float4 d = *reinterpret_cast<const float4*>(S.dl[k]);
+          gh[0] = __fmaf_rn(d.x, x, gh[0]);
+          gh[1] = __fmaf_rn(d.y, x, gh[1]);
+          gh[2] = __fmaf_rn(d.z, x, gh[2]);
+          gh[3] = __fmaf_rn(d.w, x, gh[3]);
+        }
+        tile_fence();
+      }
+    } else {
       f32x4 ghc = zero4;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        // dl of logit c (lanes c < 4) for samples 32 ks + 8 g + i, with their
-        // factors: at 2^14, a band's smallest keep their 22 bits
+        // dl of logit c (lanes c < 4) for samples 32 ks + 8 g + i
         unsigned int hw[4], lw[4];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-          float v[2], s[2] = {1.0f, 1.0f};
+          float v[2];
 #pragma unroll
-          for (int k = 0; k < 2; ++k) {
-            const int i = 32 * ks + 8 * g + 2 * p + k;
-            v[k] = c < 4 ? S.dl[i][c & 3] : 0.0f;
-            if constexpr (F16) s[k] = float(factor[i]) * 0x1p14f;
-          }
-          parts2<F16>(v[0], v[1], s[0], s[1], hw[p], lw[p]);
+          for (int k = 0; k < 2; ++k) v[k] = c < 4 ? S.dl[32 * ks + 8 * g + 2 * p + k][c & 3] : 0.0f;
+          parts2<F16>(v[0], v[1], 1.0f, 1.0f, hw[p], lw[p]);
         }
         const unsigned short* pb = &S.t[2][16 * w * kBwdRow + at_row[ks]];
         ghc = mm16x3<F16>(u32x4{hw[0], hw[1], hw[2], hw[3]}, u32x4{lw[0], lw[1], lw[2], lw[3]},
                           lds128(pb), lds128(pb + kBwdPlane), ghc);
         tile_fence();
       }
-      return ghc;
-    };
-    if constexpr (F16) {
-      BwdBands b = bands(3);
-      while (b.next(S.factor[w], lane, kHeadBand)) {
-        const f32x4 ghc = head_gradient(S.factor[w]);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          gh[r] = __fmaf_rn(__builtin_amdgcn_ldexpf(ghc[r], b.top + 127 - 409), sign, gh[r]);
-      }
-    } else {
-      gh = gh + head_gradient(nullptr);
+      gh = gh + ghc;
     }
     asm volatile("" : "+v"(gh));
     __syncthreads();
@@ -1274,6 +1281,10 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
 #pragma unroll
     for (int b = 0; b < 2; ++b)
       P[T::P_W0 + int64_t(16 * w + 4 * g + r) * D + 16 * b + c] = gw0[0][b][r];
+    if constexpr (F16) {   // a lane group's samples each
+      gh[r] = gh[r] + __shfl_xor(gh[r], 16, 64);
+      gh[r] = gh[r] + __shfl_xor(gh[r], 32, 64);
+    }
     if (g == 0) P[T::P_HEAD + int64_t(r) * H + 16 * w + c] = gh[r];
   }
 #pragma unroll

@@ -162,3 +162,19 @@ def test_chunks_beyond_the_window(device, wild):
         assert (a - b).abs().max() <= BAR * b.abs().max(), i
     again = _grads(FieldMLP, emb, ps, dout, device)
     assert all(torch.equal(a, b) for a, b in zip(got, again))
+
+
+@pytest.mark.parametrize("ratio", [1e-3, 1e-5, 1e-7, 1e-10])
+def test_logits_of_other_sizes(device, ratio):
+    """Colour gradients far below the samples' density gradients (saturated
+    colours, for one): the head's weight rows by themselves."""
+    M = 64 * 4 + 5
+    rng = np.random.default_rng(27)
+    ps = _params(27)
+    emb = (rng.standard_normal((M, 32)) * 0.1).astype(np.float32)
+    dout = rng.standard_normal((M, 4)).astype(np.float32)
+    dout[:, 1:] *= np.float32(ratio) * np.float32([1, 1e-2, 1e2])
+    want = _grads64(emb, ps, dout)
+    got = _grads(FieldMLP, emb, ps, dout, device)
+    _rows_close(got[7], want[7], "dW of the head")
+    _rows_close(got[8][:, None], want[8][:, None], "db of the head")
