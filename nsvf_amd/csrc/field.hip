@@ -1566,6 +1566,7 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void field_f16x3_kernel(
   const int64_t last = min(first + each, tiles);
   TileReader<Src> reader(src);
   if (first < last) reader.next(first * kF16Samples, M);
+  const bool beyond = mlp.beyond();
   for (int64_t t = first; t < last; ++t) {
     const int64_t base = t * kF16Samples;
     sink.begin_tile(base, M, kF16Samples);
@@ -1575,9 +1576,11 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void field_f16x3_kernel(
     };
     gather_f32_tile<D, true>(src.sc, g, x, weights);
     f32x4 out[kF32NT];
-    const bool done = mlp.tile(x, lane, g, out, [&](int l) {
-      if (l == 1 && t + 1 < last) reader.next(base + kF16Samples, M);
-    });
+    bool done = false;
+    if (!beyond)
+      done = mlp.tile(x, lane, g, out, [&](int l) {
+        if (l == 1 && t + 1 < last) reader.next(base + kF16Samples, M);
+      });
     if (!done) {
       // the weights' address as a value of this branch: its loads' addresses
       // would otherwise be formed before the loop and spilled

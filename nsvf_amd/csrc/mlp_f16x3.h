@@ -22,8 +22,9 @@
 // of 2^-39 of it, where FP32 accumulation rounds at 2^-24.  Scaling by powers
 // of two is exact and comes back out in the epilogue's fused multiply-add.
 //
-// A tile with an infinity or NaN in a layer's input (or weights), or whose
-// scales leave FP32's range, is reported; the caller then runs it on the
+// A tile with an infinity or NaN in a layer's input (or weights), whose scales
+// leave FP32's range, or whose weights one scale does not hold (kF16Spread), is
+// reported; the caller then runs it on the
 // FP32 MFMAs, so such inputs give what they gave there.
 //
 // Layout: the field kernels' transposed form Y^T = W X^T.  A wave's tile is
@@ -33,7 +34,8 @@
 // Element i of the FP16 fragment (mt, kt) is the FP32 packing's fragment
 // (mt, 8 kt + i) at the same lane, so the FP16 fragments are made from the
 // FP32 ones when a block stages its weights in LDS (152 KB for 32 -> 3 x 128
-// -> 4, hi and lo: one block of 8 waves per CU).
+// -> 4, hi and lo: one block of 8 waves per CU; the maxima that choose the scales
+// are found on the way).
 #pragma once
 
 #include "common.h"
@@ -46,6 +48,13 @@ typedef __attribute__((ext_vector_type(4))) float mfma_f32x4;
 constexpr int kF16Waves = 8;
 constexpr int kF16NT = 2;                 // n-tiles per wave tile
 constexpr int kF16Samples = 16 * kF16NT;  // samples per wave tile
+// One scale serves a layer whose rows and columns (those that are not 0) have
+// maxima of at least this share of the layer's largest weight.  A row or column
+// below it, a unit of no weight beside one of much, would be held in fewer bits
+// than FP32's: with units 1e7 as large and switched off by their biases, the
+// others' gradients were 10% off.  At 2^-10 the errors against 64 bits are
+// still the FP32 MFMAs'; layers drawn at random come to 2^-5.
+constexpr float kF16Spread = 0x1p-10f;
 
 __device__ __forceinline__ mfma_f32x4 mfma_f16(f16x8 a, f16x8 b, mfma_f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -80,6 +89,14 @@ __device__ __forceinline__ void f16_split2(float x, float y, float s, float t, f
   lo = __builtin_bit_cast(f16x2, l);
 }
 
+// Largest of the 16 lanes of a group, to its lane 15 (DPP row shifts; v >= 0).
+__device__ __forceinline__ int row_max15(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
+  return max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
+}
+
 // Maximum over the four lane groups (lanes c, c + 16, c + 32, c + 48).
 __device__ __forceinline__ float groups_max(float v) {
   v = fmaxf(v, __shfl_xor(v, 16, 64));
@@ -92,18 +109,29 @@ struct F16Mlp {
   static constexpr int KT0 = D / 32, KTH = H / 32, MT = H / 16, NT = kF16NT;
   static constexpr int FRAGS = MT * KT0 + (L - 1) * MT * KTH + KTH;
   static constexpr int BIASES = L * H + 4;
+  static constexpr int ROWS = L * H + 4, COLS = D + L * H;  // of all layers
   static constexpr size_t WEIGHT_BYTES = size_t(FRAGS) * 2048;
-  // weight fragments, biases, per-layer weight maxima
-  static constexpr size_t LDS_BYTES = WEIGHT_BYTES + (BIASES + L + 1) * sizeof(float);
+  // weight fragments, biases, per-layer weight maxima; while staging, those of
+  // the rows and columns
+  static constexpr size_t LDS_BYTES =
+      WEIGHT_BYTES + (BIASES + L + 1 + ROWS + COLS) * sizeof(float);
   static constexpr bool fits() { return H <= 128 && LDS_BYTES <= 160 * 1024; }
 
   // A block's view of its staged weights.
   const f16x8* w;       // [frag][hi, lo][64 lanes]
   const float* bias;    // hidden layers back to back, then the head's 4
-  const float* biggest; // [L + 1] largest |weight| per layer
+  const float* biggest; // [L + 1] largest |weight| per layer (infinite: no scale)
 
   static __device__ __forceinline__ int layer_of(int frag) {
     return frag < MT * KT0 ? 0 : min(1 + (frag - MT * KT0) / (MT * KTH), L);
+  }
+
+  // Whether a layer has no scale: every tile is for the FP32 units.
+  __device__ __forceinline__ bool beyond() const {
+    bool out = false;
+#pragma unroll
+    for (int l = 0; l <= L; ++l) out = out || weight_exponent(l) >= 255;
+    return __builtin_amdgcn_readfirstlane(out);
   }
 
   // Stages the FP32 fragments wfrag (field.pack_mlp's "f32") and biases into
@@ -114,18 +142,43 @@ struct F16Mlp {
     float* b = reinterpret_cast<float*>(lds + WEIGHT_BYTES);
     float* big = b + BIASES;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int* rows = reinterpret_cast<int*>(big + L + 1);
+    int* cols = rows + ROWS;
     if (threadIdx.x <= L) big[threadIdx.x] = 0.0f;
+    for (int i = threadIdx.x; i < ROWS + COLS; i += blockDim.x) rows[i] = 0;
     for (int i = threadIdx.x; i < BIASES; i += blockDim.x) b[i] = biases[i];
     __syncthreads();
     for (int f = wave; f < FRAGS; f += kF16Waves) {
+      const int l = layer_of(f), KT = l == 0 ? KT0 : KTH;
+      const int n = l == 0 ? f : f - MT * KT0 - (l - 1) * MT * KTH;
+      const int g = lane >> 4, c = lane & 15;
+      int* col = cols + (l == 0 ? 0 : D + (l - 1) * H) + 32 * (n % KT) + 4 * g;
       int m = 0;  // |x| as integer bits: NaN and infinity are the largest
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        m = max(m, __float_as_int(wfrag[(8 * f + i) * 64 + lane]) & 0x7FFFFFFF);
+      for (int i = 0; i < 8; ++i) {
+        const int v = __float_as_int(wfrag[(8 * f + i) * 64 + lane]) & 0x7FFFFFFF;
+        m = max(m, v);
+        const int top = row_max15(v);
+        if (c == 15) atomicMax(&col[i < 4 ? i : 12 + i], top);
+      }
+      m = max(m, __shfl_xor(m, 32, 64));
+      m = max(m, __shfl_xor(m, 16, 64));
+      if (g == 0 && (l < L || c < 4)) atomicMax(&rows[l * H + 16 * (n / KT) + c], m);
 #pragma unroll
-      for (int d = 32; d >= 1; d >>= 1) m = max(m, __shfl_xor(m, d, 64));
-      if (lane == 0) atomicMax(reinterpret_cast<int*>(big) + layer_of(f), m);
+      for (int d = 8; d >= 1; d >>= 1) m = max(m, __shfl_xor(m, d, 64));
+      if (lane == 0) atomicMax(reinterpret_cast<int*>(big) + l, m);
     }
+    __syncthreads();
+    unsigned int spread = 0;   // layers with a row or column below kF16Spread
+    for (int i = threadIdx.x; i < ROWS + COLS; i += blockDim.x) {
+      const int l = i < ROWS ? min(i / H, L) : max(i - ROWS - D + H, 0) / H;
+      const float v = __int_as_float(rows[i]);
+      if (v != 0.0f && v < big[l] * kF16Spread) spread |= 1u << l;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l <= L; ++l)
+      if (spread >> l & 1) big[l] = INFINITY;
     __syncthreads();
     for (int f = wave; f < FRAGS; f += kF16Waves) {
       const float s = f16_scale(min(f16_exponent(big[layer_of(f)]), 254));

@@ -230,6 +230,7 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void mlp_train_forward_kernel(
     }
   };
   if (first < last) load(first);
+  const bool beyond = mlp.beyond();
   for (int64_t t = first; t < last; ++t) {
     float x[NT][D / 4];
 #pragma unroll
@@ -242,9 +243,11 @@ __global__ __launch_bounds__(64 * kF16Waves, 1) void mlp_train_forward_kernel(
         x[j][4 * q + 3] = next[j][q].w;
       }
     f32x4 z[NT];
-    const bool done = mlp.tile(x, lane, g, z, [&](int l) {
-      if (l == 1 && t + 1 < last) load(t + 1);
-    });
+    bool done = false;
+    if (!beyond)
+      done = mlp.tile(x, lane, g, z, [&](int l) {
+        if (l == 1 && t + 1 < last) load(t + 1);
+      });
     if (!done) {
       const float4 bb = *reinterpret_cast<const float4*>(packed + T::BIAS_BASE + L * H);
 #pragma unroll
@@ -643,14 +646,6 @@ __device__ __forceinline__ void bwd_layer(const unsigned short* p, const int (&a
 #pragma unroll
     for (int m = 0; m < 4; ++m) acc[m] = acc[m] + small[m];
   }
-}
-
-// Largest of the 16 lanes of a group, to its lane 15 (DPP row shifts; v >= 0).
-__device__ __forceinline__ int row_max15(int v) {
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true));
-  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true));
-  return max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
 }
 
 // The samples of a chunk in bands of like size, for a sum over samples whose
@@ -1393,16 +1388,18 @@ __global__ __launch_bounds__(256) void split_pack_kernel(SplitLayers s,
 
 // Block l: layer l's largest |w|, row sum |w|, column sum |w| and b, the last 0
 // at least (not finite where a value is not; a bias of -inf is a unit switched
-// off).
+// off).  The largest |w| is infinite, too, where one scale does not do for the
+// layer (kF16Spread).
 template <int D, int H, int L>
 __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
                                                          float* __restrict__ stats) {
-  __shared__ int best[4];
-  __shared__ float cols[16][H];   // each wave's column sums
+  __shared__ int best[4], least;
+  __shared__ float cols[16][H], tops[16][H];   // each wave's column sums and maxima
   const int l = blockIdx.x, rows = l < L ? H : 4, in = l == 0 ? D : H;
   const float* W = net.w[l];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (threadIdx.x < 4) best[threadIdx.x] = 0;
+  if (threadIdx.x == 0) least = 0x7F800000;
   __syncthreads();
   // |x| as integer bits order as the values do, NaN and infinity on top
   const auto up = [&](int k, float v) {
@@ -1421,25 +1418,37 @@ __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
       const int r = wave + 16 * i, k = lane + 64 * q;
       v[i][q] = r < rows && k < in ? fabsf(W[r * in + k]) : 0.0f;
     }
-  float top = 0.0f, widest = 0.0f;
+  float widest = 0.0f;
+  int top = 0;
   float mine[H / 64] = {};
+  int most[H / 64] = {};
 #pragma unroll
   for (int i = 0; i < R; ++i) {
     float sum = 0.0f;
+    int row = 0;
 #pragma unroll
     for (int q = 0; q < H / 64; ++q) {
-      top = __int_as_float(max(__float_as_int(top), __float_as_int(v[i][q])));
+      row = max(row, __float_as_int(v[i][q]));
+      most[q] = max(most[q], __float_as_int(v[i][q]));
       mine[q] += v[i][q];
       sum += v[i][q];
     }
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    for (int d = 32; d >= 1; d >>= 1) {
+      sum += __shfl_xor(sum, d, 64);
+      row = max(row, __shfl_xor(row, d, 64));
+    }
     widest = __int_as_float(max(__float_as_int(widest), __float_as_int(sum) & 0x7FFFFFFF));
+    top = max(top, row);
+    if (lane == 0 && row != 0) atomicMin(&least, row);
   }
   up(1, widest);
-  up(0, top);
+  up(0, __int_as_float(top));
 #pragma unroll
-  for (int q = 0; q < H / 64; ++q) cols[wave][lane + 64 * q] = mine[q];
+  for (int q = 0; q < H / 64; ++q) {
+    cols[wave][lane + 64 * q] = mine[q];
+    tops[wave][lane + 64 * q] = __int_as_float(most[q]);
+  }
   float b = 0.0f;
   for (int i = threadIdx.x; i < rows; i += 1024) {
     const float bi = net.b[l][i];   // one below 0 only lowers its unit
@@ -1450,14 +1459,21 @@ __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
   // the waves' sums in order: the sums choose scales, so their last bits must
   // not depend on timing
   float col = 0.0f;
-  if (threadIdx.x < H)
+  if (threadIdx.x < H) {
+    int most = 0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) col += cols[w][threadIdx.x];
+    for (int w = 0; w < 16; ++w) {
+      col += cols[w][threadIdx.x];
+      most = max(most, __float_as_int(tops[w][threadIdx.x]));
+    }
+    if (most != 0) atomicMin(&least, most);
+  }
   up(2, col);
   __syncthreads();
   // row and column sums a little above their rounding
   if (threadIdx.x < 4) {
-    const float v = __int_as_float(best[threadIdx.x]);
+    float v = __int_as_float(best[threadIdx.x]);
+    if (threadIdx.x == 0 && __int_as_float(least) < v * kF16Spread) v = INFINITY;
     stats[threadIdx.x * (L + 1) + l] = threadIdx.x == 1 || threadIdx.x == 2 ? v * 1.001f : v;
   }
 }

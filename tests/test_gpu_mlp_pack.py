@@ -30,4 +30,7 @@ def test_packed_bounds_are_summed_in_one_order(device):
                 mine = mine + row
             cols = cols + mine
         assert packed[base + 8 + l] == cols.max() * np.float32(1.001), l
-        assert packed[base + l] == W.max()
+        lines = np.concatenate([W.max(0), W.max(1)])
+        spread = lines[lines > 0].min() < W.max() * np.float32(2.0 ** -10)
+        assert packed[base + l] == (np.inf if spread else W.max()), l
+        assert spread == (l == 3)   # columns of 4 weights: both forms of the rule
