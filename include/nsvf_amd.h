@@ -479,7 +479,8 @@ int nsvf_render_reuse_fill(const int32_t* hit_list, const int32_t* n_hit_dev,
  * (L hidden ReLU layers of width H on a D-wide embedding, 4-wide head).
  *   precision 0: BF16 MFMA with FP32 accumulation, wfrag = packed bf16;
  *   precision 1: FP32 (on FP16 hi / lo parts at FP32 accuracy where the
- *     shape's weights fit the LDS, else FP32 MFMA), wfrag = packed f32;
+ *     shape's weights fit the LDS and no layer's rows or columns have maxima
+ *     below 2^-10 of its largest weight, else FP32 MFMA), wfrag = packed f32;
  *   precision 2: split BF16 ("bf16x3"): every product W X as
  *     Wl Xh + Wh Xl + Wh Xh with W = Wh + Wl, X = Xh + Xl (bf16 parts),
  *     FP32 accumulation; wfrag = packed bf16 hi / lo fragment pairs; needs
@@ -696,11 +697,12 @@ int nsvf_march_end(const int32_t* hit_list, int64_t n_hit, const int32_t* off,
  * sigmoid(r, g, b)), which the reference differentiates with torch
  * autograd), forward and backward at FP32 accuracy: FP16 hi / lo parts of
  * scaled FP32 operands (22 significant bits, and an absolute error of 2^-39
- * of the layer's largest weight and of the sample's largest activation: what
- * is further below them has fewer bits), or the FP32 MFMAs for the tiles of 32
- * (forward) and chunks of 64 samples (backward) with a value that is not
- * finite or, in the backward, a sample's largest feature outside 2^-40 ..
- * 2^60 or a gradient above 2^60, and for all where a weight is.  Built for
+ * of the layer's largest weight and of the sample's largest activation), or
+ * the FP32 MFMAs for the tiles of 32 (forward) and chunks of 64 samples
+ * (backward) with a value that is not finite or, in the backward, a sample's
+ * largest feature outside 2^-40 .. 2^60 or a gradient above 2^60, and for all
+ * where a weight is or a layer's rows or columns have maxima below 2^-10 of
+ * its largest weight.  Built for
  * D=32, H=128, L=3 (nsvf_mlp_train_supported); other shapes return
  * NSVF_EINVAL and the size queries -1.
  * Parameters in torch layout: weights[l] [out][in] and biases[l] [out] for

@@ -97,6 +97,13 @@ __device__ __forceinline__ int row_max15(int v) {
   return max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true));
 }
 
+// Largest of the wave (v >= 0), in a scalar register.
+__device__ __forceinline__ int wave_max(int v) {
+  const int m = row_max15(v);
+  return max(max(__builtin_amdgcn_readlane(m, 15), __builtin_amdgcn_readlane(m, 31)),
+             max(__builtin_amdgcn_readlane(m, 47), __builtin_amdgcn_readlane(m, 63)));
+}
+
 // Maximum over the four lane groups (lanes c, c + 16, c + 32, c + 48).
 __device__ __forceinline__ float groups_max(float v) {
   v = fmaxf(v, __shfl_xor(v, 16, 64));

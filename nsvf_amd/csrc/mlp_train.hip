@@ -483,7 +483,8 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 // which are dead by then.  The ReLU masks stay in registers (a bit per value).
 // The weight gradients accumulate in registers over the whole kernel, a wave
 // holding 32 x 64 of each hidden layer's, 16 x 32 of the first's and 4 x 16 of
-// the head's; the bias gradients are FP32 sums of dz.  Block partials are
+// the head's; the bias gradients are FP32 sums of dz, and the head's weight
+// gradient (FP16 form) FP32 sums of the vector unit.  Block partials are
 // added in block order, so the gradients do not depend on timing.
 //
 // Scales (FP16 only; all powers of two, exact).  Weights as in mlp_f16x3.h.  A
@@ -514,8 +515,8 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 // Bound: LDS reads (about 15 k cycles per 64 samples at 128 B per cycle)
 // beside 12.5 k of MFMAs, and the phases' barriers.
 // Against the form before (each wave its own 16 samples, all weights from L2 for
-// each): FP32 2,970 -> 1,426 us per million samples whose gradients spread over
-// four decades, 4,093 samples 109 -> 37 us; split BF16 686 -> 475 us for the
+// each): FP32 2,970 -> 1,367 us per million samples whose gradients spread over
+// four decades, 4,093 samples 109 -> 36 us; split BF16 686 -> 475 us for the
 // 0.51 M samples of a training step of 8,192 rays.  The FP32 gradients are
 // 6.7e-7 off 64 bits at most (300,003 samples), 1.1e-6 before.
 constexpr int kBwdWaves = 8;
@@ -659,10 +660,11 @@ __device__ __forceinline__ void bwd_layer(const unsigned short* p, const int (&a
 // gradient that the larger samples do not reach.  Gradients fall along a ray
 // with its transmittance, so samples that far apart are common.
 // Rows of dW that only samples 2^-k of their neighbours' reach, error against
-// 64 bits: 1.2e-6 for every k with 16 (up to 2.3e-6 at k = 15 .. 18 with 18,
-// 4.6e-6 with 20; all of the row from k = 25 on with one band).  A million
-// samples whose gradients spread over four decades, the whole call: 1,385 us
-// with one band, 1,407 with 18, 1,519 with 16.
+// 64 bits (root mean square over 12 networks): up to 5.5e-7 for every k with 16,
+// where the FP32 MFMAs' is 6.4e-7; with 18, 3.3e-6 at k = 17, with 20, 1.1e-5 at
+// k = 19, with one band all of the row from k = 25 on.  A million samples whose
+// gradients spread over four decades, forward and backward: 1,467 us with 16,
+// 1,377 with 18, 1,366 with 20.
 constexpr int kBand = 16;
 struct BwdBands {
   int q;
@@ -673,10 +675,7 @@ struct BwdBands {
       : q(q_), us(copysignf(sign, u * sign)), left(u != 0.0f), top(0) {}
   __device__ __forceinline__ bool next(_Float16* factor, int lane) {
     if (!__any(left)) return false;
-    const int m = row_max15(left ? q : 0);   // exponents are positive
-    top = __builtin_amdgcn_readlane(m, 15);
-#pragma unroll
-    for (int r = 1; r < 4; ++r) top = max(top, __builtin_amdgcn_readlane(m, 16 * r + 15));
+    top = wave_max(left ? q : 0);   // exponents are positive
     const int d = q - top;
     const bool in = left && d > -kBand;
     wave_sync();   // the band before has been read
@@ -1434,10 +1433,8 @@ __global__ __launch_bounds__(1024) void mlp_stats_kernel(TrainLayers net,
       sum += v[i][q];
     }
 #pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-      sum += __shfl_xor(sum, d, 64);
-      row = max(row, __shfl_xor(row, d, 64));
-    }
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    row = wave_max(row);
     widest = __int_as_float(max(__float_as_int(widest), __float_as_int(sum) & 0x7FFFFFFF));
     top = max(top, row);
     if (lane == 0 && row != 0) atomicMin(&least, row);
