@@ -80,9 +80,11 @@ constexpr int kRowBlocks = 8192;  // more than the chip holds at once
 // side.  Lane against wavefront, us: 8 slots 16 and 16 for 4,096 rows, 17 and 56
 // for 65,536, 151 and 677 for 1,048,576; 16 slots 25 and 16, 31 and 58, 360 and
 // 721; 24 slots 33 and 16, 43 and 59, 593 and 782; 32 slots 44 and 17, 55 and 62,
-// 897 and 820.
-__host__ inline bool lane_per_row(int64_t rows, int slots) {
-  return slots <= 8 || (slots <= 24 && rows >= (1 << 16));
+// 897 and 820.  Where dropped samples are counted, a wavefront's rows that might
+// drop one run on one of its lanes: 33 slots with noise, 1,048,576 rows, 1,048
+// and 1,162.
+__host__ inline bool lane_per_row(int64_t rows, int slots, bool count) {
+  return slots <= 8 || (slots <= (count ? 40 : 24) && rows >= (1 << 16));
 }
 
 __device__ __forceinline__ int first_set(uint64_t mask) {
@@ -402,7 +404,7 @@ static void launch_icdf(const int32_t* pts_idx, const float* min_depth, const fl
                         int32_t* out_idx, float* out_depth, float* out_dists, int32_t* max_valid,
                         int64_t* flags, void* stream) {
   auto* fl = reinterpret_cast<unsigned long long*>(flags);
-  if (lane_per_row(N, S)) {
+  if (lane_per_row(N, S, flags != nullptr)) {
     hipLaunchKernelGGL((flags ? icdf_lanes_kernel<kNoise, kGrouped, true>
                               : icdf_lanes_kernel<kNoise, kGrouped, false>),
                        dim3(unsigned(ceil_div(N, kSampleBlock))), dim3(kSampleBlock), 0,

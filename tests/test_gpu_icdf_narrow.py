@@ -72,3 +72,28 @@ def test_full_narrow_rows_are_counted(device, S):
     for g, r in zip(out, ref):
         np.testing.assert_array_equal(g.cpu().numpy(), r[0])
     assert int(flags[1]) > 0 and int(ref[3][1]) > 0
+
+
+@pytest.mark.parametrize("S", [40, 41])
+def test_counted_rows(device, S):
+    """The same outputs with and without counting, in the forms that each takes."""
+    N, P = 1 << 16, 6
+    a = rows(N, P, S, mean_steps=(S - P) / 2)
+    a[4][:] = np.minimum(a[4], S - 2).astype(np.float32)
+    a[4][::50] = S - 0.5                      # as many steps as slots: some are dropped
+    noise = torch.rand(N, S, generator=torch.Generator().manual_seed(1)).clamp_(0.001, 0.999)
+    t = [torch.from_numpy(x).to(device) for x in a] + [noise.to(device)]
+    p = lambda x: ctypes.c_void_p(x.data_ptr())
+    outs = []
+    for count in (False, True):
+        flags = torch.zeros(4, dtype=torch.int64, device=device)
+        out = [torch.empty((N, S), dtype=d, device=device)
+               for d in (torch.int32, torch.float32, torch.float32)]
+        assert _lib.lib().nsvf_inverse_cdf_sampling(
+            *(p(x) for x in t[:3]), p(t[5]), p(t[3]), p(t[4]), 1, N, P, S, -1.0, 1,
+            *(p(o) for o in out), p(flags) if count else None, None) == 0
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert int(flags[1]) > 0
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
