@@ -518,7 +518,7 @@ __global__ __launch_bounds__(kTrainBlock) void mlp_train_backward_f32_kernel(
 // each): FP32 2,970 -> 1,367 us per million samples whose gradients spread over
 // four decades, 4,093 samples 109 -> 36 us; split BF16 686 -> 475 us for the
 // 0.51 M samples of a training step of 8,192 rays.  The FP32 gradients are
-// 6.7e-7 off 64 bits at most (300,003 samples), 1.1e-6 before.
+// 6.3e-7 off 64 bits at most (a million samples, eight networks), 3.0e-6 before.
 constexpr int kBwdWaves = 8;
 constexpr int kBwdBlock = 64 * kBwdWaves;
 constexpr int kBwdRow = 72;                  // halves per plane row
@@ -1118,6 +1118,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
     // plane set `to`; the bias gradient in true units
     const auto dz_out = [&](float (&v)[4][4], unsigned int bits, int to, int l, float sz) {
       [[maybe_unused]] float largest = 0.0f;
+      float sum = 0.0f;   // the chunk's bias gradient: fewer roundings at the total's size
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         f32x4 u = {1.0f, 1.0f, 1.0f, 1.0f};
@@ -1126,10 +1127,10 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           v[m][r] = (bits >> (4 * m + r)) & 1u ? v[m][r] : 0.0f;
-          gb[l] = F16 ? __fmaf_rn(v[m][r], u[r], gb[l]) : gb[l] + v[m][r];
+          sum = F16 ? __fmaf_rn(v[m][r], u[r], sum) : sum + v[m][r];
           if constexpr (F16) largest = fmaxf(largest, fabsf(v[m][r]));
         }
-        asm volatile("" : "+v"(gb[l]));
+        asm volatile("" : "+v"(sum));
 #pragma unroll
         for (int p = 0; p < 2; ++p) {
           unsigned int hw, lw;
@@ -1141,6 +1142,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
         *reinterpret_cast<u32x2*>(&S.t[to][kBwdPlane + at_out[m]]) = lo;
         tile_fence();
       }
+      gb[l] = gb[l] + sum;
       if constexpr (F16) {
         const int m = row_max15(__float_as_int(largest));
         if (c == 15) S.dz_top[l][w][g] = short(m >> 16);
@@ -1164,6 +1166,7 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
       // c, for the four logits in gh.  A logit's gradients can lie far below
       // its sample's largest, which is what the parts' scale would follow
       const unsigned short* ph = &S.t[2][16 * w * kBwdRow + bwd_at(c, 16 * g)];
+      f32x4 sum = zero4;   // the chunk's: fewer roundings at the total's size
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         const f16x8 h = __builtin_bit_cast(f16x8, lds128(ph + 8 * q));
@@ -1175,13 +1178,14 @@ __global__ __launch_bounds__(kBwdBlock, 1) void mlp_train_backward_kernel(
           const float f = S.unit[k] * __int_as_float((254 << 23) - __float_as_int(S.scale[2][k]));
           const float x = __fmaf_rn(float(h[i]), f, float(l[i]) * f);
           const float4 d = *reinterpret_cast<const float4*>(S.dl[k]);
-          gh[0] = __fmaf_rn(d.x, x, gh[0]);
-          gh[1] = __fmaf_rn(d.y, x, gh[1]);
-          gh[2] = __fmaf_rn(d.z, x, gh[2]);
-          gh[3] = __fmaf_rn(d.w, x, gh[3]);
+          sum[0] = __fmaf_rn(d.x, x, sum[0]);
+          sum[1] = __fmaf_rn(d.y, x, sum[1]);
+          sum[2] = __fmaf_rn(d.z, x, sum[2]);
+          sum[3] = __fmaf_rn(d.w, x, sum[3]);
         }
         tile_fence();
       }
+      gh = gh + sum;
     } else {
       f32x4 ghc = zero4;
 #pragma unroll
